@@ -26,6 +26,7 @@
 
 #include "dev_common.hpp"
 #include "device.hpp"
+#include "orders.hpp"
 
 namespace ifgf
 {
@@ -389,89 +390,6 @@ __global__ __launch_bounds__(128) void k_up(const int32_t* __restrict__ work, in
 }
 
 
-// upward pass with the precomputed geometry (per parent level of a geometry, see UpLevel in
-// plan.hpp): per (node, child) one table entry gives the child's fine cell, local coordinates
-// and transfer factor.  A workgroup takes up to K parent cones of one cell (item.box = the
-// cell's index in its table, item.pad = the table part, glist[item.first ..] the cones), so
-// each entry is read once for K boxes; children are summed in order for every cone
-// (ifgfoperator.hpp:631-688, 1639-1705).
-template <typename R, int O0, int O1, int O2, int K>
-__global__ __launch_bounds__(128) void k_up_cell(const WorkItem* __restrict__ items,
-                                                 int64_t nitems,
-                                                 const int32_t* __restrict__ glist,
-                                                 const ConeDev* __restrict__ cones,
-                                                 const BoxGeo* __restrict__ geo,
-                                                 const int32_t* __restrict__ child,
-                                                 const CellRef* __restrict__ ctab,
-                                                 const UpEnt<R>* __restrict__ ents,
-                                                 const int64_t* __restrict__ part_ent,
-                                                 const Cx<R>* __restrict__ F,
-                                                 Cx<R>* __restrict__ V, KParams kp)
-{
-    __shared__ int64_t toff[K][8]; // table offset of child c of cone k; -1: no child
-    __shared__ int32_t gs[K];
-    const int64_t it = xcd_block(kp.xlg);
-    if (it >= nitems)
-        return;
-    const WorkItem wi = items[it];
-    const int tid = threadIdx.x;
-    if (tid < K * 8)
-    {
-        const int k = tid >> 3, c = tid & 7;
-        int64_t off = -1;
-        if (k < wi.count)
-        {
-            const int32_t g = glist[wi.first + k];
-            if (c == 0)
-                gs[k] = g;
-            const int32_t ch = child[8 * cones[g].box + c];
-            if (ch >= 0)
-                off = geo[ch].table_off;
-        }
-        toff[k][c] = off;
-    }
-    __syncthreads();
-    const int n = wi.count;
-    for (int q = tid; q < kp.n_hi; q += blockDim.x)
-    {
-        const UpEnt<R>* e = ents + part_ent[wi.pad] + (int64_t(wi.box) * kp.n_hi + q) * 8;
-        Cx<R> acc[K];
-#pragma unroll
-        for (int k = 0; k < K; k++)
-            acc[k] = {0, 0};
-#pragma unroll 1
-        for (int c = 0; c < 8; c++)
-        {
-            const UpEnt<R> E = e[c];
-            if (E.cf < 0)
-                continue;
-#pragma unroll
-            for (int k = 0; k < K; k++)
-            {
-                if (k >= n)
-                    continue;
-                const int64_t to = toff[k][c];
-                if (to < 0)
-                    continue;
-                const CellRef cr = ctab[to + E.cf];
-                if (!((cr.mask >> E.sub) & 1u))
-                    continue;
-                const int slot = cr.fine_base + __popc(cr.mask & ((1u << E.sub) - 1u));
-                Cx<R> val;
-                if constexpr (O0 > 0)
-                    val = fine_eval_chunked<O0, O1, O2, R>(F, slot, E.xi0, E.xi1, E.xi2);
-                else
-                    val = fine_eval<O0, O1, O2, R>(F, slot, kp, E.xi0, E.xi1, E.xi2);
-                acc[k] = cadd(acc[k], cmul(val, Cx<R>{E.tr, E.ti}));
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < K; k++)
-            if (k < n)
-                V[int64_t(gs[k]) * kp.n_hi + q] = acc[k];
-    }
-}
-
 // Chebyshev values T_1 .. T_{n-1} at x (T_0 = 1 is implied)
 template <int N> __device__ __forceinline__ void cheb_t(float x, float (&t)[N])
 {
@@ -595,16 +513,16 @@ __device__ __forceinline__ void eval_cone_g_mem(const float2* c,
 }
 
 // Upward pass with the grouped tables (FP32, compiled orders; ifgfoperator.hpp:631-688,
-// 1639-1705).  A workgroup takes the parent cones of an item one at a time, each from its
-// UpDesc record (read into LDS at once); all the cone's
+// 1639-1705).  A workgroup takes K consecutive cones of the tiled list one at a time, each from
+// its UpDesc record (read into LDS at once); all the cone's
 // (child, group) tasks run at once: a group is up to UP_GRP nodes falling in one child cone,
 // whose coefficients the thread reads once (from memory) for all of them, and writes each
 // node's value times its transfer factor to the node's partial sum of that child in LDS.  The
 // partial sums of every node are then added in child order, as the reference's.
 template <int O0, int O1, int O2, int NHI, int NT, int H0, int H1, int H2, bool TF>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_up_grp(
-    const WorkItem* __restrict__ items, int64_t nitems, const UpDesc* __restrict__ desc,
-    const CellRef* __restrict__ ctab, const UpGrp* __restrict__ grp,
+    const UpDesc* __restrict__ desc, int64_t n, int K, const CellRef* __restrict__ ctab,
+    const UpGrp* __restrict__ grp,
     const Cx<float>* __restrict__ F, Cx<float>* __restrict__ V, const float* __restrict__ W,
     Cx<float>* __restrict__ Fo, KParams kp)
 {
@@ -620,15 +538,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     // the cone's record: child tables, task ranges, the slots of the listed child cones
     __shared__ UpDesc sd;
     __shared__ float2 part[8 * NHI + 1]; // node q's contribution from child c (+ a dump slot)
-    const int64_t it = xcd_block(kp.xlg);
-    if (it >= nitems)
-        return;
-    const WorkItem wi = items[it];
+    const int64_t first = xcd_block(kp.xlg) * K;
+    const int count = int(min<int64_t>(K, n - first));
     const int tid = threadIdx.x;
 #pragma unroll 1
-    for (int k = 0; k < wi.count; k++)
+    for (int k = 0; k < count; k++)
     {
-        const int4* src = reinterpret_cast<const int4*>(desc + (wi.first + k));
+        const int4* src = reinterpret_cast<const int4*>(desc + (first + k));
         for (int i = tid; i < NW; i += NT)
             reinterpret_cast<int4*>(&sd)[i] = src[i];
         for (int i = tid; i < 8 * NHI; i += NT)
@@ -1219,8 +1135,146 @@ static std::vector<WorkItem> make_items(const std::vector<int32_t>& boxes, const
     return out;
 }
 
-
-
+// The upward tables regrouped by child cone: per (cell, octant) row the distinct child fine
+// cones (cf, sub) its nodes fall into, in order of first appearance, and per child cone its
+// nodes (ascending) in records of at most Rec::N.  Row r's cones are dkey[2 doff[r] ..], its
+// records [goff[r], goff[r + 1]).
+template <class Rec> struct GroupTables
+{
+    std::vector<Rec> grp;
+    std::vector<int32_t> goff, doff, dkey;
+};
+// the rows of cells [c0, c1) of one part, appended to T
+template <class Rec>
+void group_cells(const UpLevel& U, int n_hi, int64_t c0, int64_t c1, GroupTables<Rec>& T)
+{
+    std::vector<int32_t> gcnt, gnode, nd(n_hi);
+    for (int64_t cell = c0; cell < c1; cell++)
+        for (int c = 0; c < 8; c++)
+        {
+            const UpEntry* row = &U.entries[size_t(cell) * n_hi * 8 + c]; // node q: row[8 q]
+            const size_t k0 = T.dkey.size() / 2;
+            T.doff.push_back(int32_t(k0));
+            T.goff.push_back(int32_t(T.grp.size()));
+            int last = -1; // neighbouring nodes mostly share the last cone found
+            for (int q = 0; q < n_hi; q++)
+            {
+                const UpEntry& E = row[8 * q];
+                nd[q] = -1;
+                if (E.cf < 0)
+                    continue;
+                const int nk = int(T.dkey.size() / 2 - k0);
+                auto is = [&](int i)
+                { return T.dkey[2 * (k0 + i)] == E.cf && T.dkey[2 * (k0 + i) + 1] == E.sub; };
+                int d = (last >= 0 && is(last)) ? last : -1;
+                for (int i = 0; d < 0 && i < nk; i++)
+                    if (is(i))
+                        d = i;
+                if (d < 0)
+                {
+                    d = nk;
+                    T.dkey.push_back(E.cf);
+                    T.dkey.push_back(E.sub);
+                }
+                nd[q] = last = d;
+            }
+            const int nk = int(T.dkey.size() / 2 - k0);
+            gcnt.assign(size_t(nk) + 1, 0);
+            for (int q = 0; q < n_hi; q++)
+                if (nd[q] >= 0)
+                    gcnt[size_t(nd[q]) + 1]++;
+            for (int i = 0; i < nk; i++)
+                gcnt[i + 1] += gcnt[i];
+            gnode.assign(size_t(gcnt[nk]), 0);
+            for (int q = 0; q < n_hi; q++)
+                if (nd[q] >= 0)
+                    gnode[size_t(gcnt[nd[q]]++)] = q;
+            for (size_t i = 0; i < gnode.size();)
+            {
+                const int d = nd[gnode[i]];
+                Rec G{};
+                G.cf = row[8 * gnode[i]].cf;
+                G.subd = row[8 * gnode[i]].sub | (d << 8);
+                uint32_t qs[4] = {0xffffu, 0xffffu, 0xffffu, 0xffffu};
+                for (int g = 0; g < Rec::N && i < gnode.size() && nd[gnode[i]] == d; g++, i++)
+                {
+                    using X = typename std::remove_reference<decltype(G.x0[0])>::type;
+                    const UpEntry& E = row[8 * gnode[i]];
+                    qs[g] = uint32_t(gnode[i]);
+                    G.x0[g] = X(E.xi[0]);
+                    G.x1[g] = X(E.xi[1]);
+                    G.x2[g] = X(E.xi[2]);
+                    G.tr[g] = X(E.tf[0]);
+                    G.ti[g] = X(E.tf[1]);
+                }
+                G.q01 = qs[0] | (qs[1] << 16);
+                if constexpr (Rec::N == 4)
+                    G.q23 = qs[2] | (qs[3] << 16);
+                T.grp.push_back(G);
+            }
+        }
+}
+// every part's rows, by up to 16 threads; part_cell[part]: the part's first cell
+template <class Rec>
+GroupTables<Rec> group_tables(const std::vector<const UpLevel*>& parts, int n_hi,
+                              std::vector<int64_t>& part_cell)
+{
+    struct Job
+    {
+        const UpLevel* U;
+        int64_t c0, c1;
+    };
+    std::vector<Job> jobs;
+    int64_t cells = 0;
+    for (const UpLevel* U : parts)
+    {
+        part_cell.push_back(cells);
+        const int64_t n = int64_t(U->entries.size()) / (int64_t(n_hi) * 8);
+        for (int64_t c = 0; c < n; c += 64)
+            jobs.push_back({U, c, std::min<int64_t>(n, c + 64)});
+        cells += n;
+    }
+    std::vector<GroupTables<Rec>> out(jobs.size());
+    const size_t nth = std::min<size_t>(16, std::max<size_t>(1, jobs.size()));
+    auto work = [&](size_t t)
+    {
+        for (size_t j = t; j < jobs.size(); j += nth)
+            group_cells(*jobs[j].U, n_hi, jobs[j].c0, jobs[j].c1, out[j]);
+    };
+    std::vector<std::thread> pool;
+    for (size_t t = 1; t < nth; t++)
+        pool.emplace_back(work, t);
+    work(0);
+    for (auto& th : pool)
+        th.join();
+    GroupTables<Rec> T;
+    size_t ng = 0, nk = 0;
+    for (const auto& o : out)
+    {
+        ng += o.grp.size();
+        nk += o.dkey.size();
+    }
+    if (nk / 2 > size_t(INT32_MAX))
+        throw std::runtime_error("upward tables: too many distinct child cones");
+    if (ng > size_t(INT32_MAX))
+        throw std::runtime_error("upward tables: too many node groups");
+    T.grp.reserve(ng);
+    T.dkey.reserve(nk);
+    for (auto& o : out)
+    {
+        const int32_t g0 = int32_t(T.grp.size()), k0 = int32_t(T.dkey.size() / 2);
+        for (int32_t v : o.goff)
+            T.goff.push_back(g0 + v);
+        for (int32_t v : o.doff)
+            T.doff.push_back(k0 + v);
+        T.grp.insert(T.grp.end(), o.grp.begin(), o.grp.end());
+        T.dkey.insert(T.dkey.end(), o.dkey.begin(), o.dkey.end());
+        o = GroupTables<Rec>();
+    }
+    T.goff.push_back(int32_t(T.grp.size()));
+    T.doff.push_back(int32_t(T.dkey.size() / 2));
+    return T;
+}
 
 // up_level >= 0: the upward pass into parent level up_level; otherwise the far field of
 // target level far_level
@@ -1232,44 +1286,24 @@ void launch_up_far_t(DevicePlan& D, hipStream_t st, const KParams& kp, const Nod
     const bool up = up_level >= 0;
     if (up)
     {
-        const int64_t i0 = D.up_item_off[up_level], i1 = D.up_item_off[up_level + 1];
         if constexpr (sizeof(R) == 4 && O0 > 0)
         {
-            // FP32, compiled orders: the grouped tables, the cones of an item one at a time,
-            // the items in tiles of boxes x cells
-            const int64_t t0 = D.up_tl_item_off[up_level], t1 = D.up_tl_item_off[up_level + 1];
-            // (at the larger orders their transform included: the cones' fine coefficients
-            // go to Fo, the values nowhere)
+            // FP32, compiled orders (at the larger orders with their transform: the cones' fine
+            // coefficients go to Fo, the values nowhere)
             constexpr bool TF = up_fuses_transform(O0 * O1 * O2);
-            if (t1 > t0 && !D.up_tl_desc)
+            const int64_t n = D.up_gl_off[up_level + 1] - D.up_gl_off[up_level];
+            if (n > 0 && !D.up_tl_desc)
                 throw std::runtime_error("upward pass: the per-cone records were not uploaded");
-            if (t1 > t0)
+            const int K = up_cones_per_block(D, n);
+            if (n > 0)
                 k_up_grp<O0, O1, O2, H0 * H1 * H2, 128, H0, H1, H2, TF>
-                    <<<dim3(unsigned(t1 - t0)), dim3(128), 0, st>>>(
-                        D.up_tl_items + t0, t1 - t0, D.up_tl_desc + D.up_gl_off[up_level],
-                        D.ctab, static_cast<const UpGrp*>(D.up_grp), F, V,
+                    <<<dim3(unsigned((n + K - 1) / K)), dim3(128), 0, st>>>(
+                        D.up_tl_desc + D.up_gl_off[up_level], n, K, D.ctab,
+                        static_cast<const UpGrp*>(D.up_grp), F, V,
                         static_cast<const float*>(D.wmat), Fo, kp);
         }
-        else if (i1 > i0)
-        {
-#define IFGF_UP_CELL(K)                                                                         \
-    k_up_cell<R, O0, O1, O2, K><<<dim3(unsigned(i1 - i0)), dim3(128), 0, st>>>(                \
-        D.up_items + i0, i1 - i0, D.up_glist + D.up_gl_off[up_level], D.cones, D.geo, D.child,  \
-        D.ctab, static_cast<const UpEnt<R>*>(D.up_entries), D.up_part_ent, F, V, kp)
-            switch (D.shape.up_k)
-            {
-            case 2: // items of at most 2 cones run as items of 4
-            case 4:
-                IFGF_UP_CELL(4);
-                break;
-            case 16:
-                IFGF_UP_CELL(16);
-                break;
-            default:
-                IFGF_UP_CELL(8);
-            }
-#undef IFGF_UP_CELL
-        }
+        else
+            launch_up_rows<R>(D, st, kp, up_level, F, V);
         if (b > a)
             k_up<PH, R, O0, O1, O2><<<dim3(unsigned(b - a)), dim3(128), 0, st>>>(
                 D.up_cones + a, b - a, D.cones, D.geo, D.child, D.ctab, tabs, F, V, kp);
@@ -1777,11 +1811,9 @@ void device_free(DevicePlan& D)
 {
     void* ptrs[] = {D.src_pts, D.tgt_pts, D.normals, D.src_perm, D.tgt_perm, D.src_begin,
                     D.src_end, D.child, D.geo, D.cones, D.ctab, D.ho_nodes, D.trig_th,
-                    D.trig_ph, D.fine_ang, D.wmat, D.up_part_ent, D.up_entries, D.up_dkey,
-                    D.up_doff, D.up_part_cell, D.up_goff, D.up_grp, D.up_items_k[0],
-                    D.up_items_k[1], D.up_items_k[2], D.up_items_k[3], D.up_glist,
-                    D.up_tl_items_k[0], D.up_tl_items_k[1], D.up_tl_items_k[2],
-                    D.up_tl_items_k[3], D.up_tl_glist, D.up_tl_gcell, D.up_tl_desc, D.tr_list,
+                    D.trig_ph, D.fine_ang, D.wmat, D.up_part_ent, D.up_entries, D.up_grp,
+                    D.up_items_k[0], D.up_items_k[1], D.up_items_k[2], D.up_items_k[3],
+                    D.up_glist, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
                     D.near_off, D.near_src, D.far_items, D.near_items, D.wsorted, D.result, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
@@ -2021,151 +2053,55 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                 parts.push_back(&pp.U);
             box_part = P.box_up_part;
         }
-        // the FP32 tables' row offsets kept on the host for k_up_grp's per-cone records (below)
-        std::vector<int64_t> h_part_cell, h_goff;
-        std::vector<int32_t> h_doff, h_dkey;
+        // the grouped tables' row offsets kept on the host for the per-cone records (below): row
+        // (h_part_cell[part] + cell) * 8 + octant (GroupTables)
+        std::vector<int64_t> h_part_cell;
+        std::vector<int32_t> h_goff, h_doff, h_dkey;
         {
             std::vector<UpEntF> ef;
             std::vector<UpEntD> ed;
-            std::vector<int64_t> part_ent, part_cell;
-            std::vector<int32_t> dkey, doff;
-            std::vector<UpGrp> grp;
-            std::vector<int64_t> goff;
-            std::vector<int32_t> gcnt, gnode;
+            std::vector<int64_t> part_ent;
             for (const UpLevel* U : parts)
             {
                 part_ent.push_back(int64_t(precision == PREC_FP64 ? ed.size() : ef.size()));
-                part_cell.push_back(int64_t(doff.size() / 8));
                 if (precision == PREC_FP64)
-                {
                     for (const UpEntry& E : U->entries)
                         ed.push_back({E.cf, E.sub, E.xi[0], E.xi[1], E.xi[2], E.tf[0], E.tf[1]});
-                    continue;
-                }
-                const size_t e0 = ef.size();
-                for (const UpEntry& E : U->entries)
-                    ef.push_back({E.cf, E.sub, float(E.xi[0]), float(E.xi[1]), float(E.xi[2]),
-                                  float(E.tf[0]), float(E.tf[1]), -1});
-                // the distinct child cones per (cell, octant); neighbouring nodes mostly share
-                // the last one found
-                const int64_t ncell = int64_t(U->entries.size()) / (int64_t(D.n_hi) * 8);
-                for (int64_t cell = 0; cell < ncell; cell++)
-                    for (int c = 0; c < 8; c++)
-                    {
-                        const int32_t k0 = int32_t(dkey.size() / 2);
-                        doff.push_back(k0);
-                        int last = -1;
-                        for (int q = 0; q < D.n_hi; q++)
-                        {
-                            UpEntF& E = ef[e0 + size_t((cell * D.n_hi + q) * 8 + c)];
-                            if (E.cf < 0)
-                                continue;
-                            const int nk = int(dkey.size() / 2) - k0;
-                            auto is = [&](int i) {
-                                return dkey[2 * (k0 + i)] == E.cf && dkey[2 * (k0 + i) + 1] == E.sub;
-                            };
-                            int d = (last >= 0 && is(last)) ? last : -1;
-                            for (int i = 0; d < 0 && i < nk; i++)
-                                if (is(i))
-                                    d = i;
-                            if (d < 0)
-                            {
-                                d = nk;
-                                dkey.push_back(E.cf);
-                                dkey.push_back(E.sub);
-                            }
-                            E.d = d;
-                            last = d;
-                        }
-                        // the nodes regrouped by child cone (in list order, nodes ascending
-                        // within a cone), runs of UP_GRP
-                        const int nk = int(dkey.size() / 2) - k0;
-                        goff.push_back(int64_t(grp.size()));
-                        gcnt.assign(size_t(nk) + 1, 0);
-                        for (int q = 0; q < D.n_hi; q++)
-                        {
-                            const UpEntF& E = ef[e0 + size_t((cell * D.n_hi + q) * 8 + c)];
-                            if (E.cf >= 0)
-                                gcnt[size_t(E.d) + 1]++;
-                        }
-                        for (int i = 0; i < nk; i++)
-                            gcnt[i + 1] += gcnt[i];
-                        gnode.assign(size_t(gcnt[nk]), 0);
-                        for (int q = 0; q < D.n_hi; q++)
-                        {
-                            const UpEntF& E = ef[e0 + size_t((cell * D.n_hi + q) * 8 + c)];
-                            if (E.cf >= 0)
-                                gnode[size_t(gcnt[E.d]++)] = q;
-                        }
-                        for (size_t i0 = 0; i0 < gnode.size();)
-                        {
-                            const UpEntF& E0 = ef[e0 + size_t((cell * D.n_hi + gnode[i0]) * 8 + c)];
-                            UpGrp G{};
-                            G.cf = E0.cf;
-                            G.subd = E0.sub | (E0.d << 8);
-                            uint32_t qs[UP_GRP];
-                            size_t i = i0;
-                            for (int g = 0; g < UP_GRP; g++)
-                            {
-                                qs[g] = 0xffffu;
-                                if (i < gnode.size() &&
-                                    ef[e0 + size_t((cell * D.n_hi + gnode[i]) * 8 + c)].d == E0.d)
-                                {
-                                    const UpEntF& E = ef[e0 + size_t((cell * D.n_hi + gnode[i]) * 8 + c)];
-                                    qs[g] = uint32_t(gnode[i]);
-                                    G.x0[g] = E.xi0;
-                                    G.x1[g] = E.xi1;
-                                    G.x2[g] = E.xi2;
-                                    G.tr[g] = E.tr;
-                                    G.ti[g] = E.ti;
-                                    i++;
-                                }
-                            }
-                            G.q01 = qs[0] | (qs[1] << 16);
-                            G.q23 = qs[2] | (qs[3] << 16);
-                            grp.push_back(G);
-                            i0 = i;
-                        }
-                    }
+                else
+                    for (const UpEntry& E : U->entries)
+                        ef.push_back({E.cf, E.sub, float(E.xi[0]), float(E.xi[1]),
+                                      float(E.xi[2]), float(E.tf[0]), float(E.tf[1]), -1});
             }
-            if (dkey.size() / 2 > size_t(INT32_MAX))
-                throw std::runtime_error("upward tables: too many distinct child cones");
-            if (grp.size() > size_t(INT32_MAX))
-                throw std::runtime_error("upward tables: too many node groups");
-            doff.push_back(int32_t(dkey.size() / 2));
-            goff.push_back(int64_t(grp.size()));
-            D.n_up_parts = int64_t(parts.size());
             D.up_part_ent = dupload(part_ent, tot);
-            if (precision != PREC_FP64)
+            auto groups = [&](auto G)
             {
-                D.up_part_cell = dupload(part_cell, tot);
-                D.up_doff = dupload(doff, tot);
-                D.up_dkey = dupload(dkey, tot);
-                std::vector<int32_t> goff32(goff.begin(), goff.end());
-                D.up_goff = dupload(goff32, tot);
-                D.up_grp = dupload(grp, tot);
-                h_part_cell = std::move(part_cell);
-                h_goff = std::move(goff);
-                h_doff = std::move(doff);
-                h_dkey = std::move(dkey);
-            }
+                D.up_grp = dupload(G.grp, tot);
+                h_goff = std::move(G.goff);
+                h_doff = std::move(G.doff);
+                h_dkey = std::move(G.dkey);
+            };
             if (precision == PREC_FP64)
+            {
                 D.up_entries = dupload(ed, tot);
+                groups(group_tables<UpGrpD>(parts, D.n_hi, h_part_cell));
+            }
             else
+            {
                 D.up_entries = dupload(ef, tot);
+                groups(group_tables<UpGrp>(parts, D.n_hi, h_part_cell));
+            }
         }
         // work lists.  Per level: leaf cones (leaf sampling), parent cones of boxes with a table
         // grouped by (part, cell) into items of at most UP_K_CHOICES[i] cones of one cell (boxes in order
         // within a cell), and the other parent cones (per-box upward pass)
         std::vector<int32_t> leaf, up, glist, tl_glist, tl_gcell, tr_list;
         D.tr_list_off.assign(D.levels + 1, 0);
-        std::vector<WorkItem> uitems[4], tl_items[4];
+        std::vector<WorkItem> uitems[4];
         D.up_off.assign(D.levels + 1, 0);
         D.up_gl_off.assign(D.levels + 1, 0);
         for (int kc = 0; kc < 4; kc++)
         {
             D.up_item_off_k[kc].assign(D.levels + 1, 0);
-            D.up_tl_item_off_k[kc].assign(D.levels + 1, 0);
         }
         D.cone_lvl_off.assign(D.levels + 1, 0);
         for (int l = 0; l < D.levels; l++)
@@ -2178,7 +2114,6 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
             for (int kc = 0; kc < 4; kc++)
             {
                 D.up_item_off_k[kc][l] = int64_t(uitems[kc].size());
-                D.up_tl_item_off_k[kc][l] = int64_t(tl_items[kc].size());
             }
             const int64_t g0 = int64_t(glist.size());
             D.tr_list_off[l] = int64_t(tr_list.size());
@@ -2241,18 +2176,6 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                              });
             for (size_t i = h0; i < tl_glist.size(); i++)
                 tl_gcell.push_back(cu(tl_glist[i]));
-            for (int kc = 0; kc < 4; kc++)
-                for (size_t i = h0; i < tl_glist.size();)
-                {
-                    const int32_t a = tl_glist[i], pa = part(a);
-                    size_t j = i;
-                    while (j < tl_glist.size() && int(j - i) < UP_K_CHOICES[kc] &&
-                           part(tl_glist[j]) == pa && tb(tl_glist[j]) == tb(a) &&
-                           tc(tl_glist[j]) == tc(a))
-                        j++;
-                    tl_items[kc].push_back({cu(a), int32_t(i - h0), int32_t(j - i), pa});
-                    i = j;
-                }
         }
         D.up_off[D.levels] = int64_t(up.size());
         D.up_gl_off[D.levels] = int64_t(glist.size());
@@ -2260,22 +2183,15 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         {
             D.up_item_off_k[kc][D.levels] = int64_t(uitems[kc].size());
             D.up_items_k[kc] = dupload(uitems[kc], tot);
-            D.up_tl_item_off_k[kc][D.levels] = int64_t(tl_items[kc].size());
-            D.up_tl_items_k[kc] = dupload(tl_items[kc], tot);
         }
         D.up_items = D.up_items_k[3]; // the default shape: 16 cones per item
         D.up_item_off = D.up_item_off_k[3];
-        D.up_tl_items = D.up_tl_items_k[3];
-        D.up_tl_item_off = D.up_tl_item_off_k[3];
         D.up_glist = dupload(glist, tot);
-        D.up_tl_glist = dupload(tl_glist, tot);
-        D.up_tl_gcell = dupload(tl_gcell, tot);
-        if (precision != PREC_FP64 && order_class(D) != 0 && !tl_glist.empty())
+        if (!tl_glist.empty())
         {
-            // k_up_grp's per-cone records, from the plan's fixed tables: the children and their
-            // cell-table offsets, the task ranges of each child's groups (the (cell, octant)
-            // rows of up_goff), the fine slots of the listed child cones (up_doff / up_dkey
-            // through the children's cell tables)
+            // the upward kernels' per-cone records, from the plan's fixed tables: the children and their
+            // cell-table offsets, the task ranges of each child's groups (the rows of h_goff), the
+            // fine slots of the listed child cones (h_dkey through the children's cell tables)
             std::vector<UpDesc> desc(tl_glist.size());
             auto fill = [&](size_t i0, size_t i1)
             {
@@ -2463,13 +2379,14 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                     " MiB) do not fit the free device memory (" + std::to_string(free_b >> 20) +
                     " MiB)");
             D.V = dalloc<unsigned char>(cs * v_lvl, tot);
-            D.F_bank[0] = dalloc<unsigned char>(cs * f_lvl[0], tot);
-            D.F_bank[1] = dalloc<unsigned char>(cs * f_lvl[1], tot);
+            D.F_bank[0] = dalloc<unsigned char>(cs * (f_lvl[0] + ROW_PAD), tot);
+            D.F_bank[1] = dalloc<unsigned char>(cs * (f_lvl[1] + ROW_PAD), tot);
         }
         else
         {
             D.V = dalloc<unsigned char>(cs * size_t(std::max<int64_t>(1, D.n_cones)) * D.n_hi, tot);
-            D.F = dalloc<unsigned char>(cs * size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo, tot);
+            D.F = dalloc<unsigned char>(
+                cs * (size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo + ROW_PAD), tot);
         }
         HIP_OK(hipDeviceSynchronize());
     }
@@ -2695,8 +2612,6 @@ std::string device_set_shape(DevicePlan& D, const LaunchShape& sh)
     D.shape = sh;
     D.up_items = D.up_items_k[kc];
     D.up_item_off = D.up_item_off_k[kc];
-    D.up_tl_items = D.up_tl_items_k[kc];
-    D.up_tl_item_off = D.up_tl_item_off_k[kc];
     if (changed)
         device_drop_graph(D); // the captured kernels have the old shapes
     return "";

@@ -77,10 +77,13 @@ constexpr int UP_K_CHOICES[4] = {2, 4, 8, 16};
 constexpr int UP_TILE_BOXES = 16;
 constexpr int UP_TILE_CELLS = 128;
 
-// What k_up_grp needs of a parent cone before its tasks, per entry of the tiled upward list
-// (FP32, compiled orders), computed at upload from the plan's fixed tables: read as one
+// What k_up_grp and k_up_rows need of a parent cone before its tasks, per entry of the tiled
+// upward list, computed at upload from the plan's fixed tables: read as one
 // 16-byte-aligned record instead of a chain of dependent loads (cone -> box -> children ->
 // their tables -> the (cell, octant) rows -> the listed child cones' slots).
+// entries allocated past the fine coefficients: kernels that read a cone's coefficients a chunk
+// of rows at a time may read up to this far past the last cone's (and use none of it)
+constexpr int ROW_PAD = 32;
 constexpr int UP_DMAX = 32; // listed child cones per (parent cone, child) with a slot here
 struct alignas(16) UpDesc
 {
@@ -137,17 +140,9 @@ struct DevicePlan
     // one geometry), up_part_ent[part] = the part's first entry
     void* up_entries = nullptr;
     int64_t* up_part_ent = nullptr;
-    int64_t n_up_parts = 0;
-    // FP32 tables: per (cell, octant) the distinct child cones (cf, sub) its entries fall into,
-    // in order of first appearance (UpEntF::d indexes them): up_dkey pairs, (cell, octant) row
-    // r = (up_part_cell[part] + cell) * 8 + octant spans up_dkey[2 up_doff[r] .. 2 up_doff[r+1])
-    int32_t* up_dkey = nullptr;
-    int32_t* up_doff = nullptr;
-    // the same tables regrouped by child cone (UpGrp records; FP32): the groups of row r span
-    // up_grp[up_goff[r] .. up_goff[r + 1])
-    int32_t* up_goff = nullptr;
+    // the same tables regrouped by child cone (UpGrp / UpGrpD records): one read of a child
+    // cone's coefficients serves the nodes that fall into it
     void* up_grp = nullptr;
-    int64_t* up_part_cell = nullptr;
 
     // (cell, cones of that cell, part) items of at most UP_K_CHOICES[i] cones, one list per
     // choice; up_items / up_item_off name the list of the current shape
@@ -157,16 +152,9 @@ struct DevicePlan
     std::vector<int64_t> up_item_off;        // per level, into up_items
     int32_t* up_glist = nullptr;             // the items' cones, level-major
     std::vector<int64_t> up_gl_off;          // per level, into up_glist
-    // the same cones for k_up_grp (which takes an item's cones one at a time): ordered by tiles
-    // of UP_TILE_BOXES boxes x UP_TILE_CELLS cells, items of at most UP_K_CHOICES[i] cones
-    // within a tile, each cone with its cell's table index (tl_gcell); same per-level offsets
-    WorkItem* up_tl_items_k[4] = {nullptr, nullptr, nullptr, nullptr};
-    std::vector<int64_t> up_tl_item_off_k[4];
-    WorkItem* up_tl_items = nullptr;
-    std::vector<int64_t> up_tl_item_off;
-    int32_t* up_tl_glist = nullptr;
-    int32_t* up_tl_gcell = nullptr;
-    UpDesc* up_tl_desc = nullptr; // per entry of up_tl_glist (FP32, compiled orders)
+    // the same cones for k_up_grp and k_up_rows (which take one cone at a time): per level (the
+    // ranges of up_gl_off) ordered by tiles of UP_TILE_BOXES boxes x UP_TILE_CELLS cells
+    UpDesc* up_tl_desc = nullptr; // one record per cone of the list
 
     int32_t* leaf_cones = nullptr;
     int64_t n_leaf_cones = 0;

@@ -1,0 +1,497 @@
+// orders.hip -- kernels that take the interpolation orders at run time.
+//
+// The tolerance estimate (ifgfoperator.hpp:108-244) raises each axis' order by itself, so the
+// orders of an operator are any of hundreds of combinations and cannot all be compiled.  These
+// kernels are compiled per first fine order O0 only (the contiguous axis of a fine cone's
+// coefficients) and walk the other two axes in loops: the coefficients of a cone are O1 O2 rows
+// of O0 values, read a chunk of rows ahead of the arithmetic, and the Chebyshev values of the
+// two outer axes come from their recurrence as the rows go by.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <stdexcept>
+
+#include "orders.hpp"
+
+namespace ifgf
+{
+namespace
+{
+using namespace dev;
+
+// a * b + c in one rounding
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return fma(a, b, c); }
+
+// A cone's coefficients are read a chunk ahead of the arithmetic, in two buffers of at most
+// CHUNK complex values (48 bytes of registers each): whole axis-2 planes where one or more fit,
+// else a plane's rows in equal parts
+template <typename R> constexpr int CHUNK = sizeof(R) == 4 ? 12 : 6;
+
+// Chebyshev values and sums of G points as the rows and planes of a cone go by
+template <typename R, int O0, int O1, int G> struct ConeSum
+{
+    R t0[G][O0], t1[G][O1], x2[G], a2[G], b2[G];
+    Cx<R> pl[G], out[G];
+    __device__ __forceinline__ ConeSum(const R (&x0)[G], const R (&x1)[G], const R (&x2_)[G])
+    {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+        {
+            t0[g][0] = t1[g][0] = R(1);
+            if constexpr (O0 > 1)
+                t0[g][1] = x0[g];
+#pragma unroll
+            for (int i = 2; i < O0; i++)
+                t0[g][i] = fma_r(R(2) * x0[g], t0[g][i - 1], -t0[g][i - 2]);
+            if constexpr (O1 > 1)
+                t1[g][1] = x1[g];
+#pragma unroll
+            for (int i = 2; i < O1; i++)
+                t1[g][i] = fma_r(R(2) * x1[g], t1[g][i - 1], -t1[g][i - 2]);
+            // T_i2 and T_i2-1 from (T_0, T_-1) = (1, x): the recurrence gives T_1 = x exactly
+            x2[g] = x2_[g];
+            a2[g] = R(1);
+            b2[g] = x2_[g];
+            out[g] = {R(0), R(0)};
+        }
+    }
+    // row i1 of the current plane
+    __device__ __forceinline__ void row(const Cx<R>* b, int i1)
+    {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+        {
+            Cx<R> sm = b[0];
+#pragma unroll
+            for (int i = 1; i < O0; i++)
+            {
+                sm.x = fma_r(b[i].x, t0[g][i], sm.x);
+                sm.y = fma_r(b[i].y, t0[g][i], sm.y);
+            }
+            if (i1 == 0)
+                pl[g] = sm;
+            else
+            {
+                pl[g].x = fma_r(sm.x, t1[g][i1], pl[g].x);
+                pl[g].y = fma_r(sm.y, t1[g][i1], pl[g].y);
+            }
+        }
+    }
+    __device__ __forceinline__ void end_plane()
+    {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+        {
+            out[g].x = fma_r(pl[g].x, a2[g], out[g].x);
+            out[g].y = fma_r(pl[g].y, a2[g], out[g].y);
+            const R t = fma_r(R(2) * x2[g], a2[g], -b2[g]);
+            b2[g] = a2[g];
+            a2[g] = t;
+        }
+    }
+};
+
+// The interpolant of one fine cone (coefficients c, index i0 + O0 (i1 + O1 i2)) at G points:
+// sum c T_i0(x0) T_i1(x1) T_i2(x2), over i0, then i1, then i2, each coefficient read once for
+// the G points.  A last chunk of several planes may run past the cone's coefficients (the
+// coefficient buffers are padded by ROW_PAD entries) and uses none of what lies there.
+template <typename R, int O0, int O1, int G>
+__device__ __forceinline__ void eval_planes(const Cx<R>* __restrict__ c, int o2, const R (&x0)[G],
+                                            const R (&x1)[G], const R (&x2)[G], Cx<R> (&out)[G])
+{
+    constexpr int NP = O0 * O1, CH = CHUNK<R>;
+    ConeSum<R, O0, O1, G> S(x0, x1, x2);
+    // loads and arithmetic stay on their sides of a fence: the next chunk's loads are in flight
+    // during this chunk's arithmetic
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+    if constexpr (NP <= CH)
+    {
+        // planes per chunk: a partly used last chunk reads for nothing, so few
+        constexpr int PB = NP >= 6 ? 1 : (NP >= 3 ? 2 : 4);
+        static_assert(PB * NP <= ROW_PAD, "the padding covers the last chunk");
+        Cx<R> ba[PB * NP], bb[PB * NP];
+        auto load = [&](Cx<R> (&b)[PB * NP])
+        {
+#pragma unroll
+            for (int i = 0; i < PB * NP; i++)
+                b[i] = c[i];
+            c += PB * NP;
+            fence();
+        };
+        auto sum = [&](const Cx<R> (&b)[PB * NP], int i2)
+        {
+#pragma unroll
+            for (int k = 0; k < PB; k++)
+            {
+                if (k > 0 && i2 + k >= o2) // uniform
+                    break;
+#pragma unroll
+                for (int i1 = 0; i1 < O1; i1++)
+                    S.row(b + k * NP + i1 * O0, i1);
+                S.end_plane();
+            }
+            fence();
+        };
+        load(ba);
+#pragma unroll 1
+        for (int i2 = 0;; i2 += 2 * PB)
+        {
+            if (i2 + PB >= o2)
+            {
+                sum(ba, i2);
+                break;
+            }
+            load(bb);
+            sum(ba, i2);
+            if (i2 + 2 * PB >= o2)
+            {
+                sum(bb, i2 + PB);
+                break;
+            }
+            load(ba);
+            sum(bb, i2 + PB);
+        }
+    }
+    else
+    {
+        constexpr int RM = CH / O0 < 1 ? 1 : CH / O0; // most rows per chunk
+        constexpr int NCH = (O1 + RM - 1) / RM;       // chunks per plane
+        constexpr int CR = (O1 + NCH - 1) / NCH;      // rows per chunk (the last may have fewer)
+        Cx<R> b[2][CR * O0];
+#pragma unroll
+        for (int i = 0; i < CR * O0; i++)
+            b[0][i] = c[i];
+        fence();
+        auto plane = [&](auto more)
+        {
+            constexpr bool MORE = decltype(more)::value;
+#pragma unroll
+            for (int j = 0; j < NCH; j++)
+            {
+                // the next chunk: of this plane, or the next plane's first
+                const Cx<R>* p = j + 1 < NCH ? c + (j + 1) * CR * O0 : c + NP;
+                const int nr = (j + 1 < NCH && (j + 2) * CR > O1) ? O1 - (j + 1) * CR : CR;
+                if (MORE || j + 1 < NCH)
+                {
+#pragma unroll
+                    for (int i = 0; i < CR * O0; i++)
+                        if (i < nr * O0)
+                            b[(j + 1) & 1][i] = p[i];
+                }
+                fence();
+#pragma unroll
+                for (int k = 0; k < CR; k++)
+                    if (j * CR + k < O1)
+                        S.row(b[j & 1] + k * O0, j * CR + k);
+                fence();
+            }
+            S.end_plane();
+            c += NP;
+            if constexpr (MORE && (NCH & 1))
+            {
+#pragma unroll
+                for (int i = 0; i < CR * O0; i++)
+                    b[0][i] = b[1][i];
+            }
+        };
+#pragma unroll 1
+        for (int i2 = 0; i2 + 1 < o2; i2++)
+            plane(std::true_type());
+        plane(std::false_type());
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++)
+        out[g] = S.out[g];
+}
+
+// the same sum for first orders without a compiled kernel
+template <typename R, int G>
+__device__ __forceinline__ void eval_any(const Cx<R>* __restrict__ c, int o0, int o1, int o2,
+                                         const R (&x0)[G], const R (&x1)[G], const R (&x2)[G],
+                                         Cx<R> (&out)[G])
+{
+    R a2[G], b2[G];
+#pragma unroll
+    for (int g = 0; g < G; g++)
+    {
+        a2[g] = R(1);
+        b2[g] = x2[g];
+        out[g] = {R(0), R(0)};
+    }
+    for (int i2 = 0; i2 < o2; i2++)
+    {
+        R a1[G], b1[G];
+        Cx<R> pl[G];
+#pragma unroll
+        for (int g = 0; g < G; g++)
+        {
+            a1[g] = R(1);
+            b1[g] = x1[g];
+            pl[g] = {R(0), R(0)};
+        }
+        for (int i1 = 0; i1 < o1; i1++)
+        {
+            R a0[G], b0[G];
+            Cx<R> sm[G];
+#pragma unroll
+            for (int g = 0; g < G; g++)
+            {
+                a0[g] = R(1);
+                b0[g] = x0[g];
+                sm[g] = {R(0), R(0)};
+            }
+            for (int i0 = 0; i0 < o0; i0++, c++)
+            {
+                const Cx<R> v = *c;
+#pragma unroll
+                for (int g = 0; g < G; g++)
+                {
+                    sm[g].x = fma_r(v.x, a0[g], sm[g].x);
+                    sm[g].y = fma_r(v.y, a0[g], sm[g].y);
+                    const R t = fma_r(R(2) * x0[g], a0[g], -b0[g]);
+                    b0[g] = a0[g];
+                    a0[g] = t;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++)
+            {
+                pl[g].x = fma_r(sm[g].x, a1[g], pl[g].x);
+                pl[g].y = fma_r(sm[g].y, a1[g], pl[g].y);
+                const R t = fma_r(R(2) * x1[g], a1[g], -b1[g]);
+                b1[g] = a1[g];
+                a1[g] = t;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < G; g++)
+        {
+            out[g].x = fma_r(pl[g].x, a2[g], out[g].x);
+            out[g].y = fma_r(pl[g].y, a2[g], out[g].y);
+            const R t = fma_r(R(2) * x2[g], a2[g], -b2[g]);
+            b2[g] = a2[g];
+            a2[g] = t;
+        }
+    }
+}
+
+// f(O0, O1) with the fine orders of the first two axes as compile-time constants: first orders
+// 1 to 6 with second orders 1 to 10; (0, 0) for the others
+template <int O0, class Fn> void with_second_order(int o1, const Fn& f)
+{
+#define IFGF_O1(N)                                                                              \
+    case N:                                                                                     \
+        return f(std::integral_constant<int, O0>(), std::integral_constant<int, N>())
+    switch (o1)
+    {
+        IFGF_O1(1);
+        IFGF_O1(2);
+        IFGF_O1(3);
+        IFGF_O1(4);
+        IFGF_O1(5);
+        IFGF_O1(6);
+        IFGF_O1(7);
+        IFGF_O1(8);
+        IFGF_O1(9);
+        IFGF_O1(10);
+    }
+#undef IFGF_O1
+    f(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+}
+template <class Fn> void with_orders(int o0, int o1, const Fn& f)
+{
+    switch (o0)
+    {
+    case 1:
+        return with_second_order<1>(o1, f);
+    case 2:
+        return with_second_order<2>(o1, f);
+    case 3:
+        return with_second_order<3>(o1, f);
+    case 4:
+        return with_second_order<4>(o1, f);
+    case 5:
+        return with_second_order<5>(o1, f);
+    case 6:
+        return with_second_order<6>(o1, f);
+    }
+    f(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+}
+
+// Upward pass with the grouped tables at any orders (ifgfoperator.hpp:631-688, 1639-1705), as
+// k_up_grp but for the orders: a workgroup takes K consecutive cones of the tiled list, each
+// from its UpDesc record, and runs the cone's (child, group) tasks; a task reads its child
+// cone's coefficients once for the group's nodes.  SEQ = false: all tasks at once, node q's value
+// from child c in part[c n_hi + q], the eight then added in child order.  SEQ = true (n_hi too
+// large for eight copies in LDS): the children one after another, each adding to part[q] (a
+// node is in one group of a child, so no two threads add to the same place): the same sums.
+template <typename R, int O0, int O1, bool SEQ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 20 ? 4 : 3) : 2))) void k_up_rows(
+    const UpDesc* __restrict__ desc, int64_t n, int K, const CellRef* __restrict__ ctab,
+    const UpGrpOf<R>* __restrict__ grp, const Cx<R>* __restrict__ F, Cx<R>* __restrict__ V,
+    KParams kp)
+{
+    constexpr int G = UpGrpOf<R>::N;
+    constexpr int NW = int(sizeof(UpDesc) / 16);
+    extern __shared__ __align__(16) unsigned char up_smem[];
+    UpDesc& sd = *reinterpret_cast<UpDesc*>(up_smem);
+    Cx<R>* part = reinterpret_cast<Cx<R>*>(up_smem + sizeof(UpDesc));
+    const int nhi = kp.n_hi, o2 = kp.lo2;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int64_t first = xcd_block(kp.xlg) * K;
+    const int count = int(min<int64_t>(K, n - first));
+#pragma unroll 1
+    for (int k = 0; k < count; k++)
+    {
+        const int4* src = reinterpret_cast<const int4*>(desc + first + k);
+        for (int i = tid; i < NW; i += nt)
+            reinterpret_cast<int4*>(&sd)[i] = src[i];
+        for (int i = tid; i < (SEQ ? nhi : 8 * nhi); i += nt)
+            part[i] = {R(0), R(0)};
+        __syncthreads();
+        auto task = [&](int t, int c)
+        {
+            // the record's header and coordinates at once (16-byte loads)
+            const UpGrpOf<R>* ep = grp + (sd.tg0[c] + t);
+            const int4* ew = reinterpret_cast<const int4*>(ep);
+            union
+            {
+                int4 w[4];
+                struct
+                {
+                    int32_t cf, subd;
+                    uint32_t q01, q23;
+                    R x0[G], x1[G], x2[G];
+                } f;
+            } e;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                e.w[i] = ew[i];
+            const int d = e.f.subd >> 8;
+            int slot;
+            if (d < UP_DMAX)
+                slot = sd.slot[c][d];
+            else
+            {
+                const int sub = e.f.subd & 255;
+                const CellRef cr = ctab[sd.toff[c] + e.f.cf];
+                slot = ((cr.mask >> sub) & 1u) ? cr.fine_base + __popc(cr.mask & ((1u << sub) - 1u))
+                                               : -1;
+            }
+            if (slot < 0)
+                return;
+            R x0[G], x1[G], x2[G];
+#pragma unroll
+            for (int g = 0; g < G; g++)
+            {
+                x0[g] = e.f.x0[g];
+                x1[g] = e.f.x1[g];
+                x2[g] = e.f.x2[g];
+            }
+            Cx<R> val[G];
+            const Cx<R>* coef = F + int64_t(slot) * kp.n_lo;
+            if constexpr (O0 > 0)
+                eval_planes<R, O0, O1, G>(coef, o2, x0, x1, x2, val);
+            else
+                eval_any<R, G>(coef, kp.lo0, kp.lo1, o2, x0, x1, x2, val);
+            R tr[G], ti[G];
+#pragma unroll
+            for (int g = 0; g < G; g++)
+            {
+                tr[g] = ep->tr[g];
+                ti[g] = ep->ti[g];
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++)
+            {
+                const int q = int(((g < 2 ? e.f.q01 : e.f.q23) >> (16 * (g & 1))) & 0xffffu);
+                if (q == 0xffff) // an empty place
+                    continue;
+                const Cx<R> v = cmul(val[g], Cx<R>{tr[g], ti[g]});
+                if constexpr (SEQ)
+                    part[q] = cadd(part[q], v);
+                else
+                    part[c * nhi + q] = v;
+            }
+        };
+        if constexpr (SEQ)
+        {
+            for (int c = 0; c < 8; c++)
+            {
+                const int t1 = sd.tend[c];
+                for (int t = (c ? sd.tend[c - 1] : 0) + tid; t < t1; t += nt)
+                    task(t, c);
+                __syncthreads();
+            }
+        }
+        else
+        {
+            const int tot = sd.tend[7];
+            for (int t = tid; t < tot; t += nt)
+            {
+                int c = 0;
+                while (t >= sd.tend[c])
+                    c++;
+                task(t, c);
+            }
+            __syncthreads();
+        }
+        for (int q = tid; q < nhi; q += nt)
+        {
+            Cx<R> a = part[q];
+            if constexpr (!SEQ)
+            {
+#pragma unroll
+                for (int c = 1; c < 8; c++)
+                    a = cadd(a, part[c * nhi + q]);
+            }
+            V[int64_t(sd.g) * nhi + q] = a;
+        }
+        __syncthreads(); // before the next cone replaces sd and part
+    }
+}
+} // namespace
+
+namespace dev
+{
+template <typename R>
+void launch_up_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int level, const Cx<R>* F,
+                    Cx<R>* V)
+{
+    const int64_t n = D.up_gl_off[level + 1] - D.up_gl_off[level];
+    if (n == 0)
+        return;
+    if (!D.up_tl_desc)
+        throw std::runtime_error("upward pass: the per-cone records were not uploaded");
+    const size_t full = sizeof(UpDesc) + 8 * size_t(D.n_hi) * sizeof(Cx<R>);
+    const bool seq = full > size_t(48) * 1024;
+    const size_t lds = seq ? sizeof(UpDesc) + size_t(D.n_hi) * sizeof(Cx<R>) : full;
+    constexpr size_t LDS_MAX = 160 * 1024; // gfx950: 160 KB of LDS per CU
+    if (lds > LDS_MAX)
+        throw std::runtime_error("interpolation orders too large for the upward kernel's LDS");
+    const int K = up_cones_per_block(D, n);
+    const dim3 grid(unsigned((n + K - 1) / K)), block(seq ? 256 : 128);
+    const UpDesc* desc = D.up_tl_desc + D.up_gl_off[level];
+    const auto* grp = static_cast<const UpGrpOf<R>*>(D.up_grp);
+    with_orders(D.lo[0], D.lo[1], [&](auto o0, auto o1)
+                {
+                    constexpr int O0 = decltype(o0)::value, O1 = decltype(o1)::value;
+                    if (lds > size_t(64) * 1024)
+                        HIP_OK(hipFuncSetAttribute(
+                            reinterpret_cast<const void*>(&k_up_rows<R, O0, O1, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+                    if (seq)
+                        k_up_rows<R, O0, O1, true><<<grid, block, lds, st>>>(desc, n, K, D.ctab,
+                                                                             grp, F, V, kp);
+                    else
+                        k_up_rows<R, O0, O1, false><<<grid, block, lds, st>>>(desc, n, K, D.ctab,
+                                                                              grp, F, V, kp);
+                });
+}
+template void launch_up_rows<float>(DevicePlan&, hipStream_t, const KParams&, int,
+                                    const Cx<float>*, Cx<float>*);
+template void launch_up_rows<double>(DevicePlan&, hipStream_t, const KParams&, int,
+                                     const Cx<double>*, Cx<double>*);
+} // namespace dev
+} // namespace ifgf

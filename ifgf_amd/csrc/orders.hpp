@@ -1,0 +1,18 @@
+// orders.hpp -- launchers of the kernels that take the interpolation orders at run time
+// (orders.hip): the upward pass over the grouped tables for any orders in both precisions.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "dev_common.hpp"
+
+namespace ifgf
+{
+namespace dev
+{
+// the upward pass into the cones of parent level `level` that have a table: the children's
+// coefficients F -> the parents' high-order values V
+template <typename R>
+void launch_up_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int level, const Cx<R>* F,
+                    Cx<R>* V);
+} // namespace dev
+} // namespace ifgf

@@ -145,6 +145,15 @@ struct Loc
     double xi[3];
 };
 
+// q / f for a fine factor f known at run time: 1 or 3 (KernelSpec::fine_factor) without an
+// integer division
+__device__ __forceinline__ int div_factor(int q, int f)
+{
+    if (f == 3)
+        return q / 3;
+    return f == 1 ? q : q / f;
+}
+
 __device__ __forceinline__ bool locate(const BoxGeo& B, const CellRef* __restrict__ ctab,
                                        double v0, double v1, double v2, int f0, int f1, int f2,
                                        Loc& out)
@@ -173,7 +182,7 @@ __device__ __forceinline__ bool locate(const BoxGeo& B, const CellRef* __restric
         q[j] = min(max(int(fl), 0), B.nf[j] - 1);
         out.xi[j] = 2.0 * (t - double(q[j])) - 1.0;
     }
-    const int c0 = q[0] / f0, c1 = q[1] / f1, c2 = q[2] / f2;
+    const int c0 = div_factor(q[0], f0), c1 = div_factor(q[1], f1), c2 = div_factor(q[2], f2);
     const int cell = c0 + B.nc[0] * (c1 + B.nc[1] * c2);
     const CellRef cr = ctab[B.table_off + cell];
     const int sub = (q[0] - c0 * f0) + f0 * ((q[1] - c1 * f1) + f1 * (q[2] - c2 * f2));
@@ -317,9 +326,9 @@ __device__ __forceinline__ bool locate_fast(const BoxGeo& B, const double* eth, 
         q[2] = min(max(int(fl), 0), n2 - 1);
         out.xi[2] = float(2.0 * (t - double(q[2])) - 1.0);
     }
-    const int c0 = q[0] / f0, s0 = q[0] - c0 * f0;
+    const int c0 = div_factor(q[0], f0), s0 = q[0] - c0 * f0;
     {
-        const int c1 = q[1] / f1, c2 = q[2] / f2;
+        const int c1 = div_factor(q[1], f1), c2 = div_factor(q[2], f2);
         const CellRef cr = ctab[B.table_off + c0 + B.nc[0] * (c1 + B.nc[1] * c2)];
         const int sub = s0 + f0 * ((q[1] - c1 * f1) + f1 * (q[2] - c2 * f2));
         if ((cr.mask >> sub) & 1u)
@@ -340,7 +349,7 @@ __device__ __forceinline__ bool locate_fast(const BoxGeo& B, const double* eth, 
         p2 = p2 < 0 ? p2 + n2 : (p2 >= n2 ? p2 - n2 : p2);
         if (p1 < 0 || p1 >= n1)
             continue;
-        const int c1 = p1 / f1, c2 = p2 / f2;
+        const int c1 = div_factor(p1, f1), c2 = div_factor(p2, f2);
         const CellRef cr = ctab[B.table_off + c0 + B.nc[0] * (c1 + B.nc[1] * c2)];
         const int sub = s0 + f0 * ((p1 - c1 * f1) + f1 * (p2 - c2 * f2));
         if ((cr.mask >> sub) & 1u)

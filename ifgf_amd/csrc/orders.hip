@@ -97,7 +97,7 @@ template <typename R, int O0, int O1, int G> struct ConeSum
 // the G points.  A last chunk of several planes may run past the cone's coefficients (the
 // coefficient buffers are padded by ROW_PAD entries) and uses none of what lies there.
 template <typename R, int O0, int O1, int G>
-__device__ __forceinline__ void eval_planes(const Cx<R>* __restrict__ c, int o2, const R (&x0)[G],
+__device__ __forceinline__ void eval_planes(const Cx<R>* c, int o2, const R (&x0)[G],
                                             const R (&x1)[G], const R (&x2)[G], Cx<R> (&out)[G])
 {
     constexpr int NP = O0 * O1, CH = CHUNK<R>;
@@ -205,9 +205,66 @@ __device__ __forceinline__ void eval_planes(const Cx<R>* __restrict__ c, int o2,
         out[g] = S.out[g];
 }
 
+// The same sum at one point, the coefficients (in LDS, or in memory where several waves hide the
+// wait) read up to about 20 at a time with nothing read ahead: fewer registers, as many waves
+template <typename R, int O0, int O1>
+__device__ __forceinline__ Cx<R> eval_point(const Cx<R>* c, int o2, R x0, R x1, R x2)
+{
+    constexpr int NP = O0 * O1, MOST = sizeof(R) == 4 ? 20 : 10;
+    const R y0[1] = {x0}, y1[1] = {x1}, y2[1] = {x2};
+    ConeSum<R, O0, O1, 1> S(y0, y1, y2);
+    if constexpr (NP <= MOST)
+    {
+        constexpr int PB = MOST / NP > 4 ? 4 : MOST / NP; // planes per chunk
+        static_assert(PB * NP <= ROW_PAD, "the padding covers the last chunk");
+#pragma unroll 1
+        for (int i2 = 0; i2 < o2; i2 += PB, c += PB * NP)
+        {
+            Cx<R> b[PB * NP];
+#pragma unroll
+            for (int i = 0; i < PB * NP; i++)
+                b[i] = c[i];
+#pragma unroll
+            for (int k = 0; k < PB; k++)
+            {
+                if (k > 0 && i2 + k >= o2) // uniform
+                    break;
+#pragma unroll
+                for (int i1 = 0; i1 < O1; i1++)
+                    S.row(b + k * NP + i1 * O0, i1);
+                S.end_plane();
+            }
+        }
+    }
+    else
+    {
+        constexpr int CR = MOST / O0 < 1 ? 1 : MOST / O0; // rows per chunk
+#pragma unroll 1
+        for (int i2 = 0; i2 < o2; i2++, c += NP)
+        {
+#pragma unroll
+            for (int r = 0; r < O1; r += CR)
+            {
+                Cx<R> b[CR * O0];
+#pragma unroll
+                for (int i = 0; i < CR * O0; i++)
+                    if (r * O0 + i < NP)
+                        b[i] = c[r * O0 + i];
+#pragma unroll
+                for (int k = 0; k < CR; k++)
+                    if (r + k < O1)
+                        S.row(b + k * O0, r + k);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            S.end_plane();
+        }
+    }
+    return S.out[0];
+}
+
 // the same sum for first orders without a compiled kernel
 template <typename R, int G>
-__device__ __forceinline__ void eval_any(const Cx<R>* __restrict__ c, int o0, int o1, int o2,
+__device__ __forceinline__ void eval_any(const Cx<R>* c, int o0, int o1, int o2,
                                          const R (&x0)[G], const R (&x1)[G], const R (&x2)[G],
                                          Cx<R> (&out)[G])
 {
@@ -326,6 +383,10 @@ template <class Fn> void with_orders(int o0, int o1, const Fn& f)
 // from child c in part[c n_hi + q], the eight then added in child order.  SEQ = true (n_hi too
 // large for eight copies in LDS): the children one after another, each adding to part[q] (a
 // node is in one group of a child, so no two threads add to the same place): the same sums.
+// Bound by the vector-memory path (each coefficient is read once per group, 64 lanes wide) and
+// the waits for it: at (3,6,4), 1M points, 11.0 ms; 14.7 without the read-ahead, 16 ms when a
+// chunk was read ahead past the last one; at (2,3,3) and (2,5,5) within 2% of k_up_grp without
+// its transform.
 template <typename R, int O0, int O1, bool SEQ>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 20 ? 4 : 3) : 2))) void k_up_rows(
     const UpDesc* __restrict__ desc, int64_t n, int K, const CellRef* __restrict__ ctab,
@@ -451,6 +512,207 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         __syncthreads(); // before the next cone replaces sd and part
     }
 }
+// distinct cones per wave and source box copied to LDS
+constexpr int FAR_STAGE = 4;
+
+// the wave's LDS writes have completed before its next LDS reads (of what other lanes wrote)
+// issue; the memory clobber keeps the compiler from moving LDS accesses across
+__device__ __forceinline__ void wave_lds_wait()
+{
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+}
+
+// the nc coefficients of cones c0 .. c3 (the first nd of them) to LDS, `stride` entries apart, by
+// the nact active lanes of a wave together; U: 16 bytes where a cone is whole 16-byte words
+template <class U>
+__device__ __forceinline__ void stage_cones(const Cx<float>* __restrict__ F, int c0, int c1, int c2,
+                                            int c3, int nd, int nc, int stride, int rank, int nact,
+                                            Cx<float>* sc)
+{
+    constexpr int E = int(sizeof(U) / sizeof(Cx<float>));
+    static_assert(FAR_STAGE == 4, "four cones");
+    const int nu = nc / E;
+#pragma unroll 2
+    for (int i = rank; i < nd * nu; i += nact)
+    {
+        const bool b1 = i >= nu, b2 = i >= 2 * nu, b3 = i >= 3 * nu;
+        const int cf = b3 ? c3 : (b2 ? c2 : (b1 ? c1 : c0));
+        const int d = int(b1) + int(b2) + int(b3), k = i - d * nu;
+        *reinterpret_cast<U*>(sc + d * stride + E * k) =
+            reinterpret_cast<const U*>(F + int64_t(cf) * nc)[k];
+    }
+}
+
+// Far field at any orders (ifgfoperator.hpp:962-1012, 1708-1891): for each target of the item,
+// the interpolants of its far source boxes times the centre factor.  One wave per item, the
+// waves of a workgroup sharing the group's angle tables in LDS (FAST: cones located by
+// locate_fast; otherwise the exact locate).  With stage > 0 (cones of stage coefficients and
+// more) the distinct cones of the wave's lanes, up to FAR_STAGE, are copied to LDS by all lanes
+// together and each lane reads its own there, `stride` entries apart so that the same
+// coefficient of different cones lies in different banks; a wave with more distinct cones, and
+// every wave without staging, reads the coefficients from memory.
+// Bound by memory latency and the cone location's arithmetic: waves per SIMD matter, so a point's
+// coefficients are not all in registers (eval_point).  Far phase against the kernel that read each
+// coefficient from memory in Clenshaw order: 24.8 -> 8.8 ms at (3,6,4), 1M points; 26 -> 6.8 ms at
+// (5,5,5), combined field on a torus, 131,072 points; with a read-ahead in two buffers instead
+// 27 registers spilled at (2,5,*).
+template <typename R, int O0, int O1, bool FAST>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : (O0 * O1 > 24 ? 1 : 2)))) void k_far_rows(
+    const WorkItem* __restrict__ items, int64_t nitems, const int32_t* __restrict__ srange,
+    const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
+    const CellRef* __restrict__ ctab, const Cx<R>* __restrict__ F,
+    const double* __restrict__ tpts, const double* __restrict__ ang, int ang_base, int ang_n,
+    int stage, int stride, int phase, Cx<R>* __restrict__ result, KParams kp)
+{
+    extern __shared__ __align__(16) unsigned char far_smem[];
+    double* sang = reinterpret_cast<double*>(far_smem);
+    const int lane = int(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wpb = int(blockDim.x >> 6);
+    Cx<R>* sc = reinterpret_cast<Cx<R>*>(far_smem + ((ang_n + 1) & ~1) * sizeof(double)) +
+                wave * (FAR_STAGE * stride + ROW_PAD);
+    const int64_t it = xcd_block(kp.xlg) * wpb + wave;
+    if constexpr (FAST)
+    {
+        for (int i = threadIdx.x; i < ang_n; i += int(blockDim.x))
+            sang[i] = ang[ang_base + i];
+        __syncthreads();
+    }
+    if (it >= nitems)
+        return;
+    const WorkItem wi = items[it];
+    const int Tp = pow2_at_least(wi.count);
+    const int ti = lane & (Tp - 1);
+    const int grp = lane / Tp, ngrp = 64 / Tp;
+    const bool valid = ti < wi.count;
+    const int64_t t = int64_t(wi.first) + (valid ? ti : 0);
+    const double y0 = tpts[3 * t], y1 = tpts[3 * t + 1], y2 = tpts[3 * t + 2];
+    Cx<R> acc = {0, 0};
+    const int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
+    auto body = [&](const BoxGeo& B)
+    {
+        int fine;
+        double r, rinv;
+        R x0[1], x1[1], x2[1];
+        if constexpr (FAST)
+        {
+            LocF L;
+            const double* eth = sang + (2 * B.fth_off - ang_base);
+            const double* eph = sang + (2 * B.fph_off - ang_base);
+            if (!locate_fast(B, eth, eph, ctab, y0 - B.ctr[0], y1 - B.ctr[1], y2 - B.ctr[2],
+                             kp.f0, kp.f1, kp.f2, L))
+                return;
+            fine = L.fine;
+            r = L.r;
+            rinv = L.rinv;
+            x0[0] = R(L.xi[0]);
+            x1[0] = R(L.xi[1]);
+            x2[0] = R(L.xi[2]);
+        }
+        else
+        {
+            Loc L;
+            if (!locate(B, ctab, y0 - B.ctr[0], y1 - B.ctr[1], y2 - B.ctr[2], kp.f0, kp.f1, kp.f2,
+                        L))
+                return;
+            fine = L.fine;
+            r = L.r;
+            rinv = 1.0 / L.r;
+            x0[0] = R(L.xi[0]);
+            x1[0] = R(L.xi[1]);
+            x2[0] = R(L.xi[2]);
+        }
+        Cx<R> val[1];
+        bool staged = false;
+        if constexpr (sizeof(R) == 4)
+            if (stage > 0)
+            {
+                const uint64_t act = __ballot(1);
+                const int rank = __popcll(act & ((1ull << lane) - 1ull));
+                const int nact = __popcll(act);
+                uint64_t rem = act;
+                int myslot = 0, nd = 0;
+                int cs[FAR_STAGE] = {};
+#pragma unroll 1
+                while (rem != 0 && nd < FAR_STAGE)
+                {
+                    const int l0 = __ffsll((unsigned long long)rem) - 1;
+                    const int f0 = __builtin_amdgcn_readlane(fine, l0);
+                    const uint64_t m = __ballot(fine == f0);
+                    if (fine == f0)
+                        myslot = nd;
+#pragma unroll
+                    for (int e = 0; e < FAR_STAGE; e++)
+                        cs[e] = nd == e ? f0 : cs[e];
+                    rem &= ~m;
+                    nd++;
+                }
+                if (rem == 0) // uniform
+                {
+                    if (kp.n_lo & 1)
+                        stage_cones<float2>(F, cs[0], cs[1], cs[2], cs[3], nd, kp.n_lo, stride,
+                                            rank, nact, sc);
+                    else
+                        stage_cones<float4>(F, cs[0], cs[1], cs[2], cs[3], nd, kp.n_lo, stride,
+                                            rank, nact, sc);
+                    wave_lds_wait();
+                    const Cx<R>* c = sc + myslot * stride;
+                    if constexpr (O0 > 0)
+                        val[0] = eval_point<R, O0, O1>(c, kp.lo2, x0[0], x1[0], x2[0]);
+                    else
+                        eval_any<R, 1>(c, kp.lo0, kp.lo1, kp.lo2, x0, x1, x2, val);
+                    staged = true;
+                    // the next source box's staging writes stay behind this box's LDS reads
+                    asm volatile("" ::: "memory");
+                }
+            }
+        if (!staged)
+        {
+            const Cx<R>* c = F + int64_t(fine) * kp.n_lo;
+            if constexpr (O0 > 0)
+                val[0] = eval_point<R, O0, O1>(c, kp.lo2, x0[0], x1[0], x2[0]);
+            else
+                eval_any<R, 1>(c, kp.lo0, kp.lo1, kp.lo2, x0, x1, x2, val);
+        }
+        Cx<R> cf;
+        if (!phase) // uniform
+            cf = {R(INV_4PI_D * rinv), R(0)};
+        else
+            cf = cscale(expmk_far<R>(B.k_re, B.k_im, r), R(INV_4PI_D * rinv));
+        acc = cadd(acc, cmul(val[0], cf));
+    };
+    // the next source box's index is loaded one box ahead, so that its geometry loads do not
+    // wait for it
+    if (ngrp == 1)
+    {
+        // uniform source box: scalar loads of its geometry
+        int32_t sn = j0 < j1 ? far_src[j0] : 0;
+        for (int32_t j = j0; j < j1; j++)
+        {
+            const int32_t sb = __builtin_amdgcn_readfirstlane(sn);
+            if (j + 1 < j1)
+                sn = far_src[j + 1];
+            body(geo[sb]);
+        }
+    }
+    else
+    {
+        int32_t sn = j0 + grp < j1 ? far_src[j0 + grp] : 0;
+        for (int32_t j = j0 + grp; j < j1; j += ngrp)
+        {
+            const int32_t sb = sn;
+            if (j + ngrp < j1)
+                sn = far_src[j + ngrp];
+            body(geo[sb]);
+        }
+        for (int m = Tp; m < 64; m <<= 1)
+        {
+            acc.x += __shfl_xor(acc.x, m, 64);
+            acc.y += __shfl_xor(acc.y, m, 64);
+        }
+    }
+    if (grp == 0 && valid)
+        result[t] = cadd(result[t], acc);
+}
 } // namespace
 
 namespace dev
@@ -493,5 +755,56 @@ template void launch_up_rows<float>(DevicePlan&, hipStream_t, const KParams&, in
                                     const Cx<float>*, Cx<float>*);
 template void launch_up_rows<double>(DevicePlan&, hipStream_t, const KParams&, int,
                                      const Cx<double>*, Cx<double>*);
+
+template <typename R>
+void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
+                     Cx<R>* res)
+{
+    const DevicePlan::FarGroup& G = D.far_groups[group];
+    const int64_t n = G.item1 - G.item0;
+    const int phase = D.kind != KL;
+    const WorkItem* items = D.far_items + G.item0;
+    const int32_t* srange = D.far_srange + 2 * G.item0;
+    if constexpr (sizeof(R) == 4)
+        if (G.ang_n > 0)
+        {
+            const int wpb = D.shape.far_waves;
+            const int stage = D.n_lo >= 40 && D.n_lo <= 400 ? D.n_lo : 0;
+            // entries from one staged cone to the next: 16-byte words, an odd number of them
+            // mod 8, so that the four cones' words start in different banks
+            const int stride = stage ? (((D.n_lo + 1) / 2) | 1) * 2 : 0;
+            const size_t lds = ((G.ang_n + 1) & ~1) * sizeof(double) +
+                               (stage ? size_t(wpb) * (FAR_STAGE * stride + ROW_PAD) * sizeof(Cx<R>)
+                                      : 0);
+            with_orders(D.lo[0], D.lo[1], [&](auto o0, auto o1)
+                        {
+                            constexpr int O0 = decltype(o0)::value, O1 = decltype(o1)::value;
+                            if (lds > size_t(64) * 1024)
+                                HIP_OK(hipFuncSetAttribute(
+                                    reinterpret_cast<const void*>(&k_far_rows<R, O0, O1, true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+                            k_far_rows<R, O0, O1, true>
+                                <<<dim3(unsigned((n + wpb - 1) / wpb)), dim3(64 * wpb), lds, st>>>(
+                                    items, n, srange, D.far_src, D.geo, D.ctab, F, D.tgt_pts,
+                                    D.fine_ang, G.ang_base, G.ang_n, stage, stride, phase, res, kp);
+                        });
+            return;
+        }
+    auto slow = [&](auto o0, auto o1)
+    {
+        constexpr int O0 = decltype(o0)::value, O1 = decltype(o1)::value;
+        k_far_rows<R, O0, O1, false><<<dim3(unsigned(n)), dim3(64), 0, st>>>(
+            items, n, srange, D.far_src, D.geo, D.ctab, F, D.tgt_pts, D.fine_ang, 0, 0, 0, 0,
+            phase, res, kp);
+    };
+    if constexpr (sizeof(R) == 4) // angle tables too large for LDS: rare
+        slow(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+    else
+        with_orders(D.lo[0], D.lo[1], slow);
+}
+template void launch_far_rows<float>(DevicePlan&, hipStream_t, const KParams&, int,
+                                     const Cx<float>*, Cx<float>*);
+template void launch_far_rows<double>(DevicePlan&, hipStream_t, const KParams&, int,
+                                      const Cx<double>*, Cx<double>*);
 } // namespace dev
 } // namespace ifgf

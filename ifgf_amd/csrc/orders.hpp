@@ -14,5 +14,9 @@ namespace dev
 template <typename R>
 void launch_up_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int level, const Cx<R>* F,
                     Cx<R>* V);
+// the far field of launch group `group`: added to the targets' results
+template <typename R>
+void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
+                     Cx<R>* res);
 } // namespace dev
 } // namespace ifgf

@@ -792,102 +792,6 @@ __global__ __launch_bounds__(256) void k_transform_t(int64_t c0, int64_t c1,
     }
 }
 
-// runtime-order version of the transform (any orders and factors)
-template <typename R>
-__global__ __launch_bounds__(256) void k_transform(int64_t c0, int64_t c1, int cpb, int xsz,
-                                                   int ysz, const ConeDev* __restrict__ cones,
-                                                   const Cx<R>* __restrict__ V,
-                                                   Cx<R>* __restrict__ F, const R* __restrict__ W,
-                                                   int w1off, int w2off, KParams kp)
-{
-    extern __shared__ unsigned char smem_raw[];
-    R* Ws = reinterpret_cast<R*>(smem_raw);
-    const int h0 = kp.ho0, h1 = kp.ho1, h2 = kp.ho2;
-    const int m0 = kp.f0 * kp.lo0, m1 = kp.f1 * kp.lo1, m2 = kp.f2 * kp.lo2;
-    const int nW = m0 * h0 + m1 * h1 + m2 * h2;
-    const int wpad = (nW + 3) & ~3;
-    Cx<R>* X = reinterpret_cast<Cx<R>*>(Ws + wpad);
-    Cx<R>* Y = X + int64_t(cpb) * xsz;
-    for (int i = threadIdx.x; i < nW; i += blockDim.x)
-        Ws[i] = W[i];
-    const int64_t first = c0 + xcd_block(kp.xlg) * cpb;
-    const int ncone = int(min<int64_t>(cpb, c1 - first));
-    const int nh = h0 * h1 * h2;
-    for (int e = threadIdx.x; e < ncone * nh; e += blockDim.x)
-    {
-        const int k = e / nh, i = e - k * nh;
-        X[k * xsz + i] = V[(first + k) * nh + i];
-    }
-    __syncthreads();
-    const R* W0 = Ws;
-    const R* W1 = Ws + w1off;
-    const R* W2 = Ws + w2off;
-    {
-        const int n = m0 * h1 * h2;
-        for (int e = threadIdx.x; e < ncone * n; e += blockDim.x)
-        {
-            const int k = e / n, i = e - k * n;
-            const int j0 = i % m0, rest = i / m0;
-            const Cx<R>* x = X + k * xsz + rest * h0;
-            Cx<R> a = {0, 0};
-            for (int t = 0; t < h0; t++)
-            {
-                const R wv = W0[j0 * h0 + t];
-                a.x += wv * x[t].x;
-                a.y += wv * x[t].y;
-            }
-            Y[k * ysz + i] = a;
-        }
-    }
-    __syncthreads();
-    {
-        const int n = m0 * m1 * h2;
-        for (int e = threadIdx.x; e < ncone * n; e += blockDim.x)
-        {
-            const int k = e / n, i = e - k * n;
-            const int j0 = i % m0, j1 = (i / m0) % m1, i2 = i / (m0 * m1);
-            const Cx<R>* y = Y + k * ysz + j0 + m0 * h1 * i2;
-            Cx<R> a = {0, 0};
-            for (int t = 0; t < h1; t++)
-            {
-                const R wv = W1[j1 * h1 + t];
-                a.x += wv * y[m0 * t].x;
-                a.y += wv * y[m0 * t].y;
-            }
-            X[k * xsz + i] = a;
-        }
-    }
-    __syncthreads();
-    {
-        const int n = m0 * m1 * m2;
-        const int lo0 = kp.lo0, lo1 = kp.lo1;
-        for (int e = threadIdx.x; e < ncone * n; e += blockDim.x)
-        {
-            const int k = e / n, i = e - k * n;
-            const int j01 = i % (m0 * m1), j2 = i / (m0 * m1);
-            const Cx<R>* x = X + k * xsz + j01;
-            Cx<R> a = {0, 0};
-            for (int t = 0; t < h2; t++)
-            {
-                const R wv = W2[j2 * h2 + t];
-                a.x += wv * x[m0 * m1 * t].x;
-                a.y += wv * x[m0 * m1 * t].y;
-            }
-            const int j0 = j01 % m0, j1 = j01 / m0;
-            const int s0 = j0 / lo0, s1 = j1 / lo1, s2 = j2 / kp.lo2;
-            const int sub = s0 + kp.f0 * (s1 + kp.f1 * s2);
-            const ConeDev cn = cones[first + k];
-            if ((cn.mask >> sub) & 1u)
-            {
-                const int slot = cn.fine_base + __popc(cn.mask & ((1u << sub) - 1u));
-                const int coef =
-                    (j0 - s0 * lo0) + lo0 * ((j1 - s1 * lo1) + lo1 * (j2 - s2 * kp.lo2));
-                F[int64_t(slot) * kp.n_lo + coef] = a;
-            }
-        }
-    }
-}
-
 // far field: for each target of the item, the interpolants of its far source boxes times the
 // centre factor (ifgfoperator.hpp:962-1012, 1708-1891).  FAST (mixed form): cones located by
 // locate_fast with the level's fine-grid angle tables (doubles [ang_base, ang_base + ang_n) of
@@ -1474,23 +1378,9 @@ void launch_transform(DevicePlan& D, hipStream_t st, const KParams& kp, int64_t 
         return;
     }
 #undef IFGF_TRANSFORM
-    const int h0 = D.ho[0], h1 = D.ho[1], h2 = D.ho[2];
-    const int m0 = D.f[0] * D.lo[0], m1 = D.f[1] * D.lo[1], m2 = D.f[2] * D.lo[2];
-    // X holds the values and the axis-1 stage, Y the axis-0 stage; axis 2 goes to memory
-    const int xsz = std::max(h0 * h1 * h2, m0 * m1 * h2);
-    const int ysz = m0 * h1 * h2;
-    const int nW = m0 * h0 + m1 * h1 + m2 * h2;
-    const size_t per_cone = size_t(xsz + ysz) * sizeof(Cx<R>);
-    const int cpb = int(std::max<size_t>(1, std::min<size_t>(8, (48 * 1024) / per_cone)));
-    const size_t smem = ((nW + 3) & ~3) * sizeof(R) + cpb * per_cone;
-    constexpr size_t LDS_MAX = 160 * 1024; // gfx950: 160 KB of LDS per CU
-    if (smem > LDS_MAX)
-        throw std::runtime_error("interpolation orders too large for the transform kernel's LDS");
-    if (smem > 64 * 1024)
-        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_transform<R>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));
-    k_transform<R><<<dim3(unsigned((c1 - c0 + cpb - 1) / cpb)), dim3(256), smem, st>>>(
-        c0, c1, cpb, xsz, ysz, D.cones, V, F, W, D.woff[1], D.woff[2], kp);
+    if (list)
+        throw std::runtime_error("transform lists are for the compiled orders");
+    launch_transform_rows<R>(D, st, kp, c0, c1, V, F);
 }
 
 // phase timing: events recorded around each segment on the mult's stream, read after the

@@ -713,6 +713,172 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
     if (grp == 0 && valid)
         result[t] = cadd(result[t], acc);
 }
+// e / n for 0 <= e < 2^16 with inv = 1 / n (the half keeps the product off the integers)
+__device__ __forceinline__ int div_small(int e, float inv)
+{
+    return int((float(e) + 0.5f) * inv);
+}
+
+// fn(H) with the high order of an axis as a compile-time constant (2 to 13; 0: any)
+template <class Fn> __device__ __forceinline__ void with_high_order(int h, const Fn& fn)
+{
+#define IFGF_H(N)                                                                               \
+    case N:                                                                                     \
+        return fn(std::integral_constant<int, N>())
+    switch (h) // uniform
+    {
+        IFGF_H(2);
+        IFGF_H(3);
+        IFGF_H(4);
+        IFGF_H(5);
+        IFGF_H(6);
+        IFGF_H(7);
+        IFGF_H(8);
+        IFGF_H(9);
+        IFGF_H(10);
+        IFGF_H(11);
+        IFGF_H(12);
+        IFGF_H(13);
+    }
+#undef IFGF_H
+    fn(std::integral_constant<int, 0>());
+}
+
+// out(j, sum_t W[j h + t] in[stride t]) for j < m: one pencil of an axis map.  H > 0 (= h): the
+// pencil's inputs in registers, the map's rows in scalar registers (uniform addresses)
+template <typename R, int H, class Out>
+__device__ __forceinline__ void map_pencil(const R* __restrict__ W, int h, int m, const Cx<R>* in,
+                                           int stride, const Out& out)
+{
+    if constexpr (H > 0)
+    {
+        Cx<R> v[H];
+#pragma unroll
+        for (int t = 0; t < H; t++)
+            v[t] = in[t * stride];
+#pragma unroll 3
+        for (int j = 0; j < m; j++)
+        {
+            Cx<R> a = {R(0), R(0)};
+#pragma unroll
+            for (int t = 0; t < H; t++)
+            {
+                const R wv = W[j * H + t];
+                a.x += wv * v[t].x;
+                a.y += wv * v[t].y;
+            }
+            out(j, a);
+        }
+    }
+    else
+        for (int j = 0; j < m; j++)
+        {
+            Cx<R> a = {R(0), R(0)};
+            for (int t = 0; t < h; t++)
+            {
+                const R wv = W[j * h + t];
+                a.x += wv * in[t * stride].x;
+                a.y += wv * in[t * stride].y;
+            }
+            out(j, a);
+        }
+}
+
+// High-order values -> fine coefficients of the active sub-cones at any orders and factors
+// (chebinterp.hpp:176-250, ifgfoperator.hpp:1539-1637), separable per axis as k_transform_t: one
+// thread per pencil and axis, cpb cones per workgroup (X: xsz entries per cone, the values, then
+// the axis-1 stage; Y: ysz, the axis-0 stage; the axis-2 stage goes to memory).  Each axis has
+// its loop compiled per number of inputs, chosen once by a uniform switch: an input is read from
+// LDS once for all its outputs and the map's entries are scalar operands, where one thread per
+// output read both from LDS for every product.  Bound by LDS and vector issue.
+// 1M points, (6,9,7)/(3,6,4): 16.8 -> 4.7 ms; torus, 131,072 points, (8,8,8)/(5,5,5): 3.8 ->
+// 0.94 ms.
+template <typename R>
+__global__ __launch_bounds__(256) void k_transform_rows(int64_t c0, int64_t c1, int cpb, int xsz,
+                                                        int ysz, const ConeDev* __restrict__ cones,
+                                                        const Cx<R>* __restrict__ V,
+                                                        Cx<R>* __restrict__ F,
+                                                        const R* __restrict__ W, KParams kp)
+{
+    extern __shared__ __align__(16) unsigned char tr_smem[];
+    Cx<R>* X = reinterpret_cast<Cx<R>*>(tr_smem);
+    Cx<R>* Y = X + cpb * xsz;
+    const int h0 = kp.ho0, h1 = kp.ho1, h2 = kp.ho2, nh = kp.n_hi;
+    const int l0 = kp.lo0, l1 = kp.lo1, l2 = kp.lo2;
+    const int m0 = kp.f0 * l0, m1 = kp.f1 * l1, m2 = kp.f2 * l2;
+    const int64_t first = c0 + xcd_block(kp.xlg) * cpb;
+    const int ncone = int(min<int64_t>(cpb, c1 - first));
+    const int tid = threadIdx.x;
+    for (int k = 0; k < ncone; k++)
+        for (int i = tid; i < nh; i += 256)
+            X[k * xsz + i] = V[(first + k) * nh + i];
+    __syncthreads();
+    const R* W1 = W + m0 * h0;
+    const R* W2 = W1 + m1 * h1;
+    {
+        const int np = h1 * h2;
+        const float inv = 1.0f / float(np);
+        with_high_order(h0, [&](auto H)
+                        {
+                            for (int e = tid; e < ncone * np; e += 256)
+                            {
+                                const int k = div_small(e, inv), p = e - k * np;
+                                Cx<R>* y = Y + k * ysz + p * m0;
+                                map_pencil<R, decltype(H)::value>(
+                                    W, h0, m0, X + k * xsz + p * h0, 1,
+                                    [&](int j, Cx<R> a) { y[j] = a; });
+                            }
+                        });
+    }
+    __syncthreads();
+    {
+        const int np = m0 * h2;
+        const float inv = 1.0f / float(np), inv0 = 1.0f / float(m0);
+        with_high_order(h1, [&](auto H)
+                        {
+                            for (int e = tid; e < ncone * np; e += 256)
+                            {
+                                const int k = div_small(e, inv), p = e - k * np;
+                                const int i2 = div_small(p, inv0), j0 = p - i2 * m0;
+                                Cx<R>* x = X + k * xsz + j0 + m0 * m1 * i2;
+                                map_pencil<R, decltype(H)::value>(
+                                    W1, h1, m1, Y + k * ysz + j0 + m0 * h1 * i2, m0,
+                                    [&](int j, Cx<R> a) { x[j * m0] = a; });
+                            }
+                        });
+    }
+    __syncthreads();
+    {
+        const int np = m0 * m1, l01 = l0 * l1;
+        const float inv = 1.0f / float(np), il0 = 1.0f / float(l0), il01 = 1.0f / float(l01),
+                    if0 = 1.0f / float(kp.f0);
+        with_high_order(h2, [&](auto H)
+                        {
+                            for (int e = tid; e < ncone * np; e += 256)
+                            {
+                                const int k = div_small(e, inv), p = e - k * np;
+                                // the pencils of one sub-cone column on consecutive lanes: their
+                                // coefficients are consecutive in memory
+                                const int s01 = div_small(p, il01), m01 = p - s01 * l01;
+                                const int s1 = div_small(s01, if0), s0 = s01 - s1 * kp.f0;
+                                const int q1 = div_small(m01, il0), q0 = m01 - q1 * l0;
+                                const int j01 = s0 * l0 + q0 + m0 * (s1 * l1 + q1);
+                                const ConeDev cn = cones[first + k];
+                                for (int s2 = 0; s2 < kp.f2; s2++)
+                                {
+                                    const int sub = s01 + kp.f0 * kp.f1 * s2;
+                                    if (!((cn.mask >> sub) & 1u))
+                                        continue;
+                                    const int rk = __popc(cn.mask & ((1u << sub) - 1u));
+                                    Cx<R>* o = F + int64_t(cn.fine_base + rk) * kp.n_lo + m01;
+                                    map_pencil<R, decltype(H)::value>(
+                                        W2 + s2 * l2 * h2, h2, l2, X + k * xsz + j01, np,
+                                        [&](int j, Cx<R> a) { o[l01 * j] = a; });
+                                }
+                            }
+                        });
+    }
+}
 } // namespace
 
 namespace dev
@@ -806,5 +972,32 @@ template void launch_far_rows<float>(DevicePlan&, hipStream_t, const KParams&, i
                                      const Cx<float>*, Cx<float>*);
 template void launch_far_rows<double>(DevicePlan&, hipStream_t, const KParams&, int,
                                       const Cx<double>*, Cx<double>*);
+
+template <typename R>
+void launch_transform_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int64_t c0, int64_t c1,
+                           const Cx<R>* V, Cx<R>* F)
+{
+    const int h0 = D.ho[0], h1 = D.ho[1], h2 = D.ho[2];
+    const int m0 = D.f[0] * D.lo[0], m1 = D.f[1] * D.lo[1];
+    const int xsz = std::max(h0 * h1 * h2, m0 * m1 * h2);
+    const int ysz = m0 * h1 * h2;
+    const size_t per_cone = size_t(xsz + ysz) * sizeof(Cx<R>);
+    // several cones fill the threads where one cone's pencils do not; 32 KB keeps 5 workgroups
+    // per CU
+    const int cpb = int(std::max<size_t>(1, std::min<size_t>(8, (32 * 1024) / per_cone)));
+    const size_t lds = cpb * per_cone;
+    constexpr size_t LDS_MAX = 160 * 1024; // gfx950: 160 KB of LDS per CU
+    if (lds > LDS_MAX)
+        throw std::runtime_error("interpolation orders too large for the transform kernel's LDS");
+    if (lds > size_t(64) * 1024)
+        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_transform_rows<R>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    k_transform_rows<R><<<dim3(unsigned((c1 - c0 + cpb - 1) / cpb)), dim3(256), lds, st>>>(
+        c0, c1, cpb, xsz, ysz, D.cones, V, F, static_cast<const R*>(D.wmat), kp);
+}
+template void launch_transform_rows<float>(DevicePlan&, hipStream_t, const KParams&, int64_t,
+                                           int64_t, const Cx<float>*, Cx<float>*);
+template void launch_transform_rows<double>(DevicePlan&, hipStream_t, const KParams&, int64_t,
+                                            int64_t, const Cx<double>*, Cx<double>*);
 } // namespace dev
 } // namespace ifgf

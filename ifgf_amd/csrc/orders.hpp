@@ -1,5 +1,6 @@
 // orders.hpp -- launchers of the kernels that take the interpolation orders at run time
-// (orders.hip): the upward pass over the grouped tables for any orders in both precisions.
+// (orders.hip): the upward pass over the grouped tables, the far field and the values ->
+// coefficients transform, for any orders in both precisions.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -18,5 +19,9 @@ void launch_up_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int level,
 template <typename R>
 void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
                      Cx<R>* res);
+// the values V -> the fine coefficients F of cones [c0, c1)
+template <typename R>
+void launch_transform_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int64_t c0, int64_t c1,
+                           const Cx<R>* V, Cx<R>* F);
 } // namespace dev
 } // namespace ifgf

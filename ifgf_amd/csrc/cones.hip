@@ -2,9 +2,9 @@
 // util.hpp:156-171 cartToInterp2, cone_domain.hpp:232-256 elementForPoint).
 //
 // Per source level, after the host has laid out the level's grids and bitmaps:
-//   k_mark_far     one workgroup per (source box, far target box) pair: every target point's
-//                  fine and coarse cells of the source box's grids, or'ed into the bitmaps
-//   k_mark_parent  one workgroup per box whose parent has far work: every high-order node of
+//   k_mark_far     a workgroup per run of far target boxes of one source box: every target point's
+//                  fine and coarse cells of the source box's grids, set in its bitmaps
+//   k_mark_parent  workgroups per box whose parent has far work: every high-order node of
 //                  every active coarse cone of the parent, located in the box's grids (from
 //                  the parent level's upward table where the host built one, otherwise by
 //                  the FP64 cone map), or'ed into the bitmaps
@@ -106,43 +106,111 @@ __device__ __forceinline__ int64_t grid_cell(const double p[3], const double lo[
     return id;
 }
 
+// Bits go to a workgroup's copy of its box's bitmaps in LDS (where most points find their cell
+// marked already: the word is read first), whose words are or'ed into memory once at the end.
+// Straight into memory, the level's few words are contended by all its threads: 32,768 points,
+// k_mark_far took 1.4 ms per launch (0.05 ms now), and longer with more threads; 1M points, level 5:
+// 39 -> 8 ms for the level's marking.  Boxes whose bitmaps exceed
+// MARK_WORDS mark in memory.
+constexpr int MARK_WORDS = 4096; // 32 KB
 __device__ __forceinline__ void set_bit(unsigned long long* words, int64_t c)
 {
-    atomicOr(words + (c >> 6), 1ull << (c & 63));
+    const unsigned long long bit = 1ull << (c & 63);
+    if (!(words[c >> 6] & bit))
+        atomicOr(words + (c >> 6), bit);
 }
 
-__device__ __forceinline__ void mark_point(const MarkBox& B, const double s[3],
-                                           unsigned long long* fbits,
-                                           unsigned long long* cbits)
+// the box's bitmaps while a workgroup marks: in LDS when they fit
+struct MarkBits
+{
+    unsigned long long *f, *c; // the box's fine and coarse words
+    unsigned long long *gf, *gc;
+    int nf, nc;
+    bool lds;
+    __device__ MarkBits(unsigned long long* sw, unsigned long long* fbits,
+                        unsigned long long* cbits, int64_t foff, int64_t coff, int64_t fcells,
+                        int64_t ccells)
+        : gf(fbits + foff), gc(cbits + coff), nf(int((fcells + 63) / 64)),
+          nc(int((ccells + 63) / 64)), lds((fcells + 63) / 64 + (ccells + 63) / 64 <= MARK_WORDS)
+    {
+        f = lds ? sw : gf;
+        c = lds ? sw + nf : gc;
+        if (lds)
+            for (int i = threadIdx.x; i < nf + nc; i += int(blockDim.x))
+                sw[i] = 0;
+        __syncthreads();
+    }
+    __device__ void flush() const
+    {
+        __syncthreads();
+        if (!lds)
+            return;
+        for (int i = threadIdx.x; i < nf + nc; i += int(blockDim.x))
+        {
+            const unsigned long long w = i < nf ? f[i] : c[i - nf];
+            unsigned long long* g = i < nf ? gf + i : gc + (i - nf);
+            if (w & ~*g)
+                atomicOr(g, w);
+        }
+    }
+};
+
+__device__ __forceinline__ void mark_point(const MarkBox& B, const double s[3], const MarkBits& M)
 {
     const int64_t cf = grid_cell(s, B.lo, B.hi, B.hf, B.nf);
     const int64_t cc = grid_cell(s, B.lo, B.hi, B.hc, B.nc);
     if (cc >= 0)
-        set_bit(cbits + B.coff, cc);
+        set_bit(M.c, cc);
     if (cf >= 0)
-        set_bit(fbits + B.foff, cf);
+        set_bit(M.f, cf);
 }
 
-__global__ __launch_bounds__(256) void k_mark_far(const MarkBox* __restrict__ boxes,
-                                                 const int32_t* __restrict__ pair_box,
+__device__ __forceinline__ int64_t cells(const int32_t n[3])
+{
+    return int64_t(n[0]) * n[1] * n[2];
+}
+
+// far target points of one source box: whole target boxes ra .. rb, or (rb = ra + 1) the points
+// [i0, i1) of one, about MARK_POINTS of them
+struct FarMark
+{
+    int32_t q, ra, rb, pad;
+    int64_t i0, i1;
+};
+constexpr int64_t MARK_POINTS = 4096;
+
+__global__ __launch_bounds__(256) void k_mark_far(const FarMark* __restrict__ items,
+                                                 const MarkBox* __restrict__ boxes,
                                                  const int32_t* __restrict__ pair_tgt,
                                                  const int64_t* __restrict__ tbeg,
                                                  const int64_t* __restrict__ tend,
                                                  const double* __restrict__ tpts,
-                                                 unsigned long long* __restrict__ fbits,
-                                                 unsigned long long* __restrict__ cbits)
+                                                 unsigned long long* fbits,
+                                                 unsigned long long* cbits)
 {
-    const int64_t r = blockIdx.x;
-    const MarkBox B = boxes[pair_box[r]];
-    const int32_t t = pair_tgt[r];
-    const int64_t i1 = tend[t];
-    for (int64_t i = tbeg[t] + threadIdx.x; i < i1; i += 256)
+    __shared__ unsigned long long sw[MARK_WORDS];
+    const FarMark W = items[blockIdx.x];
+    const MarkBox B = boxes[W.q];
+    const MarkBits M(sw, fbits, cbits, B.foff, B.coff, cells(B.nf), cells(B.nc));
+    auto point = [&](int64_t i)
     {
         const double x[3] = {tpts[3 * i], tpts[3 * i + 1], tpts[3 * i + 2]};
         double s[3];
         cart_to_interp_exact(x, B.ctr, B.H, s);
-        mark_point(B, s, fbits, cbits);
-    }
+        mark_point(B, s, M);
+    };
+    if (W.rb == W.ra + 1)
+        for (int64_t i = W.i0 + threadIdx.x; i < W.i1; i += 256)
+            point(i);
+    else // small target boxes: a wave each
+        for (int32_t r = W.ra + int(threadIdx.x >> 6); r < W.rb; r += 4)
+        {
+            const int32_t t = pair_tgt[r];
+            const int64_t e = tend[t];
+            for (int64_t i = tbeg[t] + (threadIdx.x & 63); i < e; i += 64)
+                point(i);
+        }
+    M.flush();
 }
 
 // tab_fc: (fine, coarse) of the parent level's upward-table entries, ((u * n_ho) + node) * 8
@@ -152,12 +220,14 @@ __global__ __launch_bounds__(256) void k_mark_parent(
     const MarkBox* __restrict__ boxes, const ParentWork* __restrict__ work,
     const int32_t* __restrict__ tab_fc, const int32_t* __restrict__ cone_u,
     const int64_t* __restrict__ cone_cell, const double* __restrict__ ho_nodes, int n_ho,
-    int use_table, unsigned long long* __restrict__ fbits, unsigned long long* __restrict__ cbits)
+    int use_table, unsigned long long* fbits, unsigned long long* cbits)
 {
+    __shared__ unsigned long long sw[MARK_WORDS];
     const ParentWork W = work[blockIdx.x];
     const MarkBox B = boxes[W.q];
+    const MarkBits M(sw, fbits, cbits, B.foff, B.coff, cells(B.nf), cells(B.nc));
     const int64_t n = (W.c1 - W.c0) * n_ho;
-    for (int64_t e = threadIdx.x; e < n; e += 256)
+    for (int64_t e = int64_t(blockIdx.y) * 256 + threadIdx.x; e < n; e += int64_t(gridDim.y) * 256)
     {
         const int64_t c = W.c0 + e / n_ho;
         const int k = int(e % n_ho);
@@ -168,8 +238,8 @@ __global__ __launch_bounds__(256) void k_mark_parent(
             if (fine >= 0)
             {
                 if (coarse >= 0)
-                    set_bit(cbits + B.coff, coarse);
-                set_bit(fbits + B.foff, fine);
+                    set_bit(M.c, coarse);
+                set_bit(M.f, fine);
             }
             continue;
         }
@@ -188,8 +258,9 @@ __global__ __launch_bounds__(256) void k_mark_parent(
         double y[3], s[3];
         interp_to_cart_exact(sp, W.pctr, W.pH, y);
         cart_to_interp_exact(y, B.ctr, B.H, s);
-        mark_point(B, s, fbits, cbits);
+        mark_point(B, s, M);
     }
+    M.flush();
 }
 
 // device buffers kept across the levels of one build_cones
@@ -197,7 +268,7 @@ struct MarkerState
 {
     bool ready = false;
     DBuf tpts, tbeg, tend, far_tgt, ho;
-    DBuf boxes, pair_box, fbits, cbits, work, tab_fc, cone_u, cone_cell;
+    DBuf boxes, far_items, fbits, cbits, work, tab_fc, cone_u, cone_cell;
 };
 
 void mark_level(MarkerState& st, const Plan& P, int level, const std::vector<int64_t>& far_off,
@@ -238,10 +309,30 @@ void mark_level(MarkerState& st, const Plan& P, int level, const std::vector<int
     }
     // far pairs of the level's boxes: far_tgt[far_off[l0] .. far_off[l1]) in box order
     const int64_t r0 = far_off[l0], r1 = far_off[l1];
-    std::vector<int32_t> pair_box(r1 - r0);
+    std::vector<FarMark> items;
     for (int64_t q = 0; q < nl; q++)
+    {
+        int64_t n = 0; // points of the open run of target boxes
         for (int64_t r = far_off[l0 + q]; r < far_off[l0 + q + 1]; r++)
-            pair_box[r - r0] = int32_t(q);
+        {
+            const int64_t b = T.begin[far_tgt[r]], e = T.end[far_tgt[r]];
+            if (e - b > MARK_POINTS / 4)
+            {
+                for (int64_t i = b; i < e; i += MARK_POINTS)
+                    items.push_back({int32_t(q), int32_t(r - r0), int32_t(r - r0 + 1), 0, i,
+                                     std::min(e, i + MARK_POINTS)});
+                n = 0;
+                continue;
+            }
+            if (n == 0 || n + (e - b) > MARK_POINTS)
+            {
+                items.push_back({int32_t(q), int32_t(r - r0), int32_t(r - r0), 0, b, e});
+                n = 0;
+            }
+            items.back().rb = int32_t(r - r0 + 1);
+            n += e - b;
+        }
+    }
     // parent work
     std::vector<ParentWork> work;
     const UpLevel* U = level > 0 ? &P.up[level - 1] : nullptr;
@@ -288,9 +379,9 @@ void mark_level(MarkerState& st, const Plan& P, int level, const std::vector<int
         HIP_OK(hipMemset(st.cbits.p, 0, sizeof(uint64_t) * lb.cbits.size()));
     if (r1 > r0)
     {
-        h2d(st.pair_box, pair_box.data(), pair_box.size());
-        k_mark_far<<<dim3(unsigned(r1 - r0)), dim3(256)>>>(
-            st.boxes.as<MarkBox>(), st.pair_box.as<int32_t>(), st.far_tgt.as<int32_t>() + r0,
+        h2d(st.far_items, items.data(), items.size());
+        k_mark_far<<<dim3(unsigned(items.size())), dim3(256)>>>(
+            st.far_items.as<FarMark>(), st.boxes.as<MarkBox>(), st.far_tgt.as<int32_t>() + r0,
             st.tbeg.as<int64_t>(), st.tend.as<int64_t>(), st.tpts.as<double>(),
             st.fbits.as<unsigned long long>(), st.cbits.as<unsigned long long>());
         HIP_OK(hipGetLastError());
@@ -318,7 +409,13 @@ void mark_level(MarkerState& st, const Plan& P, int level, const std::vector<int
         else
             h2d(st.cone_cell, P.cone_cell.data() + pc_base, size_t(npc));
         (void)p0;
-        k_mark_parent<<<dim3(unsigned(work.size())), dim3(256)>>>(
+        // levels of few boxes: several workgroups per box, about 16 nodes per thread, to fill the
+        // chip
+        int64_t most = 0;
+        for (const ParentWork& W : work)
+            most = std::max(most, (W.c1 - W.c0) * n_ho);
+        const unsigned split = unsigned(std::min<int64_t>(256, std::max<int64_t>(1, most / 4096)));
+        k_mark_parent<<<dim3(unsigned(work.size()), split), dim3(256)>>>(
             st.boxes.as<MarkBox>(), st.work.as<ParentWork>(), st.tab_fc.as<int32_t>(),
             st.cone_u.as<int32_t>(), st.cone_cell.as<int64_t>(), st.ho.as<double>(), n_ho,
             table ? 1 : 0, st.fbits.as<unsigned long long>(), st.cbits.as<unsigned long long>());

@@ -1050,7 +1050,7 @@ void run_batched_core(DevicePlan& D, hipStream_t st)
     // near and far fields as in the single-column mult (SidePipe)
     const int overlap = D.n_near_items ? D.shape.overlap : 0;
     auto pipe = side_pipe(
-        D, st, overlap,
+        D, D.far_groups, st, overlap,
         [&](hipStream_t s)
         {
             if (D.n_near_items)

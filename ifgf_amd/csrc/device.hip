@@ -48,23 +48,30 @@ __global__ void k_gather(const double* __restrict__ w_in, const int64_t* __restr
     w_out[i] = {R(w_in[2 * j]), R(im_sign * w_in[2 * j + 1])};
 }
 
+// the near field's results plus the far field's of each target level, in order
 template <typename R>
-__global__ void k_scatter(const Cx<R>* __restrict__ res, const int64_t* __restrict__ perm,
-                          double* __restrict__ out, int64_t n, double re_sign, double im_sign)
+__global__ void k_scatter(const Cx<R>* __restrict__ res, const Cx<R>* __restrict__ far, int nlvl,
+                          const int64_t* __restrict__ perm, double* __restrict__ out, int64_t n,
+                          double re_sign, double im_sign)
 {
     int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
     const int64_t j = perm[i];
-    out[2 * j] = re_sign * double(res[i].x);
-    out[2 * j + 1] = im_sign * double(res[i].y);
+    Cx<R> u = res[i];
+    for (int l = 0; l < nlvl; l++)
+        u = cadd(u, far[l * n + i]);
+    out[2 * j] = re_sign * double(u.x);
+    out[2 * j + 1] = im_sign * double(u.y);
 }
 
-template <typename R> __global__ void k_zero(Cx<R>* p, int64_t n)
+template <typename R> __global__ void k_zero(Cx<R>* p, int64_t n, Cx<R>* q, int64_t nq)
 {
     int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n)
         p[i] = {R(0), R(0)};
+    else if (i - n < nq)
+        q[i - n] = {R(0), R(0)};
 }
 
 
@@ -819,15 +826,19 @@ __attribute__((amdgpu_waves_per_eu(FAST && sizeof(R) == 4 ? (O1 == 3 ? 8 : 4) : 
                                             const Cx<R>* __restrict__ F,
                                             const double* __restrict__ tpts,
                                             const double* __restrict__ ang, int ang_base,
-                                            int ang_n, Cx<R>* __restrict__ result, KParams kp)
+                                            int ang_n, int split, int64_t ntgt,
+                                            Cx<R>* __restrict__ far_res, KParams kp)
 {
     extern __shared__ double sang[];
+    __shared__ Cx<R> psum[WPB > 1 ? WPB : 1][WPB > 1 ? 64 : 1];
     __shared__ float4 fstage[WPB][FAST && O0 * O1 * O2 >= 50 ? FAR_STAGE * (O0 * O1 * O2 / 2) : 1];
-    // WPB waves per workgroup, one item each, sharing the staged angle tables (one copy per
-    // workgroup: the tables, not the registers, would otherwise bound the waves per CU)
+    // WPB waves per workgroup, sharing the staged angle tables (one copy per workgroup: the
+    // tables, not the registers, would otherwise bound the waves per CU): one item each, or
+    // (split) a run each of one item's sources
     const int lane = WPB == 1 ? int(threadIdx.x) : int(threadIdx.x & 63);
-    const int64_t it =
-        WPB == 1 ? xcd_block(kp.xlg) : xcd_block(kp.xlg) * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = WPB == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool shared = WPB > 1 && split;
+    const int64_t it = shared ? xcd_block(kp.xlg) : xcd_block(kp.xlg) * WPB + wave;
     if (WPB == 1 && it >= nitems)
         return;
     if constexpr (FAST)
@@ -846,7 +857,13 @@ __attribute__((amdgpu_waves_per_eu(FAST && sizeof(R) == 4 ? (O1 == 3 ? 8 : 4) : 
     const int64_t t = int64_t(wi.first) + (valid ? ti : 0);
     const double y0 = tpts[3 * t], y1 = tpts[3 * t + 1], y2 = tpts[3 * t + 2];
     Cx<R> acc = {0, 0};
-    const int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
+    int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
+    if (shared)
+    {
+        const int32_t n = j1 - j0, a = j0;
+        j0 = a + n * wave / WPB;
+        j1 = a + n * (wave + 1) / WPB;
+    }
     auto body = [&](const BoxGeo& B)
     {
         int fine;
@@ -1002,8 +1019,22 @@ __attribute__((amdgpu_waves_per_eu(FAST && sizeof(R) == 4 ? (O1 == 3 ? 8 : 4) : 
             acc.y += __shfl_xor(acc.y, m, 64);
         }
     }
+    if constexpr (WPB > 1)
+        if (shared)
+        {
+            psum[wave][lane] = acc;
+            __syncthreads();
+            if (wave)
+                return;
+#pragma unroll
+            for (int w = 1; w < WPB; w++)
+                acc = cadd(acc, psum[w][lane]);
+        }
     if (grp == 0 && valid)
-        result[t] = cadd(result[t], acc);
+    {
+        Cx<R>* res = far_res + wi.pad * ntgt + t;
+        *res = cadd(*res, acc);
+    }
 }
 
 // ------------------------------------------------------------------------------------
@@ -1222,34 +1253,41 @@ void launch_up_far_t(DevicePlan& D, hipStream_t st, const KParams& kp, const Nod
             launch_far_rows<R>(D, st, kp, far_level, F, res);
         else
         {
-            const int abase = D.far_groups[far_level].ang_base, an = D.far_groups[far_level].ang_n;
+            const int abase = D.far_steps[far_level].ang_base, an = D.far_steps[far_level].ang_n;
             const int64_t n = b - a;
+            // few items: 2 to 8 waves share an item's sources, else the shape's waves take an
+            // item each
+            const int split = far_split(n);
 #define IFGF_FAR(FAST, WPB, LDS, BASE, AN)                                                      \
     k_far<PH, R, O0, O1, O2, FAST, WPB, DEC>                                                    \
-        <<<dim3(unsigned((n + WPB - 1) / WPB)), dim3(64 * WPB), LDS, st>>>(                     \
+        <<<dim3(unsigned(split > 1 ? n : (n + WPB - 1) / WPB)), dim3(64 * WPB), LDS, st>>>(     \
             D.far_items + a, n, D.far_srange + 2 * a, D.far_src, D.geo, D.ctab, F, D.tgt_pts,   \
-            D.fine_ang, BASE, AN, res, kp)
+            D.fine_ang, BASE, AN, split > 1, D.ntgt, res, kp)
+#define IFGF_FAR_W(FAST, WAVES, LDS, BASE, AN)                                                  \
+    switch (WAVES)                                                                              \
+    {                                                                                           \
+    case 2:                                                                                     \
+        IFGF_FAR(FAST, 2, LDS, BASE, AN);                                                       \
+        break;                                                                                  \
+    case 4:                                                                                     \
+        IFGF_FAR(FAST, 4, LDS, BASE, AN);                                                       \
+        break;                                                                                  \
+    case 8:                                                                                     \
+        IFGF_FAR(FAST, 8, LDS, BASE, AN);                                                       \
+        break;                                                                                  \
+    default:                                                                                    \
+        IFGF_FAR(FAST, 1, LDS, BASE, AN);                                                       \
+    }
             if constexpr (sizeof(R) == 4)
                 if (an > 0)
                 {
                     const size_t lds = size_t(an) * sizeof(double);
-                    switch (D.shape.far_waves)
-                    {
-                    case 2:
-                        IFGF_FAR(true, 2, lds, abase, an);
-                        break;
-                    case 8:
-                        IFGF_FAR(true, 8, lds, abase, an);
-                        break;
-                    case 4:
-                        IFGF_FAR(true, 4, lds, abase, an);
-                        break;
-                    default:
-                        IFGF_FAR(true, 1, lds, abase, an);
-                    }
+                    const int waves = split > 1 ? split : D.shape.far_waves;
+                    IFGF_FAR_W(true, waves, lds, abase, an);
                     return;
                 }
-            IFGF_FAR(false, 1, 0, 0, 0);
+            IFGF_FAR_W(false, split, 0, 0, 0);
+#undef IFGF_FAR_W
 #undef IFGF_FAR
         }
     }
@@ -1513,9 +1551,12 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
     // the shape asks for it; phase timing runs everything in order on one stream)
     const int overlap = (pt.on || !D.n_near_items || !sg.side) ? 0 : D.shape.overlap;
     pt.begin(0);
-    k_zero<R><<<dim3(unsigned((D.ntgt + 255) / 256)), dim3(256), 0, st>>>(res, D.ntgt);
+    Cx<R>* far_res = static_cast<Cx<R>*>(D.far_res);
+    const int64_t nfar = D.ntgt * D.n_far_lvls;
+    k_zero<R><<<dim3(unsigned((D.ntgt + nfar + 255) / 256)), dim3(256), 0, st>>>(res, D.ntgt,
+                                                                                far_res, nfar);
     auto pipe = side_pipe(
-        D, st, overlap,
+        D, D.far_steps, st, overlap,
         [&](hipStream_t s)
         {
             if (D.n_near_items)
@@ -1525,9 +1566,9 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
         },
         [&](int g, hipStream_t s)
         {
-            const DevicePlan::FarGroup& G = D.far_groups[g];
+            const DevicePlan::FarGroup& G = D.far_steps[g];
             launch_up_far<PH, R, DEC>(D, s, kp, tabs, -1, g, G.item0, G.item1, Fl(G.src_level), V,
-                                 res);
+                                      far_res);
         });
     if (overlap != 1)
         pipe.fork(); // the near field first, on the main stream (inside the timed near phase)
@@ -1627,7 +1668,8 @@ void run_mult(DevicePlan& D, const double* w_dev, double* out_dev, hipStream_t s
         run_core<KIND, R>(D, st, pt, sg);
     pt.begin(0);
     k_scatter<R><<<dim3(unsigned((D.ntgt + 255) / 256)), dim3(256), 0, st>>>(
-        res, D.tgt_perm, out_dev, D.ntgt, out_re, out_im);
+        res, static_cast<const Cx<R>*>(D.far_res), D.n_far_lvls, D.tgt_perm, out_dev, D.ntgt, out_re,
+        out_im);
     pt.end();
     HIP_OK(hipGetLastError());
     pt.finish(D.last_ms);
@@ -1713,7 +1755,7 @@ void device_free(DevicePlan& D)
                     D.up_items_k[0], D.up_items_k[1], D.up_items_k[2], D.up_items_k[3],
                     D.up_glist, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
-                    D.near_off, D.near_src, D.far_items, D.near_items, D.wsorted, D.result, D.V,
+                    D.near_off, D.near_src, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
                     D.b_out, D.h_in, D.h_out};
     for (void* p : ptrs)
@@ -2082,8 +2124,8 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
             D.up_item_off_k[kc][D.levels] = int64_t(uitems[kc].size());
             D.up_items_k[kc] = dupload(uitems[kc], tot);
         }
-        D.up_items = D.up_items_k[3]; // the default shape: 16 cones per item
-        D.up_item_off = D.up_item_off_k[3];
+        D.up_items = D.up_items_k[0]; // the default shape: 2 cones per item
+        D.up_item_off = D.up_item_off_k[0];
         D.up_glist = dupload(glist, tot);
         if (!tl_glist.empty())
         {
@@ -2204,9 +2246,15 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         std::vector<WorkItem> fitems;
         std::vector<int32_t> frange;
         D.far_groups.clear();
+        D.far_steps.clear();
         std::vector<std::vector<int32_t>> tb_of_level(P.T.levels);
         for (int32_t t : ftb)
             tb_of_level[P.T.level_of(t)].push_back(t);
+        std::vector<int32_t> far_lvl(P.T.levels, -1); // index among the target levels with far work
+        D.n_far_lvls = 0;
+        for (int l = 0; l < P.T.levels; l++)
+            if (!tb_of_level[l].empty())
+                far_lvl[l] = D.n_far_lvls++;
         for (int sl = P.S.levels - 1; sl >= 0; sl--)
             for (int tl = P.T.levels - 1; tl >= 0; tl--)
             {
@@ -2233,7 +2281,8 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                     const int64_t s0 = P.T.begin[t], e0 = P.T.end[t];
                     for (int64_t f = s0; f < e0; f += 64)
                     {
-                        fitems.push_back({t, int32_t(f), int32_t(std::min<int64_t>(64, e0 - f)), 0});
+                        fitems.push_back({t, int32_t(f), int32_t(std::min<int64_t>(64, e0 - f)),
+                                          far_lvl[tl]});
                         frange.push_back(j0);
                         frange.push_back(j);
                     }
@@ -2246,6 +2295,28 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                 D.far_groups.push_back({i0, int64_t(fitems.size()), fits ? int(lo) : 0,
                                         fits ? int(hi - lo) : 0, sl, tl});
             }
+        // the groups of a source level as one launch where their angle tables fit together
+        for (const auto& G : D.far_groups)
+        {
+            if (!D.far_steps.empty() && D.far_steps.back().src_level == G.src_level &&
+                (D.far_steps.back().ang_n > 0) == (G.ang_n > 0))
+            {
+                DevicePlan::FarGroup& L = D.far_steps.back();
+                const int lo = std::min(L.ang_base, G.ang_base);
+                const int n = std::max(L.ang_base + L.ang_n, G.ang_base + G.ang_n) - lo;
+                if (n * int(sizeof(double)) <= 48 * 1024)
+                {
+                    L.item1 = G.item1;
+                    if (L.ang_n > 0)
+                    {
+                        L.ang_base = lo;
+                        L.ang_n = n;
+                    }
+                    continue;
+                }
+            }
+            D.far_steps.push_back(G);
+        }
         D.far_srange = dupload(frange, tot);
         D.far_items = dupload(fitems, tot);
         auto nitems = make_items(ntb, P.T);
@@ -2255,6 +2326,7 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         const size_t cs = precision == PREC_FP64 ? 16 : 8;
         D.wsorted = dalloc<unsigned char>(cs * D.nsrc, tot);
         D.result = dalloc<unsigned char>(cs * D.ntgt, tot);
+        D.far_res = dalloc<unsigned char>(cs * D.ntgt * D.n_far_lvls, tot);
         const size_t full = cs * (size_t(std::max<int64_t>(1, D.n_cones)) * D.n_hi +
                                   size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo);
         size_t v_lvl = 1, f_lvl[2] = {1, 1};

@@ -60,14 +60,15 @@ struct WorkItem // a chunk of at most 64 consecutive target points of one target
 };
 
 // Launch shapes of the mult's kernels: choices that change speed but not results, picked by
-// device_autotune (measured on the operator itself) or set by the caller.
+// device_autotune (measured on the operator itself) or set by the caller.  The defaults at 1M
+// points, (6,9,7)/(3,6,4): 24.7 ms per mult; with 16 upward cones 25.4, with 1 far wave 25.8.
 struct LaunchShape
 {
     int xcd_log2 = 4; // work items dealt to the XCDs in runs of 2^xcd_log2 (0: plain order)
     int cpb = 0;      // transform: cones per workgroup (0: the order class's default)
-    int up_k = 16;    // upward: parent cones of one cell per workgroup (2, 4, 8 or 16)
+    int up_k = 2;     // upward: parent cones per workgroup (2, 4, 8 or 16)
     int rb = 0;       // batched: columns per pass (8 or 32; 0: 8 up to 8 columns, else 32)
-    int far_waves = 1; // mixed far field: waves (items) per workgroup sharing the LDS tables
+    int far_waves = 2; // mixed far field: waves (items) per workgroup sharing the LDS tables
     int overlap = 1;   // far field on a second stream beside the upward chain, with the near
                        // field there too (1) or first on the main stream (2); 0: one stream
 };
@@ -183,6 +184,14 @@ struct DevicePlan
         int src_level, tgt_level;
     };
     std::vector<FarGroup> far_groups;
+    // the single-column mult's far launches: the groups of one source level together (a group
+    // each where their angle tables would not fit LDS together).  The groups of a launch run
+    // side by side, so the items of target level t (WorkItem::pad: its index among the target
+    // levels with far items) add to their own results, far_res[pad * ntgt ..], and the scatter
+    // sums the levels in order.
+    std::vector<FarGroup> far_steps;
+    int n_far_lvls = 0;
+    void* far_res = nullptr; // n_far_lvls * ntgt complex (R)
     WorkItem* near_items = nullptr;
     int64_t n_near_items = 0;
 

@@ -544,8 +544,9 @@ __device__ __forceinline__ void stage_cones(const Cx<float>* __restrict__ F, int
 }
 
 // Far field at any orders (ifgfoperator.hpp:962-1012, 1708-1891): for each target of the item,
-// the interpolants of its far source boxes times the centre factor.  One wave per item, the
-// waves of a workgroup sharing the group's angle tables in LDS (FAST: cones located by
+// the interpolants of its far source boxes times the centre factor.  One wave per item, or
+// (split) all waves of the workgroup a run each of one item's sources, their sums added in order;
+// the waves share the launch's angle tables in LDS (FAST: cones located by
 // locate_fast; otherwise the exact locate).  With stage > 0 (cones of stage coefficients and
 // more) the distinct cones of the wave's lanes, up to FAR_STAGE, are copied to LDS by all lanes
 // together and each lane reads its own there, `stride` entries apart so that the same
@@ -562,7 +563,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const Cx<R>* __restrict__ F,
     const double* __restrict__ tpts, const double* __restrict__ ang, int ang_base, int ang_n,
-    int stage, int stride, int phase, Cx<R>* __restrict__ result, KParams kp)
+    int stage, int stride, int phase, int split, int64_t ntgt, Cx<R>* __restrict__ far_res,
+    KParams kp)
 {
     extern __shared__ __align__(16) unsigned char far_smem[];
     double* sang = reinterpret_cast<double*>(far_smem);
@@ -570,7 +572,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
     const int wpb = int(blockDim.x >> 6);
     Cx<R>* sc = reinterpret_cast<Cx<R>*>(far_smem + ((ang_n + 1) & ~1) * sizeof(double)) +
                 wave * (FAR_STAGE * stride + ROW_PAD);
-    const int64_t it = xcd_block(kp.xlg) * wpb + wave;
+    const int64_t it = split ? xcd_block(kp.xlg) : xcd_block(kp.xlg) * wpb + wave;
     if constexpr (FAST)
     {
         for (int i = threadIdx.x; i < ang_n; i += int(blockDim.x))
@@ -587,7 +589,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
     const int64_t t = int64_t(wi.first) + (valid ? ti : 0);
     const double y0 = tpts[3 * t], y1 = tpts[3 * t + 1], y2 = tpts[3 * t + 2];
     Cx<R> acc = {0, 0};
-    const int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
+    int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
+    if (split) // a run of the item's sources per wave
+    {
+        const int32_t n = j1 - j0, a = j0;
+        j0 = a + n * wave / wpb;
+        j1 = a + n * (wave + 1) / wpb;
+    }
     auto body = [&](const BoxGeo& B)
     {
         int fine;
@@ -710,8 +718,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
             acc.y += __shfl_xor(acc.y, m, 64);
         }
     }
+    if (split)
+    {
+        __shared__ Cx<R> psum[8][64];
+        psum[wave][lane] = acc;
+        __syncthreads();
+        if (wave)
+            return;
+        for (int w = 1; w < wpb; w++)
+            acc = cadd(acc, psum[w][lane]);
+    }
     if (grp == 0 && valid)
-        result[t] = cadd(result[t], acc);
+    {
+        Cx<R>* res = far_res + wi.pad * ntgt + t;
+        *res = cadd(*res, acc);
+    }
 }
 // e / n for 0 <= e < 2^16 with inv = 1 / n (the half keeps the product off the integers)
 __device__ __forceinline__ int div_small(int e, float inv)
@@ -924,17 +945,18 @@ template void launch_up_rows<double>(DevicePlan&, hipStream_t, const KParams&, i
 
 template <typename R>
 void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
-                     Cx<R>* res)
+                     Cx<R>* far_res)
 {
-    const DevicePlan::FarGroup& G = D.far_groups[group];
+    const DevicePlan::FarGroup& G = D.far_steps[group];
     const int64_t n = G.item1 - G.item0;
+    const int split = far_split(n);
     const int phase = D.kind != KL;
     const WorkItem* items = D.far_items + G.item0;
     const int32_t* srange = D.far_srange + 2 * G.item0;
     if constexpr (sizeof(R) == 4)
         if (G.ang_n > 0)
         {
-            const int wpb = D.shape.far_waves;
+            const int wpb = split > 1 ? split : D.shape.far_waves;
             const int stage = D.n_lo >= 40 && D.n_lo <= 400 ? D.n_lo : 0;
             // entries from one staged cone to the next: 16-byte words, an odd number of them
             // mod 8, so that the four cones' words start in different banks
@@ -950,18 +972,20 @@ void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group
                                     reinterpret_cast<const void*>(&k_far_rows<R, O0, O1, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
                             k_far_rows<R, O0, O1, true>
-                                <<<dim3(unsigned((n + wpb - 1) / wpb)), dim3(64 * wpb), lds, st>>>(
+                                <<<dim3(unsigned(split > 1 ? n : (n + wpb - 1) / wpb)),
+                                   dim3(64 * wpb), lds, st>>>(
                                     items, n, srange, D.far_src, D.geo, D.ctab, F, D.tgt_pts,
-                                    D.fine_ang, G.ang_base, G.ang_n, stage, stride, phase, res, kp);
+                                    D.fine_ang, G.ang_base, G.ang_n, stage, stride, phase,
+                                    split > 1, D.ntgt, far_res, kp);
                         });
             return;
         }
     auto slow = [&](auto o0, auto o1)
     {
         constexpr int O0 = decltype(o0)::value, O1 = decltype(o1)::value;
-        k_far_rows<R, O0, O1, false><<<dim3(unsigned(n)), dim3(64), 0, st>>>(
+        k_far_rows<R, O0, O1, false><<<dim3(unsigned(n)), dim3(64 * split), 0, st>>>(
             items, n, srange, D.far_src, D.geo, D.ctab, F, D.tgt_pts, D.fine_ang, 0, 0, 0, 0,
-            phase, res, kp);
+            phase, split > 1, D.ntgt, far_res, kp);
     };
     if constexpr (sizeof(R) == 4) // angle tables too large for LDS: rare
         slow(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());

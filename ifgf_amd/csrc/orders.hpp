@@ -15,10 +15,10 @@ namespace dev
 template <typename R>
 void launch_up_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int level, const Cx<R>* F,
                     Cx<R>* V);
-// the far field of launch group `group`: added to the targets' results
+// far launch `group` (of far_steps): added to the far results of its targets' levels
 template <typename R>
 void launch_far_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
-                     Cx<R>* res);
+                     Cx<R>* far_res);
 // the values V -> the fine coefficients F of cones [c0, c1)
 template <typename R>
 void launch_transform_rows(DevicePlan& D, hipStream_t st, const KParams& kp, int64_t c0, int64_t c1,

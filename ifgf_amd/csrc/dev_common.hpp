@@ -834,20 +834,6 @@ __device__ __forceinline__ int pow2_at_least(int n)
     return p;
 }
 
-// upward-geometry table entries (host-built per parent level, see UpLevel in plan.hpp)
-struct UpEntF
-{
-    int32_t cf, sub;
-    float xi0, xi1, xi2, tr, ti;
-    int32_t d; // index of (cf, sub) among the distinct child cones of its (cell, octant)
-};
-struct UpEntD
-{
-    int32_t cf, sub;
-    double xi0, xi1, xi2, tr, ti;
-};
-template <typename R> using UpEnt = typename std::conditional<sizeof(R) == 4, UpEntF, UpEntD>::type;
-
 // The upward table of one (cell, octant) regrouped for evaluation (FP32): the parent nodes
 // whose positions fall in one child fine cone, in runs of at most UP_GRP nodes, so that one
 // thread evaluates the interpolant of that cone at all of them from one read of its

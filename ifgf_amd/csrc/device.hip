@@ -1593,7 +1593,7 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
             launch_leaf<KIND, R>(D, st, D.leaf_boxes + a, nb, ws, tabs, Vl(l), Fl(l), kp, fused);
             pt.end();
         }
-        if (u1 > u0 || D.up_item_off[l + 1] > D.up_item_off[l])
+        if (u1 > u0 || D.up_gl_off[l + 1] > D.up_gl_off[l])
         {
             pt.begin(2);
             launch_up_far<PH, R, DEC>(D, st, kp, tabs, l, -1, u0, u1, Fl(l + 1), Vl(l), res,
@@ -1747,13 +1747,23 @@ int64_t device_transform_cones(const DevicePlan& D)
     return up_fused_transform(D) ? D.tr_list_off.back() : D.n_cones;
 }
 
+static void drop_batch_graphs(DevicePlan& D)
+{
+    for (auto& g : D.b_graphs)
+    {
+        if (g.second.second)
+            (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(g.second.second));
+        if (g.second.first)
+            (void)hipGraphDestroy(static_cast<hipGraph_t>(g.second.first));
+    }
+    D.b_graphs.clear();
+}
+
 void device_free(DevicePlan& D)
 {
     void* ptrs[] = {D.src_pts, D.tgt_pts, D.normals, D.src_perm, D.tgt_perm, D.src_begin,
                     D.src_end, D.child, D.geo, D.cones, D.ctab, D.ho_nodes, D.trig_th,
-                    D.trig_ph, D.fine_ang, D.wmat, D.up_part_ent, D.up_entries, D.up_grp,
-                    D.up_items_k[0], D.up_items_k[1], D.up_items_k[2], D.up_items_k[3],
-                    D.up_glist, D.up_tl_desc, D.tr_list,
+                    D.trig_ph, D.fine_ang, D.wmat, D.up_grp, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
                     D.near_off, D.near_src, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
@@ -1765,10 +1775,7 @@ void device_free(DevicePlan& D)
         (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(D.graph_exec));
     if (D.graph)
         (void)hipGraphDestroy(static_cast<hipGraph_t>(D.graph));
-    if (D.b_graph_exec)
-        (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(D.b_graph_exec));
-    if (D.b_graph)
-        (void)hipGraphDestroy(static_cast<hipGraph_t>(D.b_graph));
+    drop_batch_graphs(D);
     if (D.cap_stream)
         (void)hipStreamDestroy(static_cast<hipStream_t>(D.cap_stream));
     if (D.side_stream)
@@ -1998,21 +2005,6 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         std::vector<int64_t> h_part_cell;
         std::vector<int32_t> h_goff, h_doff, h_dkey;
         {
-            std::vector<UpEntF> ef;
-            std::vector<UpEntD> ed;
-            std::vector<int64_t> part_ent;
-            for (const UpLevel* U : parts)
-            {
-                part_ent.push_back(int64_t(precision == PREC_FP64 ? ed.size() : ef.size()));
-                if (precision == PREC_FP64)
-                    for (const UpEntry& E : U->entries)
-                        ed.push_back({E.cf, E.sub, E.xi[0], E.xi[1], E.xi[2], E.tf[0], E.tf[1]});
-                else
-                    for (const UpEntry& E : U->entries)
-                        ef.push_back({E.cf, E.sub, float(E.xi[0]), float(E.xi[1]),
-                                      float(E.xi[2]), float(E.tf[0]), float(E.tf[1]), -1});
-            }
-            D.up_part_ent = dupload(part_ent, tot);
             auto groups = [&](auto G)
             {
                 D.up_grp = dupload(G.grp, tot);
@@ -2021,28 +2013,16 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                 h_dkey = std::move(G.dkey);
             };
             if (precision == PREC_FP64)
-            {
-                D.up_entries = dupload(ed, tot);
                 groups(group_tables<UpGrpD>(parts, D.n_hi, h_part_cell));
-            }
             else
-            {
-                D.up_entries = dupload(ef, tot);
                 groups(group_tables<UpGrp>(parts, D.n_hi, h_part_cell));
-            }
         }
-        // work lists.  Per level: leaf cones (leaf sampling), parent cones of boxes with a table
-        // grouped by (part, cell) into items of at most UP_K_CHOICES[i] cones of one cell (boxes in order
-        // within a cell), and the other parent cones (per-box upward pass)
-        std::vector<int32_t> leaf, up, glist, tl_glist, tl_gcell, tr_list;
+        // work lists.  Per level: leaf cones (leaf sampling), parent cones of boxes with a table (in
+        // tiles of boxes x cells), and the other parent cones (per-box upward pass)
+        std::vector<int32_t> leaf, up, glist, gcell, tr_list;
         D.tr_list_off.assign(D.levels + 1, 0);
-        std::vector<WorkItem> uitems[4];
         D.up_off.assign(D.levels + 1, 0);
         D.up_gl_off.assign(D.levels + 1, 0);
-        for (int kc = 0; kc < 4; kc++)
-        {
-            D.up_item_off_k[kc].assign(D.levels + 1, 0);
-        }
         D.cone_lvl_off.assign(D.levels + 1, 0);
         for (int l = 0; l < D.levels; l++)
         {
@@ -2051,10 +2031,6 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
             D.cone_lvl_off[l + 1] = P.cone_off[b1];
             D.up_off[l] = int64_t(up.size());
             D.up_gl_off[l] = int64_t(glist.size());
-            for (int kc = 0; kc < 4; kc++)
-            {
-                D.up_item_off_k[kc][l] = int64_t(uitems[kc].size());
-            }
             const int64_t g0 = int64_t(glist.size());
             D.tr_list_off[l] = int64_t(tr_list.size());
             for (int64_t g = b0; g < b1; g++)
@@ -2064,82 +2040,51 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                     if (!P.S.leaf[g] && box_part[g] < 0)
                         tr_list.push_back(int32_t(c));
                 }
-            auto part = [&](int32_t c) { return box_part[P.cone_box[c]]; };
-            auto cu = [&](int32_t c) { return parts[part(c)]->cellmap[P.cone_cell[c]]; };
-            // within a cell, cones of boxes with the same children next to one another: the
-            // cones of an item then have their children in the same octants
-            auto cmask = [&](int32_t c)
+            // tiles of boxes x cells (measured at 1M points, (6,8,7)/(3,5,4): 7.81 -> 7.4 ms for
+            // the upward phase against one cell after another, the same results); the cells of
+            // a tile in order, within a cell the cones of boxes with the same children together
+            struct Key
             {
-                int m = 0;
-                for (int o = 0; o < 8; o++)
-                    m |= (P.S.child[8 * int64_t(P.cone_box[c]) + o] >= 0 ? 1 : 0) << o;
-                return m;
+                uint64_t hi, lo; // (part, box tile), (cell tile, cell, children)
+                int32_t c, cell;
             };
-            std::stable_sort(glist.begin() + g0, glist.end(), [&](int32_t a, int32_t b)
-                             {
-                                 if (part(a) != part(b))
-                                     return part(a) < part(b);
-                                 if (cu(a) != cu(b))
-                                     return cu(a) < cu(b);
-                                 return cmask(a) < cmask(b);
-                             });
-            for (int kc = 0; kc < 4; kc++)
-                for (int64_t i = g0; i < int64_t(glist.size());)
-                {
-                    const int32_t pa = part(glist[i]), u = cu(glist[i]);
-                    if (u < 0)
-                        throw std::runtime_error("upward table has no entry for an active cell");
-                    int64_t j = i;
-                    while (j < int64_t(glist.size()) && j - i < UP_K_CHOICES[kc] &&
-                           part(glist[j]) == pa && cu(glist[j]) == u)
-                        j++;
-                    uitems[kc].push_back({u, int32_t(i - g0), int32_t(j - i), pa});
-                    i = j;
-                }
-            // the grouped kernel's list: tiles of boxes x cells (measured at 1M points,
-            // (6,8,7)/(3,5,4): 7.81 -> 7.4 ms for the upward phase, the same results)
-            const size_t h0 = tl_glist.size();
-            tl_glist.insert(tl_glist.end(), glist.begin() + g0, glist.end());
-            auto tb = [&](int32_t c) { return int64_t(P.cone_box[c] - b0) / UP_TILE_BOXES; };
-            auto tc = [&](int32_t c) { return cu(c) / UP_TILE_CELLS; };
-            std::stable_sort(tl_glist.begin() + h0, tl_glist.end(), [&](int32_t a, int32_t b)
-                             {
-                                 if (part(a) != part(b))
-                                     return part(a) < part(b);
-                                 if (tb(a) != tb(b))
-                                     return tb(a) < tb(b);
-                                 if (tc(a) != tc(b))
-                                     return tc(a) < tc(b);
-                                 if (cu(a) != cu(b))
-                                     return cu(a) < cu(b);
-                                 return cmask(a) < cmask(b);
-                             });
-            for (size_t i = h0; i < tl_glist.size(); i++)
-                tl_gcell.push_back(cu(tl_glist[i]));
+            std::vector<Key> keys(glist.size() - size_t(g0));
+            for (size_t i = 0; i < keys.size(); i++)
+            {
+                const int32_t c = glist[size_t(g0) + i];
+                const int64_t box = P.cone_box[c];
+                const int32_t pa = box_part[box], u = parts[pa]->cellmap[P.cone_cell[c]];
+                if (u < 0)
+                    throw std::runtime_error("upward table has no entry for an active cell");
+                uint64_t m = 0;
+                for (int o = 0; o < 8; o++)
+                    m |= uint64_t(P.S.child[8 * box + o] >= 0) << o;
+                keys[i] = {uint64_t(pa) << 32 | uint64_t((box - b0) / UP_TILE_BOXES),
+                           uint64_t(u / UP_TILE_CELLS) << 40 | uint64_t(u) << 8 | m, c, u};
+            }
+            std::stable_sort(keys.begin(), keys.end(), [](const Key& x, const Key& y)
+                             { return x.hi != y.hi ? x.hi < y.hi : x.lo < y.lo; });
+            for (size_t i = 0; i < keys.size(); i++)
+            {
+                glist[size_t(g0) + i] = keys[i].c;
+                gcell.push_back(keys[i].cell);
+            }
         }
         D.up_off[D.levels] = int64_t(up.size());
         D.up_gl_off[D.levels] = int64_t(glist.size());
-        for (int kc = 0; kc < 4; kc++)
-        {
-            D.up_item_off_k[kc][D.levels] = int64_t(uitems[kc].size());
-            D.up_items_k[kc] = dupload(uitems[kc], tot);
-        }
-        D.up_items = D.up_items_k[0]; // the default shape: 2 cones per item
-        D.up_item_off = D.up_item_off_k[0];
-        D.up_glist = dupload(glist, tot);
-        if (!tl_glist.empty())
+        if (!glist.empty())
         {
             // the upward kernels' per-cone records, from the plan's fixed tables: the children and their
             // cell-table offsets, the task ranges of each child's groups (the rows of h_goff), the
             // fine slots of the listed child cones (h_dkey through the children's cell tables)
-            std::vector<UpDesc> desc(tl_glist.size());
+            std::vector<UpDesc> desc(glist.size());
             auto fill = [&](size_t i0, size_t i1)
             {
                 for (size_t i = i0; i < i1; i++)
                 {
-                    const int32_t g = tl_glist[i];
+                    const int32_t g = glist[i];
                     const int64_t box = P.cone_box[g];
-                    const int64_t row = (h_part_cell[box_part[box]] + tl_gcell[i]) * 8;
+                    const int64_t row = (h_part_cell[box_part[box]] + gcell[i]) * 8;
                     UpDesc& u = desc[i];
                     u.g = g;
                     u.mask = cones[g].mask;
@@ -2368,17 +2313,25 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
     return "";
 }
 
-// batch buffers for rb columns (all-or-nothing; false when the device memory is short)
-static bool ensure_batch(DevicePlan& D, int rb, bool host_io)
+// bytes of the batch buffers for rb columns
+static size_t batch_bytes(const DevicePlan& D, int rb, bool host_io, size_t n[4])
 {
-    if (D.b_rb == rb && (!host_io || D.b_in))
-        return true;
-    // a captured batched graph holds the old buffers
-    if (D.b_graph_exec)
-        (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(D.b_graph_exec));
-    if (D.b_graph)
-        (void)hipGraphDestroy(static_cast<hipGraph_t>(D.b_graph));
-    D.b_graph_exec = D.b_graph = nullptr;
+    const size_t cs = D.prec == PREC_FP64 ? 16 : 8;
+    n[0] = cs * size_t(D.nsrc) * rb;
+    n[1] = cs * size_t(D.ntgt) * rb * size_t(1 + D.n_far_lvls);
+    n[2] = cs * size_t(std::max<int64_t>(1, D.n_cones)) * D.n_hi * rb;
+    n[3] = cs * (size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo + ROW_PAD) * rb;
+    return n[0] + n[1] + n[2] + n[3] + (host_io ? 16 * size_t(rb) * size_t(D.nsrc + D.ntgt) : 0);
+}
+
+// Batch buffers for up to want columns; the number of columns they hold (as many as leave half of
+// the free memory and 1 GiB of it; below 2: none).  Buffers that hold enough are kept.
+static int ensure_batch(DevicePlan& D, int want, bool host_io)
+{
+    if (D.b_rb >= want && (!host_io || D.b_in))
+        return want;
+    want = std::max(want, D.b_rb);
+    drop_batch_graphs(D); // captured graphs hold the old buffers
     for (void* p : {D.b_ws, D.b_res, D.b_V, D.b_F, static_cast<void*>(D.b_in),
                     static_cast<void*>(D.b_out)})
         if (p)
@@ -2387,20 +2340,19 @@ static bool ensure_batch(DevicePlan& D, int rb, bool host_io)
     D.b_in = D.b_out = nullptr;
     D.b_rb = 0;
     D.b_bytes = 0;
-    const size_t cs = D.prec == PREC_FP64 ? 16 : 8;
-    const size_t n_ws = size_t(D.nsrc) * rb, n_res = size_t(D.ntgt) * rb;
-    const size_t n_V = size_t(std::max<int64_t>(1, D.n_cones)) * D.n_hi * rb;
-    const size_t n_F = size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo * rb;
-    size_t need = cs * (n_ws + n_res + n_V + n_F);
-    if (host_io)
-        need += 16 * size_t(rb) * size_t(D.nsrc + D.ntgt);
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || need + (size_t(1) << 30) > free_b)
-        return false;
-    HIP_OK(hipMalloc(&D.b_ws, cs * n_ws));
-    HIP_OK(hipMalloc(&D.b_res, cs * n_res));
-    HIP_OK(hipMalloc(&D.b_V, cs * n_V));
-    HIP_OK(hipMalloc(&D.b_F, cs * n_F));
+    size_t free_b = 0, total_b = 0, n[4];
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
+        return 0;
+    int rb = want;
+    while (rb >= 2 && 2 * batch_bytes(D, rb, host_io, n) + (size_t(2) << 30) > free_b)
+        rb = rb > 8 ? (rb + 1) / 2 : rb - 1;
+    if (rb < 2)
+        return 0;
+    const size_t need = batch_bytes(D, rb, host_io, n);
+    HIP_OK(hipMalloc(&D.b_ws, n[0]));
+    HIP_OK(hipMalloc(&D.b_res, n[1]));
+    HIP_OK(hipMalloc(&D.b_V, n[2]));
+    HIP_OK(hipMalloc(&D.b_F, n[3]));
     if (host_io)
     {
         HIP_OK(hipMalloc(&D.b_in, 16 * size_t(rb) * size_t(D.nsrc)));
@@ -2408,7 +2360,7 @@ static bool ensure_batch(DevicePlan& D, int rb, bool host_io)
     }
     D.b_rb = rb;
     D.b_bytes = int64_t(need);
-    return true;
+    return rb;
 }
 
 std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, bool device_ptrs,
@@ -2445,15 +2397,24 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                 e = ev;
             }
         }
-        // several columns: the batched pipeline (8 or 32 columns per pass) when the orders
-        // have compiled kernels and the batch buffers fit
-        if (nrhs >= 2 && batched_supported(D) && !D.ring && std::getenv("IFGF_NO_BATCH") == nullptr)
+        // several columns: the batched pipeline, in as few equal passes as the shape's most
+        // columns per pass and the device memory allow.  Two columns are faster one by one (mixed
+        // form, 262,144 points order 6: 5.4 against 8.0 ms; FP64, 50,000 points: 6.5 against 6.6),
+        // three about even (8.1 against 8.6 ms; 20,000 points: 1.16 against 1.00)
+        if (nrhs >= 3 && !D.ring && std::getenv("IFGF_NO_BATCH") == nullptr)
         {
-            int rb = D.shape.rb > 0 ? D.shape.rb : (nrhs <= 8 ? 8 : 32);
-            bool ok = ensure_batch(D, rb, !device_ptrs);
-            if (!ok && rb == 32)
-                ok = ensure_batch(D, rb = 8, !device_ptrs);
-            if (ok)
+            auto equal = [&](int most)
+            {
+                const int64_t passes = (nrhs + most - 1) / most;
+                return int((nrhs + passes - 1) / passes);
+            };
+            int rb = equal(D.shape.rb > 0 ? D.shape.rb : MAX_COLUMNS);
+            // (the MFMA transform pads a pass to whole tiles of 8 columns)
+            const bool tiles = std::getenv("IFGF_TRANSFORM_MFMA") != nullptr;
+            const int have = ensure_batch(D, tiles ? (rb + 7) / 8 * 8 : rb, !device_ptrs);
+            if (have < rb)
+                rb = have >= 2 ? equal(have) : 0;
+            if (rb >= 2)
             {
                 for (int64_t c = 0; c < nrhs; c += rb)
                 {
@@ -2462,12 +2423,12 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                     double* oc = static_cast<double*>(out) + 2 * c * D.ntgt;
                     if (device_ptrs)
                     {
-                        mult_batched(D, wc, oc, rb, ncol, st, io, graph && !timed);
+                        mult_batched(D, wc, oc, ncol, st, io, graph && !timed);
                         continue;
                     }
                     HIP_OK(hipMemcpyAsync(D.b_in, wc, 16 * size_t(ncol) * size_t(D.nsrc),
                                           hipMemcpyHostToDevice, st));
-                    mult_batched(D, D.b_in, D.b_out, rb, ncol, st, io, graph && !timed);
+                    mult_batched(D, D.b_in, D.b_out, ncol, st, io, graph && !timed);
                     HIP_OK(hipMemcpyAsync(oc, D.b_out, 16 * size_t(ncol) * size_t(D.ntgt),
                                           hipMemcpyDeviceToHost, st));
                 }
@@ -2557,11 +2518,7 @@ std::string device_set_shape(DevicePlan& D, const LaunchShape& sh)
 {
     if (sh.xcd_log2 < 0 || sh.xcd_log2 > 8)
         return "launch shape: XCD run length must be 2^0 .. 2^8";
-    int kc = -1;
-    for (int i = 0; i < 4; i++)
-        if (UP_K_CHOICES[i] == sh.up_k)
-            kc = i;
-    if (kc < 0)
+    if (sh.up_k != 2 && sh.up_k != 4 && sh.up_k != 8 && sh.up_k != 16)
         return "launch shape: upward cones per item must be 2, 4, 8 or 16";
     if (sh.rb != 0 && sh.rb != 8 && sh.rb != 32)
         return "launch shape: batched columns per pass must be 8 or 32";
@@ -2580,8 +2537,6 @@ std::string device_set_shape(DevicePlan& D, const LaunchShape& sh)
                          sh.up_k != D.shape.up_k || sh.far_waves != D.shape.far_waves ||
                          sh.overlap != D.shape.overlap;
     D.shape = sh;
-    D.up_items = D.up_items_k[kc];
-    D.up_item_off = D.up_item_off_k[kc];
     if (changed)
         device_drop_graph(D); // the captured kernels have the old shapes
     return "";
@@ -2597,12 +2552,7 @@ void device_drop_graph(DevicePlan& D)
     if (D.graph)
         (void)hipGraphDestroy(static_cast<hipGraph_t>(D.graph));
     D.graph = nullptr;
-    if (D.b_graph_exec)
-        (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(D.b_graph_exec));
-    D.b_graph_exec = nullptr;
-    if (D.b_graph)
-        (void)hipGraphDestroy(static_cast<hipGraph_t>(D.b_graph));
-    D.b_graph = nullptr;
+    drop_batch_graphs(D);
 }
 
 std::string device_autotune(DevicePlan& D, int64_t nrhs, int reps, LaunchShape& best)
@@ -2632,7 +2582,7 @@ std::string device_autotune(DevicePlan& D, int64_t nrhs, int reps, LaunchShape& 
         HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
         HIP_OK(hipEventCreate(&e0));
         HIP_OK(hipEventCreate(&e1));
-        const bool batched = nrhs >= 2 && batched_supported(D);
+        const bool batched = nrhs >= 3 && !D.ring;
         // fastest of reps mults with the shape s (one untimed mult first): the phase's time
         // from the phase events, or the whole mult's (phase < 0)
         auto measure = [&](const LaunchShape& s, int phase) -> double

@@ -2,7 +2,9 @@
 #pragma once
 
 #include <cstdint>
+#include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "plan.hpp"
@@ -67,13 +69,12 @@ struct LaunchShape
     int xcd_log2 = 4; // work items dealt to the XCDs in runs of 2^xcd_log2 (0: plain order)
     int cpb = 0;      // transform: cones per workgroup (0: the order class's default)
     int up_k = 2;     // upward: parent cones per workgroup (2, 4, 8 or 16)
-    int rb = 0;       // batched: columns per pass (8 or 32; 0: 8 up to 8 columns, else 32)
+    int rb = 0;       // batched: most columns per pass (8 or 32; 0: 32)
     int far_waves = 2; // mixed far field: waves (items) per workgroup sharing the LDS tables
     int overlap = 1;   // far field on a second stream beside the upward chain, with the near
                        // field there too (1) or first on the main stream (2); 0: one stream
 };
-constexpr int UP_K_CHOICES[4] = {2, 4, 8, 16};
-// tiles of the grouped upward kernel's work list: parent boxes (in Morton order within a level)
+// tiles of the grouped upward kernels' work list: parent boxes (in Morton order within a level)
 // x cells (table index) per tile
 constexpr int UP_TILE_BOXES = 16;
 constexpr int UP_TILE_CELLS = 128;
@@ -84,7 +85,7 @@ constexpr int UP_TILE_CELLS = 128;
 // their tables -> the (cell, octant) rows -> the listed child cones' slots).
 // entries allocated past the fine coefficients: kernels that read a cone's coefficients a chunk
 // of rows at a time may read up to this far past the last cone's (and use none of it)
-constexpr int ROW_PAD = 32;
+constexpr int ROW_PAD = 40;
 constexpr int UP_DMAX = 32; // listed child cones per (parent cone, child) with a slot here
 struct alignas(16) UpDesc
 {
@@ -137,24 +138,13 @@ struct DevicePlan
     void* wmat = nullptr;         // axis maps (R): W0 | W1 | W2
     int woff[4] = {0, 0, 0, 0};
 
-    // upward geometry tables: entries {cf, sub, xi[3], tf[2]} in R of every part (a level of
-    // one geometry), up_part_ent[part] = the part's first entry
-    void* up_entries = nullptr;
-    int64_t* up_part_ent = nullptr;
-    // the same tables regrouped by child cone (UpGrp / UpGrpD records): one read of a child
-    // cone's coefficients serves the nodes that fall into it
+    // the upward geometry tables of every part (a level of one geometry) regrouped by child cone
+    // (UpGrp / UpGrpD records): one read of a child cone's coefficients serves the nodes that
+    // fall into it
     void* up_grp = nullptr;
-
-    // (cell, cones of that cell, part) items of at most UP_K_CHOICES[i] cones, one list per
-    // choice; up_items / up_item_off name the list of the current shape
-    WorkItem* up_items_k[4] = {nullptr, nullptr, nullptr, nullptr};
-    std::vector<int64_t> up_item_off_k[4];
-    WorkItem* up_items = nullptr;
-    std::vector<int64_t> up_item_off;        // per level, into up_items
-    int32_t* up_glist = nullptr;             // the items' cones, level-major
-    std::vector<int64_t> up_gl_off;          // per level, into up_glist
-    // the same cones for k_up_grp and k_up_rows (which take one cone at a time): per level (the
-    // ranges of up_gl_off) ordered by tiles of UP_TILE_BOXES boxes x UP_TILE_CELLS cells
+    // the parent cones with a table, per level (up_gl_off) in tiles of UP_TILE_BOXES boxes x
+    // UP_TILE_CELLS cells
+    std::vector<int64_t> up_gl_off;
     UpDesc* up_tl_desc = nullptr; // one record per cone of the list
 
     int32_t* leaf_cones = nullptr;
@@ -211,14 +201,12 @@ struct DevicePlan
     std::vector<void*> ev_far_done;       // ring on two streams: far groups of a source level done
     int64_t bytes_total = 0;
 
-    // work buffers of the batched mult (b_rb columns, column-minor), allocated on first use;
-    // b_in / b_out stage host densities and results
     // the single-column mult's core captured as a graph (on first use with graphs enabled),
-    // and the batched mult's core for the current batch buffers
-    void* graph = nullptr;      // hipGraph_t
-    void* graph_exec = nullptr; // hipGraphExec_t
-    void* b_graph = nullptr;
-    void* b_graph_exec = nullptr;
+    // and the batched mult's core for the current batch buffers, per number of columns (at most
+    // MAX_COLUMNS of them): hipGraph_t, hipGraphExec_t
+    void* graph = nullptr;
+    void* graph_exec = nullptr;
+    std::map<int, std::pair<void*, void*>> b_graphs;
     void* cap_stream = nullptr; // hipStream_t of the capture
     // the second stream of the overlapped near field and its fork / join events
     void* side_stream = nullptr;
@@ -235,6 +223,9 @@ struct DevicePlan
     // staging of host densities and results of single-column mults (first use)
     double *h_in = nullptr, *h_out = nullptr;
 
+    // work buffers of the batched mult (up to b_rb columns, column-minor; the results followed by
+    // the far results of each target level), allocated on first use; b_in / b_out stage host
+    // densities and results
     int b_rb = 0;
     void *b_ws = nullptr, *b_res = nullptr, *b_V = nullptr, *b_F = nullptr;
     double *b_in = nullptr, *b_out = nullptr;
@@ -248,11 +239,10 @@ void device_free(DevicePlan& D);
 // coarse cones of one mult's standalone values -> coefficients transform (all of them unless
 // leaf sampling and the grouped upward kernel transform their own)
 int64_t device_transform_cones(const DevicePlan& D);
-// batched mult (batched.hip): ncol <= rb columns (rb = 8 or 32) of device densities with the
-// batch buffers allocated for rb; the compiled order classes only (batched_supported)
-bool batched_supported(const DevicePlan& D);
-void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int rb, int ncol,
-                  void* stream, int io, bool graph = false);
+// batched mult (batched.hip): ncol <= b_rb columns of device densities
+constexpr int MAX_COLUMNS = 32;
+void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int ncol, void* stream,
+                  int io, bool graph = false);
 // w: complex128 (host or device), out: complex128 (host or device); nrhs columns of length
 // N / M stored one after another.  io: IO_* bits applied while the densities are gathered and
 // the results scattered (conjugations and a sign, for adjoint products).
@@ -278,7 +268,7 @@ void device_drop_graph(DevicePlan& D);
 // Time the candidate shapes on this operator with synthetic densities (nrhs columns, each
 // candidate `reps` times, the fastest kept), one choice after another: the XCD run length on
 // the whole mult, then the transform's cones per workgroup, the upward cones per item and the
-// far field's waves per workgroup on their phases, then (nrhs >= 2) the batched columns per
+// far field's waves per workgroup on their phases, then (nrhs >= 3) the batched columns per
 // pass.  Leaves the best shape applied.
 std::string device_autotune(DevicePlan& D, int64_t nrhs, int reps, LaunchShape& best);
 // per-phase timings of the last mult (ms): near, leaf, upward, transform, far, total

@@ -81,10 +81,8 @@ template <int KIND, typename R, int RB>
 __global__ __launch_bounds__(64) void k_near_b(const WorkItem* __restrict__ items,
                                                int64_t nitems,
                                                const int32_t* __restrict__ near_off,
-                                               const int32_t* __restrict__ near_src,
+                                               const PointRun* __restrict__ near_run,
                                                const BoxGeo* __restrict__ geo,
-                                               const int64_t* __restrict__ sbeg,
-                                               const int64_t* __restrict__ send,
                                                const double* __restrict__ spts,
                                                const double* __restrict__ snrm,
                                                const Cx<R>* __restrict__ w,
@@ -111,11 +109,10 @@ __global__ __launch_bounds__(64) void k_near_b(const WorkItem* __restrict__ item
     for (int r = 0; r < RB; r++)
         acc[r] = {0, 0};
     const int32_t j0 = near_off[wi.box], j1 = near_off[wi.box + 1];
+    const KParams kb = with_k(kp, geo[wi.pad]);
     for (int32_t j = j0; j < j1; j++)
     {
-        const int32_t s = near_src[j];
-        const KParams kb = with_k(kp, geo[s]);
-        const int64_t b = sbeg[s], e = send[s];
+        const int64_t b = near_run[j].begin, e = near_run[j].end;
         for (int64_t c0 = b; c0 < e; c0 += 64)
         {
             const int n = int(min<int64_t>(64, e - c0));
@@ -411,8 +408,8 @@ void run_batched_core(DevicePlan& D, hipStream_t st, int nc)
         {
             if (D.n_near_items)
                 k_near_b<KIND, R, RB><<<dim3(unsigned(D.n_near_items)), dim3(64), 0, s>>>(
-                    D.near_items, D.n_near_items, D.near_off, D.near_src, D.geo, D.src_begin,
-                    D.src_end, D.src_pts, D.normals, ws, D.tgt_pts, res, nc, kp);
+                    D.near_items, D.n_near_items, D.near_off, D.near_run, D.geo, D.src_pts,
+                    D.normals, ws, D.tgt_pts, res, nc, kp);
         },
         [&](int g, hipStream_t s) { launch_far_cols<R>(D, s, kp, g, F, far_res, nc); });
     if (overlap != 1)

@@ -76,31 +76,40 @@ template <typename R> __global__ void k_zero(Cx<R>* p, int64_t n, Cx<R>* q, int6
 
 
 // near field: for each target of the item, sum over the points of its near source leaves
-// (ifgfoperator.hpp:900-960; octree.hpp:302-307).  The wave walks the source leaves in order
-// and stages each (64 points at a time) in LDS with one coalesced load; lane = (target, group),
-// the groups splitting the staged points; xor-shuffle reduction over the groups at the end.
+// (ifgfoperator.hpp:900-960; octree.hpp:302-307), which the plan lists as runs of consecutive
+// points (neighbouring leaves follow one another in Morton order).  The workgroup's waves share the
+// item's sources, an equal part each; a wave stages 64 points at a time in its own LDS, the next
+// 64 read from memory meanwhile; lane = (target, group), the groups splitting the staged points;
+// xor-shuffle reduction over the groups, then the waves' sums added in order.
+// Many items: VALU-bound (1M points: 1.0 ms, 610-634 wave instructions per ns).  Few items: the
+// chain of waits of one item, which the runs (a third as many steps as leaves), the read-ahead and
+// up to 8 waves per item shorten: 10,000 points 0.20 -> 0.05 ms;
+// 30,001 field points near 40,000 sources 0.76 -> 0.13 ms; FP64, 99,991 points 0.98 -> 0.67 ms.
 template <int KIND, typename R>
-__global__ __launch_bounds__(64) void k_near(const WorkItem* __restrict__ items, int64_t nitems,
-                                             const int32_t* __restrict__ near_off,
-                                             const int32_t* __restrict__ near_src,
-                                             const BoxGeo* __restrict__ geo,
-                                             const int64_t* __restrict__ sbeg,
-                                             const int64_t* __restrict__ send,
-                                             const double* __restrict__ spts,
-                                             const double* __restrict__ snrm,
-                                             const Cx<R>* __restrict__ w,
-                                             const double* __restrict__ tpts,
-                                             Cx<R>* __restrict__ result, KParams kp)
+__global__ __launch_bounds__(512) void k_near(const WorkItem* __restrict__ items, int64_t nitems,
+                                              const int32_t* __restrict__ near_off,
+                                              const PointRun* __restrict__ near_run,
+                                              const int32_t* __restrict__ near_pts,
+                                              const BoxGeo* __restrict__ geo,
+                                              const double* __restrict__ spts,
+                                              const double* __restrict__ snrm,
+                                              const Cx<R>* __restrict__ w,
+                                              const double* __restrict__ tpts,
+                                              Cx<R>* __restrict__ result, KParams kp)
 {
     constexpr bool NRM = KIND == KD || KIND == KC;
-    __shared__ double sp[3 * 64];
-    __shared__ double sn[NRM ? 3 * 64 : 1];
-    __shared__ Cx<R> sw[64];
+    constexpr int WD = (NRM ? 6 : 3) * 64; // doubles of a wave's staged points and normals
+    extern __shared__ __align__(16) unsigned char near_smem[];
+    const int nw = int(blockDim.x >> 6);
+    const int lane = int(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double* sp = reinterpret_cast<double*>(near_smem) + wave * WD;
+    double* sn = sp + 3 * 64;
+    Cx<R>* sw = reinterpret_cast<Cx<R>*>(reinterpret_cast<double*>(near_smem) + nw * WD) + wave * 64;
     const int64_t it = xcd_block(kp.xlg);
     if (it >= nitems)
         return;
-    const WorkItem wi = items[it];
-    const int lane = threadIdx.x;
+    const WorkItem wi = items[it]; // pad: a source box of the targets' geometry
+    const KParams kb = with_k(kp, geo[wi.pad]);
     const int Tp = pow2_at_least(wi.count);
     const int ti = lane & (Tp - 1);
     const int grp = lane / Tp, ngrp = 64 / Tp;
@@ -108,45 +117,98 @@ __global__ __launch_bounds__(64) void k_near(const WorkItem* __restrict__ items,
     const int64_t t = int64_t(wi.first) + (valid ? ti : 0);
     const double y0 = tpts[3 * t], y1 = tpts[3 * t + 1], y2 = tpts[3 * t + 2];
     Cx<R> acc = {0, 0};
-    const int32_t j0 = near_off[wi.box], j1 = near_off[wi.box + 1];
-    for (int32_t j = j0; j < j1; j++)
+    const int32_t j1 = near_off[wi.box + 1];
+    // this wave's sources: [lo, hi) of the item's sources, counted along its runs
+    const int32_t tot = near_pts[wi.box];
+    int32_t lo = int32_t(int64_t(tot) * wave / nw);
+    const int32_t hi = int32_t(int64_t(tot) * (wave + 1) / nw);
+    int32_t j = near_off[wi.box], at = 0; // run j starts at source `at`
+    PointRun run = {0, 0};
+    if (j < j1)
+        run = near_run[j];
+    int32_t i0 = 0;
+    int n = 0; // the staged chunk: points [i0, i0 + n)
+    auto next = [&]() -> bool
     {
-        const int32_t s = near_src[j];
-        const KParams kb = with_k(kp, geo[s]);
-        const int64_t b = sbeg[s], e = send[s];
-        for (int64_t c0 = b; c0 < e; c0 += 64)
+        if (lo >= hi)
+            return false;
+        while (lo >= at + (run.end - run.begin)) // uniform
         {
-            const int n = int(min<int64_t>(64, e - c0));
-            __syncthreads();
-            if (lane < n)
-            {
-                const int64_t i = c0 + lane;
-                sp[3 * lane] = spts[3 * i];
-                sp[3 * lane + 1] = spts[3 * i + 1];
-                sp[3 * lane + 2] = spts[3 * i + 2];
-                if constexpr (NRM)
-                {
-                    sn[3 * lane] = snrm[3 * i];
-                    sn[3 * lane + 1] = snrm[3 * i + 1];
-                    sn[3 * lane + 2] = snrm[3 * i + 2];
-                }
-                sw[lane] = w[i];
-            }
-            __syncthreads();
-            for (int k = grp; k < n; k += ngrp)
-            {
-                const double d0 = sp[3 * k] - y0, d1 = sp[3 * k + 1] - y1, d2 = sp[3 * k + 2] - y2;
-                double xn = 0;
-                if constexpr (NRM)
-                    xn = d0 * sn[3 * k] + d1 * sn[3 * k + 1] + d2 * sn[3 * k + 2];
-                acc = cadd(acc, p2p<KIND, R>(kb, R(d0), R(d1), R(d2), xn, sw[k]));
-            }
+            at += run.end - run.begin;
+            run = near_run[++j];
         }
+        i0 = run.begin + (lo - at);
+        n = min(min(64, run.end - i0), hi - lo);
+        lo += n;
+        return true;
+    };
+    double p[NRM ? 6 : 3] = {};
+    Cx<R> pw = {0, 0};
+    auto load = [&]
+    {
+        if (lane < n)
+        {
+            const int64_t i = i0 + lane;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                p[d] = spts[3 * i + d];
+            if constexpr (NRM)
+            {
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    p[3 + d] = snrm[3 * i + d];
+            }
+            pw = w[i];
+        }
+    };
+    bool more = next();
+    if (more)
+        load();
+    while (more) // uniform
+    {
+        const int nn = n;
+        if (lane < nn)
+        {
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                sp[3 * lane + d] = p[d];
+            if constexpr (NRM)
+            {
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    sn[3 * lane + d] = p[3 + d];
+            }
+            sw[lane] = pw;
+        }
+        more = next();
+        if (more)
+            load();
+        // the wave's LDS writes have completed before it reads them (one wave: no barrier)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        for (int k = grp; k < nn; k += ngrp)
+        {
+            const double d0 = sp[3 * k] - y0, d1 = sp[3 * k + 1] - y1, d2 = sp[3 * k + 2] - y2;
+            double xn = 0;
+            if constexpr (NRM)
+                xn = d0 * sn[3 * k] + d1 * sn[3 * k + 1] + d2 * sn[3 * k + 2];
+            acc = cadd(acc, p2p<KIND, R>(kb, R(d0), R(d1), R(d2), xn, sw[k]));
+        }
+        // the next chunk's writes stay behind these reads
+        asm volatile("" ::: "memory");
     }
     for (int m = Tp; m < 64; m <<= 1)
     {
         acc.x += __shfl_xor(acc.x, m, 64);
         acc.y += __shfl_xor(acc.y, m, 64);
+    }
+    if (nw > 1) // uniform
+    {
+        sw[lane] = acc; // each wave's staged densities are done with
+        __syncthreads();
+        if (wave)
+            return;
+        for (int v = 1; v < nw; v++)
+            acc = cadd(acc, sw[64 * v + lane]);
     }
     if (grp == 0 && valid)
         result[t] = cadd(result[t], acc);
@@ -1560,9 +1622,15 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
         [&](hipStream_t s)
         {
             if (D.n_near_items)
-                k_near<KIND, R><<<dim3(unsigned(D.n_near_items)), dim3(64), 0, s>>>(
-                    D.near_items, D.n_near_items, D.near_off, D.near_src, D.geo, D.src_begin,
-                    D.src_end, D.src_pts, D.normals, ws, D.tgt_pts, res, kp);
+            {
+                // waves per item: as many as give the chip about 8192
+                const int nw = far_split(D.n_near_items);
+                constexpr size_t wd = (KIND == KD || KIND == KC ? 6 : 3) * 64 * sizeof(double);
+                k_near<KIND, R><<<dim3(unsigned(D.n_near_items)), dim3(64 * nw),
+                                  nw * (wd + 64 * sizeof(Cx<R>)), s>>>(
+                    D.near_items, D.n_near_items, D.near_off, D.near_run, D.near_pts, D.geo,
+                    D.src_pts, D.normals, ws, D.tgt_pts, res, kp);
+            }
         },
         [&](int g, hipStream_t s)
         {
@@ -1765,7 +1833,7 @@ void device_free(DevicePlan& D)
                     D.src_end, D.child, D.geo, D.cones, D.ctab, D.ho_nodes, D.trig_th,
                     D.trig_ph, D.fine_ang, D.wmat, D.up_grp, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
-                    D.near_off, D.near_src, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.V,
+                    D.near_off, D.near_run, D.near_pts, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
                     D.b_out, D.h_in, D.h_out};
     for (void* p : ptrs)
@@ -2137,12 +2205,25 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         D.leaf_cones = dupload(leaf, tot);
         D.n_leaf_cones = int64_t(leaf.size());
         {
-            // leaf boxes with active cones: (box, first cone, number of cones)
+            // leaf boxes with active cones: (box, first cone, number of cones).  Operators of few
+            // leaf cones: items of few cones each, so that they fill the chip (10,000 points,
+            // 660 nodes per cone: leaf sampling 0.23 ->
+            // 0.075 ms; 131,072 points on a torus, whose leaves differ most: 3.3 -> 1.2 ms)
+            const int64_t most = std::max<int64_t>(1, int64_t(leaf.size()) / 2048);
             std::vector<WorkItem> lb;
             for (int64_t g = 0; g < P.S.num_boxes(); g++)
                 if (P.S.leaf[g] && P.cone_off[g + 1] > P.cone_off[g])
-                    lb.push_back({int32_t(g), int32_t(P.cone_off[g]),
-                                  int32_t(P.cone_off[g + 1] - P.cone_off[g]), 0});
+                {
+                    const int64_t n = P.cone_off[g + 1] - P.cone_off[g];
+                    const int64_t parts = std::max<int64_t>(1, (n + most / 2) / most);
+                    for (int64_t k = 0; k < parts; k++)
+                    {
+                        const int64_t c0 = n * k / parts, c1 = n * (k + 1) / parts;
+                        if (c1 > c0)
+                            lb.push_back({int32_t(g), int32_t(P.cone_off[g] + c0),
+                                          int32_t(c1 - c0), 0});
+                    }
+                }
             D.leaf_boxes = dupload(lb, tot);
             D.n_leaf_boxes = int64_t(lb.size());
             // per level (boxes are level-major): the range of the leaf boxes, of the fine slots
@@ -2183,8 +2264,30 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         csr(P.far, foff, fsrc, ftb);
         csr(P.near, noff, nsrcv, ntb);
         D.far_src = dupload(fsrc, tot);
-        D.near_off = dupload(noff, tot);
-        D.near_src = dupload(nsrcv, tot);
+        {
+            // the near source leaves of each target box as runs of consecutive points
+            std::vector<PointRun> runs;
+            std::vector<int32_t> roff(nt + 1, 0), pts(nt, 0);
+            for (int64_t t = 0; t < nt; t++)
+            {
+                const size_t r0 = runs.size();
+                for (int32_t m = noff[t]; m < noff[t + 1]; m++)
+                {
+                    const int32_t b = int32_t(P.S.begin[nsrcv[m]]), e = int32_t(P.S.end[nsrcv[m]]);
+                    if (b == e)
+                        continue;
+                    pts[t] += e - b;
+                    if (runs.size() > r0 && runs.back().end == b)
+                        runs.back().end = e;
+                    else
+                        runs.push_back({b, e});
+                }
+                roff[t + 1] = int32_t(runs.size());
+            }
+            D.near_off = dupload(roff, tot);
+            D.near_run = dupload(runs, tot);
+            D.near_pts = dupload(pts, tot);
+        }
         // far work: items of at most 64 targets of one target box against its far sources of
         // one source level (contiguous in its list: box ids are level-major), grouped by (source
         // level, target level), deepest source level first, then deepest target level
@@ -2265,6 +2368,8 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
         D.far_srange = dupload(frange, tot);
         D.far_items = dupload(fitems, tot);
         auto nitems = make_items(ntb, P.T);
+        for (WorkItem& w : nitems)
+            w.pad = nsrcv[noff[w.box]];
         D.near_items = dupload(nitems, tot);
         D.n_near_items = int64_t(nitems.size());
         // work buffers

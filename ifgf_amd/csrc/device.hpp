@@ -61,6 +61,11 @@ struct WorkItem // a chunk of at most 64 consecutive target points of one target
     int32_t pad;
 };
 
+struct PointRun // consecutive source points [begin, end) in Morton order
+{
+    int32_t begin, end;
+};
+
 // Launch shapes of the mult's kernels: choices that change speed but not results, picked by
 // device_autotune (measured on the operator itself) or set by the caller.  The defaults at 1M
 // points, (6,9,7)/(3,6,4): 24.7 ms per mult; with 16 upward cones 25.4, with 1 far wave 25.8.
@@ -161,8 +166,11 @@ struct DevicePlan
 
     int32_t* far_src = nullptr;   // far source boxes, by target box then source box
     int32_t* far_srange = nullptr; // per far item: its sources far_src[2i] .. far_src[2i + 1]
+    // near sources by target box: runs of consecutive points near_run[near_off[t]] ..
+    // near_run[near_off[t + 1]], near_pts[t] points in all
     int32_t* near_off = nullptr;
-    int32_t* near_src = nullptr;
+    PointRun* near_run = nullptr;
+    int32_t* near_pts = nullptr;
     WorkItem* far_items = nullptr;
     // far work in launch groups of one source level and one target level, deepest source level
     // first: a group can run as soon as its source level's coefficients exist; groups run one

@@ -10,6 +10,7 @@
 #include <stdexcept>
 
 #include "columns.hpp"
+#include "orders.hpp"
 #include "rows.hpp"
 
 namespace ifgf
@@ -260,7 +261,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const Cx<R>* __restrict__ F,
     const double* __restrict__ tpts, const double* __restrict__ ang, int ang_base, int ang_n,
-    int phase, int nc, int tpt, int64_t ntgt, Cx<R>* __restrict__ far_res, KParams kp)
+    const int64_t* __restrict__ rec_off, const FarRec<R>* __restrict__ rec,
+    const Cx<R>* __restrict__ cfs, int phase, int nc, int tpt, int64_t ntgt,
+    Cx<R>* __restrict__ far_res, KParams kp)
 {
     constexpr int TM = 8; // targets per thread at most
     extern __shared__ __align__(16) unsigned char far_smem[];
@@ -298,7 +301,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
             int slot = -1;
             double rr = 1, ri = 1;
             R x[3] = {R(0), R(0), R(0)};
-            if (tvalid)
+            const int64_t e = rec ? rec_off[it] + int64_t(jb - j0 + wave) * wi.count + lane : 0;
+            if (tvalid && rec) // the pairs' records
+            {
+                const FarRec<R> q = rec[e];
+                ok = q.slot >= 0;
+                slot = q.slot;
+                x[0] = q.x0;
+                x[1] = q.x1;
+                x[2] = q.x2;
+            }
+            else if (tvalid)
             {
                 if constexpr (FAST)
                 {
@@ -344,7 +357,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
                         q = v;
                     }
                 }
-                if (!phase)
+                if (rec)
+                    s_cf[wave][lane] = cfs[e];
+                else if (!phase)
                     s_cf[wave][lane] = {R(INV_4PI_D * ri), R(0)};
                 else
                     s_cf[wave][lane] = cscale(expmk_far<R>(B.k_re, B.k_im, rr), R(INV_4PI_D * ri));
@@ -482,8 +497,8 @@ typedef float mf4 __attribute__((ext_vector_type(4)));
 // item's targets are sums over a fine cone's n_lo coefficients, the same cone for many of them, so
 // a block of 16 targets x 16 real columns is a product basis (16 x n_lo) times coefficients (n_lo x
 // 16) on v_mfma_f32_16x16x4f32.  Four waves; per step of nbox source boxes a wave locates the
-// item's targets in one box and writes the products of their Chebyshev values to LDS (ks floats
-// per target).  Then each wave takes one tile of 16 columns and its share of the four blocks of
+// item's targets in one box (or reads their records) and writes the products of their Chebyshev
+// values to LDS (ks floats per target).  Then each wave takes one tile of 16 columns and its share of the four blocks of
 // targets, and goes through the distinct cones of each box (2 to 3 for 64 targets), 32 coefficients
 // at a time: the next chunk's (or cone's, or box's) coefficients are loaded while the current
 // ones are multiplied into every block that has targets in the cone, rows of other targets zeroed.
@@ -499,7 +514,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const float* __restrict__ F,
     const double* __restrict__ tpts, const double* __restrict__ ang, int ang_base, int ang_n,
-    int phase, int nc, int nbox, int ks, int64_t ntgt, float* __restrict__ far_res, KParams kp)
+    const int64_t* __restrict__ rec_off, const FarRec<float>* __restrict__ rec,
+    const Cx<float>* __restrict__ cfs, int phase, int nc, int nbox, int ks, int64_t ntgt,
+    float* __restrict__ far_res, KParams kp)
 {
     extern __shared__ __align__(16) unsigned char far_smem[];
     double* sang = reinterpret_cast<double*>(far_smem);
@@ -548,11 +565,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             const BoxGeo& B = geo[__builtin_amdgcn_readfirstlane(far_src[jb + wave])];
             bool ok = false;
             LocF L;
-            if (tvalid)
+            Cx<float> cf = {0.f, 0.f};
+            if (tvalid && rec) // the pairs' records
+            {
+                const int64_t e = rec_off[it] + int64_t(jb - j0 + wave) * wi.count + lane;
+                const FarRec<float> q = rec[e];
+                cf = cfs[e];
+                ok = q.slot >= 0;
+                L.fine = q.slot;
+                L.xi[0] = q.x0;
+                L.xi[1] = q.x1;
+                L.xi[2] = q.x2;
+            }
+            else if (tvalid)
                 ok = locate_fast(B, sang + (2 * B.fth_off - ang_base),
                                  sang + (2 * B.fph_off - ang_base), ctab, y0 - B.ctr[0],
                                  y1 - B.ctr[1], y2 - B.ctr[2], kp.f0, kp.f1, kp.f2, L);
-            Cx<float> cf = {0.f, 0.f};
             {
                 const int slot = ok ? L.fine : -1;
                 const uint64_t act = __ballot(ok);
@@ -600,9 +628,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     b2 = a2;
                     a2 = v;
                 }
-                if (!phase)
+                if (!rec && !phase)
                     cf = {float(INV_4PI_D * L.rinv), 0.f};
-                else
+                else if (!rec)
                     cf = cscale(expmk_far<float>(B.k_re, B.k_im, L.r), float(INV_4PI_D * L.rinv));
             }
             s_cf[wave][lane] = cf;
@@ -827,6 +855,8 @@ void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
         kernel<<<dim3(unsigned(n)), dim3(256), lds, st>>>(
             items, srange, D.far_src, D.geo, D.ctab, F, D.tgt_pts, D.fine_ang, G.ang_base, an,
+            D.far_rec ? D.far_rec_off + G.item0 : nullptr,
+            static_cast<const FarRec<R>*>(D.far_rec), static_cast<const Cx<R>*>(D.far_cf),
             D.kind != KL, nc, tpt, D.ntgt, far_res, kp);
     };
     if constexpr (sizeof(R) == 4)
@@ -844,7 +874,10 @@ void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(mlds)));
             k_far_mfma<<<dim3(unsigned(n)), dim3(256), mlds, st>>>(
                 items, srange, D.far_src, D.geo, D.ctab, reinterpret_cast<const float*>(F),
-                D.tgt_pts, D.fine_ang, G.ang_base, an, D.kind != KL, nc, nbox, ks, D.ntgt,
+                D.tgt_pts, D.fine_ang, G.ang_base, an,
+                D.far_rec ? D.far_rec_off + G.item0 : nullptr,
+                static_cast<const FarRec<float>*>(D.far_rec),
+                static_cast<const Cx<float>*>(D.far_cf), D.kind != KL, nc, nbox, ks, D.ntgt,
                 reinterpret_cast<float*>(far_res), kp);
         }
         else if (fast) // coefficients by the hundred

@@ -469,60 +469,11 @@ template <int N> __device__ __forceinline__ void cheb_t(float x, float (&t)[N])
         t[k] = fmaf(2.0f * x, t[k - 1], -(k == 2 ? 1.0f : t[k - 2]));
 }
 
-// The interpolants of one fine cone (coefficients c, index i0 + O0 (i1 + O1 i2)) at G points
-// from their Chebyshev values: sum_{i0,i1,i2} c T_i0(x0) T_i1(x1) T_i2(x2), summed over i0,
-// then i1, then i2 (each coefficient read once for the G points)
-template <int O0, int O1, int O2, int G>
-__device__ __forceinline__ void eval_cone_g(const float2* __restrict__ c,
-                                            const float (&t0)[G][O0], const float (&t1)[G][O1],
-                                            const float (&t2)[G][O2], float2 (&out)[G])
-{
-#pragma unroll
-    for (int i2 = 0; i2 < O2; i2++)
-    {
-        float2 pl[G];
-#pragma unroll
-        for (int i1 = 0; i1 < O1; i1++)
-        {
-            float2 row[O0];
-#pragma unroll
-            for (int i0 = 0; i0 < O0; i0++)
-                row[i0] = c[i0 + O0 * (i1 + O1 * i2)];
-#pragma unroll
-            for (int g = 0; g < G; g++)
-            {
-                float2 sm = row[0];
-#pragma unroll
-                for (int i0 = 1; i0 < O0; i0++)
-                {
-                    sm.x = fmaf(row[i0].x, t0[g][i0], sm.x);
-                    sm.y = fmaf(row[i0].y, t0[g][i0], sm.y);
-                }
-                if (i1 == 0)
-                    pl[g] = sm;
-                else
-                {
-                    pl[g].x = fmaf(sm.x, t1[g][i1], pl[g].x);
-                    pl[g].y = fmaf(sm.y, t1[g][i1], pl[g].y);
-                }
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < G; g++)
-        {
-            if (i2 == 0)
-                out[g] = pl[g];
-            else
-            {
-                out[g].x = fmaf(pl[g].x, t2[g][i2], out[g].x);
-                out[g].y = fmaf(pl[g].y, t2[g][i2], out[g].y);
-            }
-        }
-    }
-}
-
-// eval_cone_g with the coefficients in memory, read PB axis-2 planes at a time (the loads of a
-// batch are not hoisted above the previous batch's arithmetic: fewer live registers)
+// The interpolants of one fine cone (coefficients c in memory, index i0 + O0 (i1 + O1 i2)) at G
+// points from their Chebyshev values: sum_{i0,i1,i2} c T_i0(x0) T_i1(x1) T_i2(x2), summed over
+// i0, then i1, then i2, each coefficient read once for the G points, PB axis-2 planes at a time
+// (the loads of a batch are not hoisted above the previous batch's arithmetic: fewer live
+// registers)
 template <int O0, int O1, int O2, int G, int PB = (O2 % 2 == 0) ? 2 : 1>
 __device__ __forceinline__ void eval_cone_g_mem(const float2* c,
                                                 const float (&t0)[G][O0], const float (&t1)[G][O1],
@@ -861,244 +812,6 @@ __global__ __launch_bounds__(256) void k_transform_t(int64_t c0, int64_t c1,
     }
 }
 
-// far field: for each target of the item, the interpolants of its far source boxes times the
-// centre factor (ifgfoperator.hpp:962-1012, 1708-1891).  FAST (mixed form): cones located by
-// locate_fast with the level's fine-grid angle tables (doubles [ang_base, ang_base + ang_n) of
-// ang, shared by every source box of the level) staged in LDS; otherwise the exact locate.
-constexpr int FAR_STAGE = 4; // distinct cones per wave and source box staged in LDS
-
-// one-wave exchanges through LDS: the wave's LDS writes have completed before its next LDS
-// reads issue (other lanes read what a lane wrote); the memory clobber keeps the compiler from
-// moving LDS accesses across
-__device__ __forceinline__ void lds_wait()
-{
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-}
-
-template <bool PH, typename R, int O0, int O1, int O2, bool FAST, int WPB, bool DEC>
-// the mixed order-6 kernel fits 64 VGPRs without spilling: ask for 8 waves per SIMD (the far
-// field is latency-bound; 74 registers would allow 6); at larger orders 4 waves (128 VGPRs)
-__global__ __launch_bounds__(64 * WPB)
-__attribute__((amdgpu_waves_per_eu(FAST && sizeof(R) == 4 ? (O1 == 3 ? 8 : 4) : 1))) void k_far(const WorkItem* __restrict__ items,
-                                                 int64_t nitems,
-                                            const int32_t* __restrict__ srange,
-                                            const int32_t* __restrict__ far_src,
-                                            const BoxGeo* __restrict__ geo,
-                                            const CellRef* __restrict__ ctab,
-                                            const Cx<R>* __restrict__ F,
-                                            const double* __restrict__ tpts,
-                                            const double* __restrict__ ang, int ang_base,
-                                            int ang_n, int split, int64_t ntgt,
-                                            Cx<R>* __restrict__ far_res, KParams kp)
-{
-    extern __shared__ double sang[];
-    __shared__ Cx<R> psum[WPB > 1 ? WPB : 1][WPB > 1 ? 64 : 1];
-    __shared__ float4 fstage[WPB][FAST && O0 * O1 * O2 >= 50 ? FAR_STAGE * (O0 * O1 * O2 / 2) : 1];
-    // WPB waves per workgroup, sharing the staged angle tables (one copy per workgroup: the
-    // tables, not the registers, would otherwise bound the waves per CU): one item each, or
-    // (split) a run each of one item's sources
-    const int lane = WPB == 1 ? int(threadIdx.x) : int(threadIdx.x & 63);
-    const int wave = WPB == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool shared = WPB > 1 && split;
-    const int64_t it = shared ? xcd_block(kp.xlg) : xcd_block(kp.xlg) * WPB + wave;
-    if (WPB == 1 && it >= nitems)
-        return;
-    if constexpr (FAST)
-    {
-        for (int i = threadIdx.x; i < ang_n; i += 64 * WPB)
-            sang[i] = ang[ang_base + i];
-        __syncthreads();
-    }
-    if (WPB > 1 && it >= nitems)
-        return;
-    const WorkItem wi = items[it];
-    const int Tp = pow2_at_least(wi.count);
-    const int ti = lane & (Tp - 1);
-    const int grp = lane / Tp, ngrp = 64 / Tp;
-    const bool valid = ti < wi.count;
-    const int64_t t = int64_t(wi.first) + (valid ? ti : 0);
-    const double y0 = tpts[3 * t], y1 = tpts[3 * t + 1], y2 = tpts[3 * t + 2];
-    Cx<R> acc = {0, 0};
-    int32_t j0 = srange[2 * it], j1 = srange[2 * it + 1];
-    if (shared)
-    {
-        const int32_t n = j1 - j0, a = j0;
-        j0 = a + n * wave / WPB;
-        j1 = a + n * (wave + 1) / WPB;
-    }
-    auto body = [&](const BoxGeo& B)
-    {
-        int fine;
-        double r, rinv;
-        R x0, x1, x2;
-        if constexpr (FAST)
-        {
-            LocF L;
-            const double* eth = sang + (2 * B.fth_off - ang_base);
-            const double* eph = sang + (2 * B.fph_off - ang_base);
-            constexpr int FF = O0 > 0 ? 3 : 0; // the compiled order classes use factor 3
-            if (!locate_fast<FF>(B, eth, eph, ctab, y0 - B.ctr[0], y1 - B.ctr[1], y2 - B.ctr[2],
-                                 kp.f0, kp.f1, kp.f2, L))
-                return;
-            fine = L.fine;
-            r = L.r;
-            rinv = L.rinv;
-            x0 = L.xi[0];
-            x1 = L.xi[1];
-            x2 = L.xi[2];
-        }
-        else
-        {
-            Loc L;
-            if (!locate(B, ctab, y0 - B.ctr[0], y1 - B.ctr[1], y2 - B.ctr[2], kp.f0, kp.f1, kp.f2,
-                        L))
-                return;
-            fine = L.fine;
-            r = L.r;
-            rinv = 1.0 / L.r;
-            x0 = R(L.xi[0]);
-            x1 = R(L.xi[1]);
-            x2 = R(L.xi[2]);
-        }
-        Cx<R> val;
-        if constexpr (FAST && O0 > 0)
-        {
-            // FP32, compiled orders: the interpolant from its Chebyshev values, the cone's
-            // coefficients loaded first as whole float4
-            float t0[1][O0], t1[1][O1], t2[1][O2];
-            cheb_t<O0>(x0, t0[0]);
-            cheb_t<O1>(x1, t1[0]);
-            cheb_t<O2>(x2, t2[0]);
-            float2 v[1];
-            constexpr int NC = O0 * O1 * O2;
-            constexpr int NQ = NC / 2; // float4 per cone
-            float2 cc[NC];
-            // at 50 and more coefficients the distinct cones of the wave's lanes (2.4 on
-            // average at 1M points; up to FAR_STAGE) are read from memory once, by all lanes
-            // together, into LDS, and every lane reads its cone there: the same values with
-            // a tenth of the vector-memory traffic.  A wave with more distinct cones, and
-            // every wave at fewer coefficients, reads memory directly.
-            bool staged = false;
-            if constexpr (NC >= 50)
-            {
-                const uint64_t act = __ballot(1);
-                const int rank = __popcll(act & ((1ull << lane) - 1ull));
-                const int nact = __popcll(act);
-                uint64_t rem = act;
-                int myslot = 0, nd = 0;
-                int cs[FAR_STAGE] = {};
-#pragma unroll 1
-                while (rem != 0 && nd < FAR_STAGE)
-                {
-                    const int l0 = __ffsll((unsigned long long)rem) - 1;
-                    const int f0 = __builtin_amdgcn_readlane(fine, l0);
-                    const uint64_t m = __ballot(fine == f0);
-                    if (fine == f0)
-                        myslot = nd;
-#pragma unroll
-                    for (int e = 0; e < FAR_STAGE; e++)
-                        cs[e] = nd == e ? f0 : cs[e];
-                    rem &= ~m;
-                    nd++;
-                }
-                if (rem == 0) // uniform
-                {
-                    float4* st4 = fstage[WPB == 1 ? 0 : (threadIdx.x >> 6)];
-                    for (int i = rank; i < nd * NQ; i += nact)
-                    {
-                        const int d = i / NQ, k = i - d * NQ;
-                        int cf = cs[0];
-#pragma unroll
-                        for (int e = 1; e < FAR_STAGE; e++)
-                            cf = d == e ? cs[e] : cf;
-                        st4[i] = reinterpret_cast<const float4*>(F + int64_t(cf) * NC)[k];
-                    }
-                    lds_wait(); // the wave's LDS writes are complete before it reads them
-                    const float4* q4 = st4 + myslot * NQ;
-#pragma unroll
-                    for (int i = 0; i < NQ; i++)
-                    {
-                        const float4 q = q4[i];
-                        cc[2 * i] = make_float2(q.x, q.y);
-                        cc[2 * i + 1] = make_float2(q.z, q.w);
-                    }
-                    eval_cone_g<O0, O1, O2, 1>(cc, t0, t1, t2, v);
-                    staged = true;
-                }
-            }
-            if (!staged)
-            {
-                const float4* p4 = reinterpret_cast<const float4*>(F + int64_t(fine) * NC);
-#pragma unroll
-                for (int i = 0; i < NQ; i++)
-                {
-                    const float4 q = p4[i];
-                    cc[2 * i] = make_float2(q.x, q.y);
-                    cc[2 * i + 1] = make_float2(q.z, q.w);
-                }
-                eval_cone_g<O0, O1, O2, 1>(cc, t0, t1, t2, v);
-            }
-            // the next source box's staging writes stay behind this box's LDS reads
-            asm volatile("" ::: "memory");
-            val = {v[0].x, v[0].y};
-        }
-        else
-            val = fine_eval<O0, O1, O2, R>(F, fine, kp, x0, x1, x2);
-        Cx<R> cf;
-        if constexpr (!PH)
-            cf = {R(INV_4PI_D * rinv), R(0)};
-        else
-            cf = cscale(expmk_far<R, DEC>(B.k_re, B.k_im, r), R(INV_4PI_D * rinv));
-        acc = cadd(acc, cmul(val, cf));
-    };
-    // the next source box's index is loaded one box ahead, so that its geometry loads do not
-    // wait for it
-    if (ngrp == 1)
-    {
-        // uniform source box: scalar loads of its geometry
-        int32_t sn = j0 < j1 ? far_src[j0] : 0;
-        for (int32_t j = j0; j < j1; j++)
-        {
-            const int32_t sb = __builtin_amdgcn_readfirstlane(sn);
-            if (j + 1 < j1)
-                sn = far_src[j + 1];
-            body(geo[sb]);
-        }
-    }
-    else
-    {
-        int32_t sn = j0 + grp < j1 ? far_src[j0 + grp] : 0;
-        for (int32_t j = j0 + grp; j < j1; j += ngrp)
-        {
-            const int32_t sb = sn;
-            if (j + ngrp < j1)
-                sn = far_src[j + ngrp];
-            body(geo[sb]);
-        }
-        for (int m = Tp; m < 64; m <<= 1)
-        {
-            acc.x += __shfl_xor(acc.x, m, 64);
-            acc.y += __shfl_xor(acc.y, m, 64);
-        }
-    }
-    if constexpr (WPB > 1)
-        if (shared)
-        {
-            psum[wave][lane] = acc;
-            __syncthreads();
-            if (wave)
-                return;
-#pragma unroll
-            for (int w = 1; w < WPB; w++)
-                acc = cadd(acc, psum[w][lane]);
-        }
-    if (grp == 0 && valid)
-    {
-        Cx<R>* res = far_res + wi.pad * ntgt + t;
-        *res = cadd(*res, acc);
-    }
-}
-
 // ------------------------------------------------------------------------------------
 // host helpers
 // ------------------------------------------------------------------------------------
@@ -1273,105 +986,48 @@ GroupTables<Rec> group_tables(const std::vector<const UpLevel*>& parts, int n_hi
     return T;
 }
 
-// up_level >= 0: the upward pass into parent level up_level; otherwise the far field of
-// target level far_level
-template <bool PH, typename R, int H0, int H1, int H2, int O0, int O1, int O2, bool DEC>
-void launch_up_far_t(DevicePlan& D, hipStream_t st, const KParams& kp, const NodeTabs& tabs,
-                     int up_level, int far_level, int64_t a, int64_t b, Cx<R>* F, Cx<R>* V,
-                     Cx<R>* res, Cx<R>* Fo)
+// the upward pass into parent level `level`: cones with a table, then cones a .. b of the others
+template <bool PH, typename R, int H0, int H1, int H2, int O0, int O1, int O2>
+void launch_up_t(DevicePlan& D, hipStream_t st, const KParams& kp, const NodeTabs& tabs, int level,
+                 int64_t a, int64_t b, Cx<R>* F, Cx<R>* V, Cx<R>* Fo)
 {
-    const bool up = up_level >= 0;
-    if (up)
+    if constexpr (sizeof(R) == 4 && O0 > 0)
     {
-        if constexpr (sizeof(R) == 4 && O0 > 0)
-        {
-            // FP32, compiled orders (at the larger orders with their transform: the cones' fine
-            // coefficients go to Fo, the values nowhere)
-            constexpr bool TF = up_fuses_transform(O0 * O1 * O2);
-            const int64_t n = D.up_gl_off[up_level + 1] - D.up_gl_off[up_level];
-            if (n > 0 && !D.up_tl_desc)
-                throw std::runtime_error("upward pass: the per-cone records were not uploaded");
-            const int K = up_cones_per_block(D, n);
-            if (n > 0)
-                k_up_grp<O0, O1, O2, H0 * H1 * H2, 128, H0, H1, H2, TF>
-                    <<<dim3(unsigned((n + K - 1) / K)), dim3(128), 0, st>>>(
-                        D.up_tl_desc + D.up_gl_off[up_level], n, K, D.ctab,
-                        static_cast<const UpGrp*>(D.up_grp), F, V,
-                        static_cast<const float*>(D.wmat), Fo, kp);
-        }
-        else
-            launch_up_rows<R>(D, st, kp, up_level, F, V);
-        if (b > a)
-            k_up<PH, R, O0, O1, O2><<<dim3(unsigned(b - a)), dim3(128), 0, st>>>(
-                D.up_cones + a, b - a, D.cones, D.geo, D.child, D.ctab, tabs, F, V, kp);
+        // FP32, compiled orders (at the larger orders with their transform: the cones' fine
+        // coefficients go to Fo, the values nowhere)
+        constexpr bool TF = up_fuses_transform(O0 * O1 * O2);
+        const int64_t n = D.up_gl_off[level + 1] - D.up_gl_off[level];
+        if (n > 0 && !D.up_tl_desc)
+            throw std::runtime_error("upward pass: the per-cone records were not uploaded");
+        const int K = up_cones_per_block(D, n);
+        if (n > 0)
+            k_up_grp<O0, O1, O2, H0 * H1 * H2, 128, H0, H1, H2, TF>
+                <<<dim3(unsigned((n + K - 1) / K)), dim3(128), 0, st>>>(
+                    D.up_tl_desc + D.up_gl_off[level], n, K, D.ctab,
+                    static_cast<const UpGrp*>(D.up_grp), F, V, static_cast<const float*>(D.wmat),
+                    Fo, kp);
     }
     else
-    {
-        // far_level: the far group; a, b: its items
-        // (the compiled order classes keep k_far, which has the orders and the kernel family at
-        // compile time: far phase 4.3 against 5.8 ms at (2,3,3), 7.1 against 7.7 ms at (2,5,5),
-        // 1M points; FP64 at (3,5,4), 99,991 points, 2.2 against 2.8 ms)
-        if constexpr (O0 == 0)
-            launch_far_rows<R>(D, st, kp, far_level, F, res);
-        else
-        {
-            const int abase = D.far_steps[far_level].ang_base, an = D.far_steps[far_level].ang_n;
-            const int64_t n = b - a;
-            // few items: 2 to 8 waves share an item's sources, else the shape's waves take an
-            // item each
-            const int split = far_split(n);
-#define IFGF_FAR(FAST, WPB, LDS, BASE, AN)                                                      \
-    k_far<PH, R, O0, O1, O2, FAST, WPB, DEC>                                                    \
-        <<<dim3(unsigned(split > 1 ? n : (n + WPB - 1) / WPB)), dim3(64 * WPB), LDS, st>>>(     \
-            D.far_items + a, n, D.far_srange + 2 * a, D.far_src, D.geo, D.ctab, F, D.tgt_pts,   \
-            D.fine_ang, BASE, AN, split > 1, D.ntgt, res, kp)
-#define IFGF_FAR_W(FAST, WAVES, LDS, BASE, AN)                                                  \
-    switch (WAVES)                                                                              \
-    {                                                                                           \
-    case 2:                                                                                     \
-        IFGF_FAR(FAST, 2, LDS, BASE, AN);                                                       \
-        break;                                                                                  \
-    case 4:                                                                                     \
-        IFGF_FAR(FAST, 4, LDS, BASE, AN);                                                       \
-        break;                                                                                  \
-    case 8:                                                                                     \
-        IFGF_FAR(FAST, 8, LDS, BASE, AN);                                                       \
-        break;                                                                                  \
-    default:                                                                                    \
-        IFGF_FAR(FAST, 1, LDS, BASE, AN);                                                       \
-    }
-            if constexpr (sizeof(R) == 4)
-                if (an > 0)
-                {
-                    const size_t lds = size_t(an) * sizeof(double);
-                    const int waves = split > 1 ? split : D.shape.far_waves;
-                    IFGF_FAR_W(true, waves, lds, abase, an);
-                    return;
-                }
-            IFGF_FAR_W(false, split, 0, 0, 0);
-#undef IFGF_FAR_W
-#undef IFGF_FAR
-        }
-    }
+        launch_up_rows<R>(D, st, kp, level, F, V);
+    if (b > a)
+        k_up<PH, R, O0, O1, O2><<<dim3(unsigned(b - a)), dim3(128), 0, st>>>(
+            D.up_cones + a, b - a, D.cones, D.geo, D.child, D.ctab, tabs, F, V, kp);
 }
 
-// DEC: the kernel family's wavenumber may have a real part (e^{-k r} decays); false for the
-// real-kappa families, whose far field then forms the phase only
-template <bool PH, typename R, bool DEC>
-void launch_up_far(DevicePlan& D, hipStream_t st, const KParams& kp, const NodeTabs& tabs, int up,
-                   int far, int64_t a, int64_t b, Cx<R>* F, Cx<R>* V, Cx<R>* res,
-                   Cx<R>* Fo = nullptr)
+template <bool PH, typename R>
+void launch_up(DevicePlan& D, hipStream_t st, const KParams& kp, const NodeTabs& tabs, int level,
+               int64_t a, int64_t b, Cx<R>* F, Cx<R>* V, Cx<R>* Fo)
 {
     switch (order_class(D))
     {
     case 1:
-        return launch_up_far_t<PH, R, 3, 6, 6, 2, 3, 3, DEC>(D, st, kp, tabs, up, far, a, b, F, V, res, Fo);
+        return launch_up_t<PH, R, 3, 6, 6, 2, 3, 3>(D, st, kp, tabs, level, a, b, F, V, Fo);
     case 2:
-        return launch_up_far_t<PH, R, 5, 8, 8, 2, 5, 5, DEC>(D, st, kp, tabs, up, far, a, b, F, V, res, Fo);
+        return launch_up_t<PH, R, 5, 8, 8, 2, 5, 5>(D, st, kp, tabs, level, a, b, F, V, Fo);
     case 3:
-        return launch_up_far_t<PH, R, 6, 8, 7, 3, 5, 4, DEC>(D, st, kp, tabs, up, far, a, b, F, V, res, Fo);
+        return launch_up_t<PH, R, 6, 8, 7, 3, 5, 4>(D, st, kp, tabs, level, a, b, F, V, Fo);
     default:
-        return launch_up_far_t<PH, R, 0, 0, 0, 0, 0, 0, DEC>(D, st, kp, tabs, up, far, a, b, F, V, res, Fo);
+        return launch_up_t<PH, R, 0, 0, 0, 0, 0, 0>(D, st, kp, tabs, level, a, b, F, V, Fo);
     }
 }
 
@@ -1583,7 +1239,6 @@ template <int KIND, typename R>
 void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
 {
     constexpr bool PH = KIND != KL;
-    constexpr bool DEC = KIND != KH && KIND != KC; // real kappa: kr = 0
     // k_up_grp transforms the cones it computes (FP32, compiled orders, enough coefficients)
     const bool fused = sizeof(R) == 4 && up_fused_transform(D);
     const KParams kp = kparams(D);
@@ -1634,9 +1289,11 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
         },
         [&](int g, hipStream_t s)
         {
-            const DevicePlan::FarGroup& G = D.far_steps[g];
-            launch_up_far<PH, R, DEC>(D, s, kp, tabs, -1, g, G.item0, G.item1, Fl(G.src_level), V,
-                                      far_res);
+            Cx<R>* f = Fl(D.far_steps[g].src_level);
+            if (D.far_rec)
+                launch_far_rec<R>(D, s, kp, g, f, far_res);
+            else
+                launch_far_rows<R>(D, s, kp, g, f, far_res);
         });
     if (overlap != 1)
         pipe.fork(); // the near field first, on the main stream (inside the timed near phase)
@@ -1664,8 +1321,7 @@ void run_core(DevicePlan& D, hipStream_t st, PhaseTimer& pt, const Stage& sg)
         if (u1 > u0 || D.up_gl_off[l + 1] > D.up_gl_off[l])
         {
             pt.begin(2);
-            launch_up_far<PH, R, DEC>(D, st, kp, tabs, l, -1, u0, u1, Fl(l + 1), Vl(l), res,
-                                      Fl(l));
+            launch_up<PH, R>(D, st, kp, tabs, l, u0, u1, Fl(l + 1), Vl(l), Fl(l));
             pt.end();
         }
         if (c1 > c0)
@@ -1833,7 +1489,7 @@ void device_free(DevicePlan& D)
                     D.src_end, D.child, D.geo, D.cones, D.ctab, D.ho_nodes, D.trig_th,
                     D.trig_ph, D.fine_ang, D.wmat, D.up_grp, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
-                    D.near_off, D.near_run, D.near_pts, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.V,
+                    D.near_off, D.near_run, D.near_pts, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.far_rec_off, D.far_rec, D.far_cf, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
                     D.b_out, D.h_in, D.h_out};
     for (void* p : ptrs)
@@ -2407,6 +2063,25 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
             D.V = dalloc<unsigned char>(cs * size_t(std::max<int64_t>(1, D.n_cones)) * D.n_hi, tot);
             D.F = dalloc<unsigned char>(
                 cs * (size_t(std::max<int64_t>(1, D.n_fine)) * D.n_lo + ROW_PAD), tot);
+        }
+        {
+            // the far pair records
+            std::vector<int64_t> roff(fitems.size() + 1, 0);
+            for (size_t i = 0; i < fitems.size(); i++)
+                roff[i + 1] = roff[i] + int64_t(fitems[i].count) * (frange[2 * i + 1] - frange[2 * i]);
+            const size_t pairs = size_t(roff.back());
+            const size_t rs = precision == PREC_FP64 ? sizeof(FarRec<double>) : sizeof(FarRec<float>);
+            HIP_OK(hipMemGetInfo(&free_b, &total_b));
+            if (pairs > 0 && (rs + cs) * pairs <= free_b / 4)
+            {
+                D.far_rec_off = dupload(roff, tot);
+                D.far_rec = dalloc<unsigned char>(rs * pairs, tot);
+                D.far_cf = dalloc<unsigned char>(cs * pairs, tot);
+                if (precision == PREC_FP64)
+                    record_far<double>(D);
+                else
+                    record_far<float>(D);
+            }
         }
         HIP_OK(hipDeviceSynchronize());
     }

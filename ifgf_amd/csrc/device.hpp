@@ -188,6 +188,15 @@ struct DevicePlan
     // levels with far items) add to their own results, far_res[pad * ntgt ..], and the scatter
     // sums the levels in order.
     std::vector<FarGroup> far_steps;
+    // Where each (target, far source box) pair lies, in the order of the far items (item i's
+    // records from far_rec_off[i] on, its targets fastest): the fine slot and local coordinates
+    // (FarRec) and the centre factor.  All from the geometry and the wavenumber, so recorded once
+    // at upload by the location the far field would otherwise repeat in every mult; null when
+    // they would take more than a quarter of the free device memory (24 bytes a pair in the mixed
+    // form, 48 in FP64).
+    int64_t* far_rec_off = nullptr;
+    void* far_rec = nullptr; // FarRec<R>
+    void* far_cf = nullptr;  // Cx<R>
     int n_far_lvls = 0;
     void* far_res = nullptr; // n_far_lvls * ntgt complex (R)
     WorkItem* near_items = nullptr;

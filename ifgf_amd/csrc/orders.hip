@@ -168,12 +168,12 @@ __device__ __forceinline__ void wave_lds_wait()
 
 // the nc coefficients of cones c0 .. c3 (the first nd of them) to LDS, `stride` entries apart, by
 // the nact active lanes of a wave together; U: 16 bytes where a cone is whole 16-byte words
-template <class U>
-__device__ __forceinline__ void stage_cones(const Cx<float>* __restrict__ F, int c0, int c1, int c2,
+template <class U, typename R>
+__device__ __forceinline__ void stage_cones(const Cx<R>* __restrict__ F, int c0, int c1, int c2,
                                             int c3, int nd, int nc, int stride, int rank, int nact,
-                                            Cx<float>* sc)
+                                            Cx<R>* sc)
 {
-    constexpr int E = int(sizeof(U) / sizeof(Cx<float>));
+    constexpr int E = int(sizeof(U) / sizeof(Cx<R>));
     static_assert(FAR_STAGE == 4, "four cones");
     const int nu = nc / E;
 #pragma unroll 2
@@ -378,6 +378,215 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         *res = cadd(*res, acc);
     }
 }
+// the pair records of the items of one far launch: one wave per item (the order of the records:
+// DevicePlan::far_rec)
+template <typename R, bool FAST>
+__global__ __launch_bounds__(64) void k_far_record(
+    const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
+    const int64_t* __restrict__ rec_off, const int32_t* __restrict__ far_src,
+    const BoxGeo* __restrict__ geo, const CellRef* __restrict__ ctab,
+    const double* __restrict__ tpts, const double* __restrict__ ang, int ang_base, int ang_n,
+    int phase, FarRec<R>* __restrict__ rec, Cx<R>* __restrict__ cfs, KParams kp)
+{
+    extern __shared__ double rec_ang[];
+    const int64_t it = blockIdx.x;
+    if constexpr (FAST)
+    {
+        for (int i = threadIdx.x; i < ang_n; i += 64)
+            rec_ang[i] = ang[ang_base + i];
+        __syncthreads();
+    }
+    const WorkItem wi = items[it];
+    const int32_t j0 = srange[2 * it], n = srange[2 * it + 1] - j0;
+    const int64_t off = rec_off[it];
+    for (int e = threadIdx.x; e < n * wi.count; e += 64)
+    {
+        const int j = e / wi.count;
+        const int64_t t = int64_t(wi.first) + (e - j * wi.count);
+        const BoxGeo& B = geo[far_src[j0 + j]];
+        const double v0 = tpts[3 * t] - B.ctr[0], v1 = tpts[3 * t + 1] - B.ctr[1],
+                     v2 = tpts[3 * t + 2] - B.ctr[2];
+        FarRec<R> q{};
+        q.slot = -1;
+        Cx<R> cf = {R(0), R(0)};
+        double r = 1, ri = 1;
+        bool ok;
+        if constexpr (FAST)
+        {
+            LocF L;
+            ok = locate_fast(B, rec_ang + (2 * B.fth_off - ang_base),
+                             rec_ang + (2 * B.fph_off - ang_base), ctab, v0, v1, v2, kp.f0, kp.f1,
+                             kp.f2, L);
+            if (ok)
+            {
+                q.slot = L.fine;
+                q.x0 = R(L.xi[0]);
+                q.x1 = R(L.xi[1]);
+                q.x2 = R(L.xi[2]);
+                r = L.r;
+                ri = L.rinv;
+            }
+        }
+        else
+        {
+            Loc L;
+            ok = locate(B, ctab, v0, v1, v2, kp.f0, kp.f1, kp.f2, L);
+            if (ok)
+            {
+                q.slot = L.fine;
+                q.x0 = R(L.xi[0]);
+                q.x1 = R(L.xi[1]);
+                q.x2 = R(L.xi[2]);
+                r = L.r;
+                ri = 1.0 / L.r;
+            }
+        }
+        if (ok)
+            cf = phase ? cscale(expmk_far<R>(B.k_re, B.k_im, r), R(INV_4PI_D * ri))
+                       : Cx<R>{R(INV_4PI_D * ri), R(0)};
+        rec[off + e] = q;
+        cfs[off + e] = cf;
+    }
+}
+
+// Far field from the pair records, any orders: as k_far_rows without the cone location.  A step
+// reads the pairs' records (one step ahead), then their cones: with stage > 0 the distinct cones
+// of the wave's lanes copied to LDS by all lanes together, otherwise each lane's from memory.
+// Bound by memory: the records are most of its traffic.  Far phase against locating the cones in
+// every mult: 7.5 -> 4.5 ms
+// at (3,6,4), 1M points; 3.7 -> 2.4 ms at (2,3,3), 1M points; FP64 at (3,5,4), 99,991 points,
+// 1.6 -> 0.63 ms.
+template <typename R, int O0, int O1>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 9 ? 7 : 5) : 3))) void k_far_rec(
+    const WorkItem* __restrict__ items, int64_t nitems, const int32_t* __restrict__ srange,
+    const int64_t* __restrict__ rec_off, const FarRec<R>* __restrict__ rec,
+    const Cx<R>* __restrict__ cfs, const Cx<R>* __restrict__ F, int stage, int stride, int split,
+    int64_t ntgt, Cx<R>* __restrict__ far_res, KParams kp)
+{
+    extern __shared__ __align__(16) unsigned char far_smem[];
+    __shared__ Cx<R> psum[8][64];
+    const int lane = int(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wpb = int(blockDim.x >> 6);
+    Cx<R>* sc = reinterpret_cast<Cx<R>*>(far_smem) + wave * (FAR_STAGE * stride + ROW_PAD);
+    const int64_t it = split ? xcd_block(kp.xlg) : xcd_block(kp.xlg) * wpb + wave;
+    if (it >= nitems)
+        return;
+    const WorkItem wi = items[it];
+    const int Tp = pow2_at_least(wi.count);
+    const int ti = lane & (Tp - 1);
+    const int grp = lane / Tp, ngrp = 64 / Tp;
+    const bool valid = ti < wi.count;
+    const int32_t n = srange[2 * it + 1] - srange[2 * it];
+    int32_t ja = 0, jb = n;
+    if (split) // a run of the item's sources per wave
+    {
+        ja = n * wave / wpb;
+        jb = n * (wave + 1) / wpb;
+    }
+    const FarRec<R>* rp = rec + rec_off[it] + ti;
+    const Cx<R>* cp = cfs + rec_off[it] + ti;
+    Cx<R> acc = {0, 0};
+    FarRec<R> q;
+    Cx<R> cf;
+    auto fetch = [&](int32_t j)
+    {
+        q.slot = -1;
+        if (valid && j + grp < jb)
+        {
+            const int64_t e = int64_t(j + grp) * wi.count;
+            q = rp[e];
+            cf = cp[e];
+        }
+    };
+    fetch(ja);
+    for (int32_t j = ja; j < jb; j += ngrp)
+    {
+        const int fine = q.slot;
+        const R x0 = q.x0, x1 = q.x1, x2 = q.x2;
+        const Cx<R> c0 = cf;
+        fetch(j + ngrp);
+        const Cx<R>* c = F + int64_t(fine) * kp.n_lo;
+        bool staged = false;
+        if (stage > 0)
+        {
+            uint64_t rem = __ballot(fine >= 0);
+            int myslot = 0, nd = 0;
+            int cs[FAR_STAGE] = {};
+#pragma unroll 1
+            while (rem != 0 && nd < FAR_STAGE)
+            {
+                const int f0 = __builtin_amdgcn_readlane(fine, __ffsll((unsigned long long)rem) - 1);
+                const uint64_t m = __ballot(fine == f0);
+                if (fine == f0)
+                    myslot = nd;
+#pragma unroll
+                for (int e = 0; e < FAR_STAGE; e++)
+                    cs[e] = nd == e ? f0 : cs[e];
+                rem &= ~m;
+                nd++;
+            }
+            if (rem == 0) // uniform
+            {
+                if (sizeof(R) == 4 && (kp.n_lo & 1))
+                    stage_cones<typename std::conditional<sizeof(R) == 4, float2, float4>::type>(
+                        F, cs[0], cs[1], cs[2], cs[3], nd, kp.n_lo, stride, lane,
+                                        64, sc);
+                else
+                    stage_cones<float4>(F, cs[0], cs[1], cs[2], cs[3], nd, kp.n_lo, stride, lane,
+                                        64, sc);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                staged = true;
+                if (fine >= 0)
+                {
+                    const Cx<R>* l = sc + myslot * stride;
+                    Cx<R> v[1];
+                    if constexpr (O0 > 0)
+                        v[0] = eval_point<R, O0, O1>(l, kp.lo2, x0, x1, x2);
+                    else
+                    {
+                        const R y0[1] = {x0}, y1[1] = {x1}, y2[1] = {x2};
+                        eval_any<R, 1>(l, kp.lo0, kp.lo1, kp.lo2, y0, y1, y2, v);
+                    }
+                    acc = cadd(acc, cmul(v[0], c0));
+                }
+                // the next step's staging writes stay behind this step's LDS reads
+                asm volatile("" ::: "memory");
+            }
+        }
+        if (!staged && fine >= 0)
+        {
+            Cx<R> v[1];
+            if constexpr (O0 > 0)
+                v[0] = eval_point<R, O0, O1>(c, kp.lo2, x0, x1, x2);
+            else
+            {
+                const R y0[1] = {x0}, y1[1] = {x1}, y2[1] = {x2};
+                eval_any<R, 1>(c, kp.lo0, kp.lo1, kp.lo2, y0, y1, y2, v);
+            }
+            acc = cadd(acc, cmul(v[0], c0));
+        }
+    }
+    for (int m = Tp; m < 64; m <<= 1)
+    {
+        acc.x += __shfl_xor(acc.x, m, 64);
+        acc.y += __shfl_xor(acc.y, m, 64);
+    }
+    if (split)
+    {
+        psum[wave][lane] = acc;
+        __syncthreads();
+        if (wave)
+            return;
+        for (int w = 1; w < wpb; w++)
+            acc = cadd(acc, psum[w][lane]);
+    }
+    if (grp == 0 && valid)
+    {
+        Cx<R>* res = far_res + wi.pad * ntgt + wi.first + ti;
+        *res = cadd(*res, acc);
+    }
+}
+
 // High-order values -> fine coefficients of the active sub-cones at any orders and factors
 // (chebinterp.hpp:176-250, ifgfoperator.hpp:1539-1637), separable per axis as k_transform_t: one
 // thread per pencil and axis, cpb cones per workgroup (X: xsz entries per cone, the values, then
@@ -596,5 +805,65 @@ template void launch_transform_rows<float>(DevicePlan&, hipStream_t, const KPara
                                            int64_t, const Cx<float>*, Cx<float>*);
 template void launch_transform_rows<double>(DevicePlan&, hipStream_t, const KParams&, int64_t,
                                             int64_t, const Cx<double>*, Cx<double>*);
+
+template <typename R> void record_far(DevicePlan& D)
+{
+    const KParams kp = kparams(D);
+    const int phase = D.kind != KL;
+    for (const DevicePlan::FarGroup& G : D.far_steps)
+    {
+        const dim3 grid(unsigned(G.item1 - G.item0));
+        const int64_t i0 = G.item0;
+        auto* rec = static_cast<FarRec<R>*>(D.far_rec);
+        auto* cf = static_cast<Cx<R>*>(D.far_cf);
+        if (sizeof(R) == 4 && G.ang_n > 0)
+            k_far_record<R, true><<<grid, dim3(64), size_t(G.ang_n) * sizeof(double)>>>(
+                D.far_items + i0, D.far_srange + 2 * i0, D.far_rec_off + i0, D.far_src, D.geo,
+                D.ctab, D.tgt_pts, D.fine_ang, G.ang_base, G.ang_n, phase, rec, cf, kp);
+        else
+            k_far_record<R, false><<<grid, dim3(64)>>>(
+                D.far_items + i0, D.far_srange + 2 * i0, D.far_rec_off + i0, D.far_src, D.geo,
+                D.ctab, D.tgt_pts, D.fine_ang, 0, 0, phase, rec, cf, kp);
+        HIP_OK(hipGetLastError());
+    }
+}
+template void record_far<float>(DevicePlan&);
+template void record_far<double>(DevicePlan&);
+
+template <typename R>
+void launch_far_rec(DevicePlan& D, hipStream_t st, const KParams& kp, int group, const Cx<R>* F,
+                    Cx<R>* far_res)
+{
+    const DevicePlan::FarGroup& G = D.far_steps[group];
+    const int64_t n = G.item1 - G.item0;
+    const int split = far_split(n);
+    const int wpb = split > 1 ? split : D.shape.far_waves;
+    // (staging from 16 coefficients on: far phase at (2,3,3), 262,144 points, 0.76 against 0.98 ms
+    // with every lane reading its cone from memory; at (2,5,5), 1M points, 3.5 against 6.7 ms)
+    // up to 112 KB per workgroup
+    const int stride = (((D.n_lo + 1) / 2) | 1) * 2;
+    const size_t staged = size_t(wpb) * (FAR_STAGE * stride + ROW_PAD) * sizeof(Cx<R>);
+    const int stage = D.n_lo >= 16 && staged <= size_t(112) * 1024 ? D.n_lo : 0;
+    const size_t lds = stage ? staged : 0;
+    with_orders(D.lo[0], D.lo[1], [&](auto o0, auto o1)
+                {
+                    constexpr int O0 = decltype(o0)::value, O1 = decltype(o1)::value;
+                    if (lds > size_t(64) * 1024)
+                        HIP_OK(hipFuncSetAttribute(
+                            reinterpret_cast<const void*>(&k_far_rec<R, O0, O1>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+                    k_far_rec<R, O0, O1>
+                        <<<dim3(unsigned(split > 1 ? n : (n + wpb - 1) / wpb)), dim3(64 * wpb),
+                           lds, st>>>(D.far_items + G.item0, n, D.far_srange + 2 * G.item0,
+                                      D.far_rec_off + G.item0,
+                                      static_cast<const FarRec<R>*>(D.far_rec),
+                                      static_cast<const Cx<R>*>(D.far_cf), F, stage, stride,
+                                      split > 1, D.ntgt, far_res, kp);
+                });
+}
+template void launch_far_rec<float>(DevicePlan&, hipStream_t, const KParams&, int,
+                                    const Cx<float>*, Cx<float>*);
+template void launch_far_rec<double>(DevicePlan&, hipStream_t, const KParams&, int,
+                                     const Cx<double>*, Cx<double>*);
 } // namespace dev
 } // namespace ifgf

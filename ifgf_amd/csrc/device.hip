@@ -1523,6 +1523,10 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
     {
         device_free(D);
         HIP_OK(hipGetDevice(&D.device));
+        // Two parent cones per upward workgroup: a cone's tasks fill its threads, so more of them
+        // only make the workgroups fewer and longer.  Whole mult with 2 / 16 at 1M points:
+        // 22.7 / 23.4 ms at (6,9,7)/(3,6,4), 14.9 / 15.6 at (5,8,8)/(2,5,5), 7.0 / 7.2 at order 6.
+        D.shape.up_k = 2;
         {
             // the allocation-free mult's scratch address on this device (once per device)
             std::string serr;
@@ -2082,6 +2086,10 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
                 else
                     record_far<float>(D);
             }
+            else
+                // the location runs per pair: two waves share the staged angle tables.  Whole
+                // mult with 2 / 1 at 1M points, (6,9,7)/(3,6,4): 24.7 / 25.8 ms
+                D.shape.far_waves = 2;
         }
         HIP_OK(hipDeviceSynchronize());
     }

@@ -67,15 +67,15 @@ struct PointRun // consecutive source points [begin, end) in Morton order
 };
 
 // Launch shapes of the mult's kernels: choices that change speed but not results, picked by
-// device_autotune (measured on the operator itself) or set by the caller.  The defaults at 1M
-// points, (6,9,7)/(3,6,4): 24.7 ms per mult; with 16 upward cones 25.4, with 1 far wave 25.8.
+// device_autotune (measured on the operator itself), set by the caller, or where the upload
+// starts from something else than these defaults (device_upload).
 struct LaunchShape
 {
     int xcd_log2 = 4; // work items dealt to the XCDs in runs of 2^xcd_log2 (0: plain order)
     int cpb = 0;      // transform: cones per workgroup (0: the order class's default)
-    int up_k = 2;     // upward: parent cones per workgroup (2, 4, 8 or 16)
+    int up_k = 16;    // upward: parent cones per workgroup (2, 4, 8 or 16)
     int rb = 0;       // batched: most columns per pass (8 or 32; 0: 32)
-    int far_waves = 2; // mixed far field: waves (items) per workgroup sharing the LDS tables
+    int far_waves = 1; // mixed far field: waves (items) per workgroup sharing the LDS tables
     int overlap = 1;   // far field on a second stream beside the upward chain, with the near
                        // field there too (1) or first on the main stream (2); 0: one stream
 };

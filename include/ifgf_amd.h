@@ -182,8 +182,8 @@ int ifgf_last_timings(const ifgf_operator* op, double* ms6);
  * shape: IFGF_LAUNCH_SHAPE_FIELDS ints
  *         [0] XCD run log2 (work items dealt to the 8 XCDs in runs of 2^v; 0 = plain order)
  *         [1] transform cones per workgroup (0 = default; the compiled order classes only)
- *         [2] upward parent cones per workgroup (2, 4, 8, 16; default 2)
- *         [3] batched columns per pass (0 = by nrhs, 8, 32)
+ *         [2] upward parent cones per workgroup, at most (2, 4, 8, 16; 2 after an init)
+ *         [3] batched columns per pass, at most (0 = 32, 8, 32)
  *         [4] mixed far field: waves per workgroup sharing the staged angle tables (1, 2, 4, 8)
  *         [5] second stream for the far field beside the upward chain, with the near field
  *             there (1) or first on the main stream (2); 0: one stream

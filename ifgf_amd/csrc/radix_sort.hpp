@@ -6,8 +6,9 @@
 // (stable scatter of each tile).  In the scatter, wave w of a tile owns records
 // [w * 512, (w + 1) * 512) taken 64 at a time in order; a record's rank among the equal digits
 // of its wave is the wave's running count of that digit (LDS) plus the lanes below it with the
-// same digit (eight ballots); per-wave prefix sums then place the waves' runs one after another.  Every pass is stable, so the passes together sort by the
-// digits of the last pass first, ties keeping the input order.
+// same digit (eight ballots); per-wave prefix sums then place the waves' runs one after another.
+// Every pass is stable, so the passes together sort by the digits of the last pass first, ties
+// keeping the input order.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -51,18 +51,19 @@ def direct_sum_torch(x, w, idx, kappa, dev):
 
 # the kernels of each phase, the first one found in a counter summary is the phase's
 KERNEL_OF_PHASE = {"near": ("k_near",), "leaf": ("k_leaf_box", "k_leaf"),
-                   "upward": ("k_up_grp", "k_up_cell"), "transform": ("k_transform_t",),
-                   "far": ("k_far",)}
+                   "upward": ("k_up_grp", "k_up_rows"),
+                   "transform": ("k_transform_t", "k_transform_rows"),
+                   "far": ("k_far_rec", "k_far_rows")}
 # what bounds each phase's kernel below the FP32 vector roofline, from the rocprofv3 SQ
 # instruction and HBM counters of the 1M-point workloads (profiles/)
 LIMITER = {
     "near": "VALU (issue rate near the practical ceiling)",
     "leaf": "VALU (issue rate near the practical ceiling)",
-    "upward": "vector-memory latency of the dependent record / coefficient loads (about three "
-              "quarters of the wave cycles wait), then VALU",
+    "upward": "child coefficients fetched about 3.5 times at 4.1 TB/s (a plain copy reaches "
+              "4.8), then VALU",
     "transform": "LDS traffic between the axis stages and the coefficient writes to HBM",
-    "far": "vector-memory latency of the cell-table and coefficient gathers (more than half of "
-           "the wave cycles wait) at 4 waves per SIMD, then VALU in the FP64 cone location",
+    "far": "streaming the pair records and the coefficients at 4.0-4.9 TB/s (a plain copy "
+           "reaches 4.8), then VALU",
 }
 # rocprofv3 counter summaries of the 1M-point workloads, by tolerance
 COUNTERS = {

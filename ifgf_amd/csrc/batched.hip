@@ -271,7 +271,7 @@ __device__ __forceinline__ void lds_fence()
 // axis 2, then axis 0 (171 MFMAs when every sub-cone is active; the 6 x 3 and 9 x 6 maps fill
 // 28% and 42% of a tile). Tile operands: lane l holds A[l % 16][l / 16] (map row, input index)
 // and B[l / 16][l % 16] (input index, column); the result tile row 4 (l / 16) + i, column
-// l % 16 is element i of lane l. The same map as k_transform_b up to rounding (the axes in
+// l % 16 is element i of lane l. The same map as k_transform_cols up to rounding (the axes in
 // another order), and slower than it on the 32-column spheroid (8.5 against 6.7 ms per mult):
 // the pass moves 19 GB (values read, coefficients of the active sub-cones written) and the
 // arithmetic is not what bounds it. Kept for that comparison: it runs only when the

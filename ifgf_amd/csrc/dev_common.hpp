@@ -898,7 +898,7 @@ inline KParams kparams(const DevicePlan& D)
 // which compile-time order set (high / low orders, fine factors 3) matches the plan:
 // 1 = (3,6,6)/(2,3,3), order 6 without a tolerance; 2 = (5,8,8)/(2,5,5), order 8 without a
 // tolerance; 3 = (6,8,7)/(3,5,4), what the tolerance estimate picks for order 6 at tol 1e-5 on
-// the unit sphere at N = 1M, kappa = 100.  0: the runtime-order kernels.
+// the unit sphere at N = 1M, kappa = 100.  0: the kernels of orders.hip.
 inline int order_class(const DevicePlan& D)
 {
     const bool f3 = D.f[0] == 3 && D.f[1] == 3 && D.f[2] == 3;

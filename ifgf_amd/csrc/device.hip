@@ -7,8 +7,8 @@
 //   level -> scatter.
 // Every kernel is templated on the arithmetic type R (double: the plain form; float: the
 // mixed form, which keeps cone coordinates, phases and box geometry in FP64).  The kernels
-// that evaluate or build fine interpolants are specialised on the interpolation orders of
-// the common configurations (orders 6 and 8), with a runtime-order fallback.
+// that evaluate or build fine interpolants here are specialised on the interpolation orders of
+// the common configurations (orders 6 and 8); those of orders.hip take any orders.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

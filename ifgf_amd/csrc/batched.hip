@@ -389,7 +389,7 @@ template <typename R> bool use_mfma(const DevicePlan& D)
 // results: it reads and writes only the batch buffers, so one captured graph per number of
 // columns serves every call with these buffers
 template <int KIND, typename R, int RB>
-void run_batched_core(DevicePlan& D, hipStream_t st, int nc)
+void run_batched_core(DevicePlan& D, hipStream_t st, int nc, bool few)
 {
     const KParams kp = kparams(D);
     const NodeTabs tabs{D.ho_nodes, D.trig_th, D.trig_ph};
@@ -411,7 +411,7 @@ void run_batched_core(DevicePlan& D, hipStream_t st, int nc)
                     D.near_items, D.n_near_items, D.near_off, D.near_run, D.geo, D.src_pts,
                     D.normals, ws, D.tgt_pts, res, nc, kp);
         },
-        [&](int g, hipStream_t s) { launch_far_cols<R>(D, s, kp, g, F, far_res, nc); });
+        [&](int g, hipStream_t s) { launch_far_cols<R>(D, s, kp, g, F, far_res, nc, few); });
     if (overlap != 1)
         pipe.fork();
     if (D.n_leaf_cones)
@@ -447,7 +447,7 @@ void run_batched_core(DevicePlan& D, hipStream_t st, int nc)
 // columns), scatter
 template <int KIND, typename R, int RB>
 void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, int ncol,
-                 hipStream_t st, int io, bool graph)
+                 hipStream_t st, int io, bool graph, bool few)
 {
     Cx<R>* ws = static_cast<Cx<R>*>(D.b_ws);
     Cx<R>* res = static_cast<Cx<R>*>(D.b_res);
@@ -459,7 +459,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
         w_dev, D.src_perm, ws, D.nsrc, nc, ncol, in_im);
     if (graph)
     {
-        auto& g = D.b_graphs[nc];
+        auto& g = D.b_graphs[few ? -nc : nc];
         if (!g.second)
         {
             // captured on the plan's capture stream (the caller's may be the null stream,
@@ -472,7 +472,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
             }
             hipStream_t cs = static_cast<hipStream_t>(D.cap_stream);
             HIP_OK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-            run_batched_core<KIND, R, RB>(D, cs, nc);
+            run_batched_core<KIND, R, RB>(D, cs, nc, few);
             hipGraph_t gr = nullptr;
             HIP_OK(hipStreamEndCapture(cs, &gr));
             hipGraphExec_t ex = nullptr;
@@ -482,7 +482,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
         HIP_OK(hipGraphLaunch(static_cast<hipGraphExec_t>(g.second), st));
     }
     else
-        run_batched_core<KIND, R, RB>(D, st, nc);
+        run_batched_core<KIND, R, RB>(D, st, nc, few);
     k_scatter_b<R><<<dim3(unsigned((nt + 255) / 256)), dim3(256), 0, st>>>(
         res, res + nt, D.n_far_lvls, D.tgt_perm, out_dev, D.ntgt, nc, ncol, out_re, out_im);
     HIP_OK(hipGetLastError());
@@ -490,55 +490,55 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
 
 template <typename R, int RB>
 void run_kind(DevicePlan& D, const double* w, double* o, int nc, int ncol, hipStream_t st, int io,
-              bool graph)
+              bool graph, bool few)
 {
     switch (D.kind)
     {
     case KIND_HELMHOLTZ:
-        return run_batched<KH, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KH, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     case KIND_MODHELMHOLTZ:
-        return run_batched<KM, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KM, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     case KIND_LAPLACE:
-        return run_batched<KL, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KL, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     case KIND_DOUBLELAYER:
-        return run_batched<KD, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KD, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     case KIND_COMBINED:
-        return run_batched<KC, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KC, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     case KIND_GRAD:
-        return run_batched<KG, R, RB>(D, w, o, nc, ncol, st, io, graph);
+        return run_batched<KG, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
     }
     throw std::runtime_error("unknown kernel kind");
 }
 
 template <typename R>
 void run_width(DevicePlan& D, const double* w, double* o, int ncol, hipStream_t st, int io,
-               bool graph)
+               bool graph, bool few)
 {
     // the MFMA tiles take 8 columns at a time: zero columns fill the last
     int nc = use_mfma<R>(D) ? (ncol + 7) / 8 * 8 : ncol;
     if (nc > D.b_rb)
         nc = ncol;
     if (nc <= 2)
-        return run_kind<R, 2>(D, w, o, nc, ncol, st, io, graph);
+        return run_kind<R, 2>(D, w, o, nc, ncol, st, io, graph, few);
     if (nc <= 4)
-        return run_kind<R, 4>(D, w, o, nc, ncol, st, io, graph);
+        return run_kind<R, 4>(D, w, o, nc, ncol, st, io, graph, few);
     if (nc <= 8)
-        return run_kind<R, 8>(D, w, o, nc, ncol, st, io, graph);
+        return run_kind<R, 8>(D, w, o, nc, ncol, st, io, graph, few);
     if (nc <= 16)
-        return run_kind<R, 16>(D, w, o, nc, ncol, st, io, graph);
-    run_kind<R, 32>(D, w, o, nc, ncol, st, io, graph);
+        return run_kind<R, 16>(D, w, o, nc, ncol, st, io, graph, few);
+    run_kind<R, 32>(D, w, o, nc, ncol, st, io, graph, few);
 }
 } // namespace
 
 void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int ncol, void* stream,
-                  int io, bool graph)
+                  int io, bool graph, bool few)
 {
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (ncol < 1 || ncol > D.b_rb || ncol > MAX_COLUMNS)
         throw std::runtime_error("mult_batched: column count or buffers");
     if (D.prec == PREC_FP64)
-        run_width<double>(D, w_dev, out_dev, ncol, st, io, graph);
+        run_width<double>(D, w_dev, out_dev, ncol, st, io, graph, few);
     else
-        run_width<float>(D, w_dev, out_dev, ncol, st, io, graph);
+        run_width<float>(D, w_dev, out_dev, ncol, st, io, graph, few);
 }
 } // namespace ifgf

@@ -25,7 +25,9 @@ using namespace dev;
 // times the transfer factors to part (a node is in one group of a child), so that one copy of the
 // node values in LDS serves all eight.
 template <typename R, int O0, int O1>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 12 ? 4 : (O0 * O1 <= 18 ? 3 : 2)) : 2))) void k_up_cols(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 12 ? 4 : (O0 * O1 <= 18 ? 3 : 2)) : 2)))
+void k_up_cols(
     const UpDesc* __restrict__ desc, const CellRef* __restrict__ ctab,
     const UpGrpOf<R>* __restrict__ grp, const Cx<R>* __restrict__ F, Cx<R>* __restrict__ V, int nc,
     int cw, int nch, KParams kp)
@@ -256,7 +258,9 @@ template <typename R> constexpr int FAR_CHUNK = sizeof(R) == 4 ? 24 : 12;
 // cones of its targets (neighbours in Morton order, mostly one or two) one after another, each
 // cone's coefficients read once, a chunk at a time, for all the run's targets in it.
 template <typename R, int O0, int O1, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 3 : 2))) void k_far_cols(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 3 : 2)))
+void k_far_cols(
     const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const Cx<R>* __restrict__ F,
@@ -493,15 +497,210 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
 }
 typedef float mf4 __attribute__((ext_vector_type(4)));
 
+// Far field from the pair records for NC of the nc columns (blockIdx.y picks which), any orders: a
+// workgroup per item, its waves sharing the item's sources; lanes = (target, run of sources) as in
+// k_far_rec.  Per step the wave copies its lanes' distinct cones (up to most at a time, the NC
+// columns' coefficients next to one another) to LDS and each lane adds coefficient times
+// Chebyshev product for its target, one product for the columns.  Bound by the LDS reads (8 NC
+// bytes per lane and coefficient).  Whole mult of 3 and 5 columns, with the kernels that evaluate
+// 16 columns at a time -> with this one: 8.0 -> 4.1 and 9.1 -> 5.3 ms at (2,3,3), 262,144 points;
+// 6.8 -> 3.3 and 7.7 -> 4.8 at (3,5,4), 100,000 points; FP64 at (3,5,4), 50,000 points, 6.9 -> 4.9
+// and 10.3 -> 8.3.  NC of 8 and 16 instead (fewer groups, more registers and LDS per wave): 12
+// columns 12.4 and 17.9 ms against 11.9.
+template <typename R, int O0, int NC>
+__global__ __launch_bounds__(512)
+void k_far_rec_cols(const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
+                    const int64_t* __restrict__ rec_off, const FarRec<R>* __restrict__ rec,
+                    const Cx<R>* __restrict__ cfs, const Cx<R>* __restrict__ F, int nc, int most,
+                    int stride, int64_t ntgt, Cx<R>* __restrict__ far_res, KParams kp)
+{
+    extern __shared__ __align__(16) unsigned char far_smem[];
+    const int lane = int(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wpb = int(blockDim.x >> 6);
+    Cx<R>* sm = reinterpret_cast<Cx<R>*>(far_smem);
+    Cx<R>* sc = sm + wave * most * stride;
+    const int64_t it = xcd_block(kp.xlg);
+    const int c0 = int(blockIdx.y) * NC, ncg = min(NC, nc - c0);
+    const WorkItem wi = items[it];
+    const int Tp = pow2_at_least(wi.count);
+    const int ti = lane & (Tp - 1);
+    const int grp = lane / Tp, ngrp = 64 / Tp;
+    const bool valid = ti < wi.count;
+    const int32_t n = srange[2 * it + 1] - srange[2 * it];
+    const int32_t ja = n * wave / wpb, jb = n * (wave + 1) / wpb;
+    const FarRec<R>* rp = rec + rec_off[it] + ti;
+    const Cx<R>* cp = cfs + rec_off[it] + ti;
+    constexpr int ROWS = 64 / NC; // rows of NC columns the wave copies at a time
+    const int n_lo = kp.n_lo;
+    const int col = lane % NC, row0 = lane < ROWS * NC ? lane / NC : 4 * n_lo;
+    Cx<R> acc[NC];
+#pragma unroll
+    for (int r = 0; r < NC; r++)
+        acc[r] = {R(0), R(0)};
+    int qs = -1;
+    R q0 = R(0), q1 = R(0), q2 = R(0);
+    Cx<R> cf = {R(0), R(0)};
+    auto fetch = [&](int32_t j)
+    {
+        qs = -1;
+        if (valid && j + grp < jb)
+        {
+            const int64_t e = int64_t(j + grp) * wi.count;
+            const FarRec<R> q = rp[e];
+            qs = q.slot;
+            q0 = q.x0;
+            q1 = q.x1;
+            q2 = q.x2;
+            cf = cp[e];
+        }
+    };
+    fetch(ja);
+    for (int32_t j = ja; j < jb; j += ngrp)
+    {
+        const int fine = qs;
+        const R x0 = q0, x1 = q1, x2 = q2;
+        const Cx<R> cc = cf;
+        fetch(j + ngrp);
+        uint64_t rem = __ballot(fine >= 0);
+        while (rem != 0)
+        {
+            int my = -1, nd = 0;
+            int cs0 = 0, cs1 = 0, cs2 = 0, cs3 = 0;
+#pragma unroll 1
+            while (rem != 0 && nd < most)
+            {
+                const int f0 = __builtin_amdgcn_readlane(fine, __ffsll((unsigned long long)rem) - 1);
+                const uint64_t m = __ballot(fine == f0);
+                if (fine == f0)
+                    my = nd;
+                cs0 = nd == 0 ? f0 : cs0;
+                cs1 = nd == 1 ? f0 : cs1;
+                cs2 = nd == 2 ? f0 : cs2;
+                cs3 = nd == 3 ? f0 : cs3;
+                rem &= ~m;
+                nd++;
+            }
+            // the staging writes stay behind the reads of the step before
+            asm volatile("" ::: "memory");
+#pragma unroll 4
+            for (int k = row0; k < nd * n_lo; k += ROWS)
+            {
+                const int d = (k >= n_lo) + (k >= 2 * n_lo) + (k >= 3 * n_lo);
+                const int f0 = d == 0 ? cs0 : (d == 1 ? cs1 : (d == 2 ? cs2 : cs3));
+                const int i = k - d * n_lo;
+                Cx<R> v = {R(0), R(0)};
+                if (col < ncg)
+                    v = F[(int64_t(f0) * n_lo + i) * nc + c0 + col];
+                sc[d * stride + i * NC + col] = v;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (my >= 0)
+            {
+                const Cx<R>* l = sc + my * stride;
+                Cx<R> p[NC];
+#pragma unroll
+                for (int r = 0; r < NC; r++)
+                    p[r] = {R(0), R(0)};
+                auto add = [&](R w)
+                {
+#pragma unroll
+                    for (int r = 0; r < NC; r++)
+                    {
+                        const Cx<R> b = l[r];
+                        p[r].x = fma_r(w, b.x, p[r].x);
+                        p[r].y = fma_r(w, b.y, p[r].y);
+                    }
+                    l += NC;
+                };
+                // T_k T_j T_i from the recurrences of the three axes, each started from T_0 = 1
+                // and T_-1 = x, the inner ones scaled by the outer's value
+                R a2 = R(1), b2 = x2;
+#pragma unroll 1
+                for (int i2 = 0; i2 < kp.lo2; i2++)
+                {
+                    R a1 = a2, b1 = a2 * x1;
+#pragma unroll 1
+                    for (int i1 = 0; i1 < kp.lo1; i1++)
+                    {
+                        R a0 = a1, b0 = a1 * x0;
+                        auto term = [&]()
+                        {
+                            add(a0);
+                            const R t = fma_r(R(2) * x0, a0, -b0);
+                            b0 = a0;
+                            a0 = t;
+                        };
+                        if constexpr (O0 > 0)
+                        {
+#pragma unroll
+                            for (int i0 = 0; i0 < O0; i0++)
+                                term();
+                        }
+                        else
+                        {
+#pragma unroll 1
+                            for (int i0 = 0; i0 < kp.lo0; i0++)
+                                term();
+                        }
+                        const R t = fma_r(R(2) * x1, a1, -b1);
+                        b1 = a1;
+                        a1 = t;
+                    }
+                    const R t = fma_r(R(2) * x2, a2, -b2);
+                    b2 = a2;
+                    a2 = t;
+                }
+#pragma unroll
+                for (int r = 0; r < NC; r++)
+                    acc[r] = cadd(acc[r], cmul(p[r], cc));
+            }
+        }
+    }
+    for (int m = Tp; m < 64; m <<= 1)
+    {
+#pragma unroll
+        for (int r = 0; r < NC; r++)
+        {
+            acc[r].x += __shfl_xor(acc[r].x, m, 64);
+            acc[r].y += __shfl_xor(acc[r].y, m, 64);
+        }
+    }
+    if (wpb > 1)
+    {
+        __syncthreads(); // the waves are done with their cones
+#pragma unroll
+        for (int r = 0; r < NC; r++)
+            sm[(wave * NC + r) * 64 + lane] = acc[r];
+        __syncthreads();
+        if (wave)
+            return;
+        for (int w = 1; w < wpb; w++)
+        {
+#pragma unroll
+            for (int r = 0; r < NC; r++)
+                acc[r] = cadd(acc[r], sm[(w * NC + r) * 64 + lane]);
+        }
+    }
+    if (grp == 0 && valid)
+    {
+        Cx<R>* res = far_res + (wi.pad * ntgt + wi.first + ti) * nc + c0;
+#pragma unroll
+        for (int r = 0; r < NC; r++)
+            if (r < ncg)
+                res[r] = cadd(res[r], acc[r]);
+    }
+}
+
 // Far field for nc columns on the FP32 matrix cores (mixed form, any orders): per source box the
 // item's targets are sums over a fine cone's n_lo coefficients, the same cone for many of them, so
 // a block of 16 targets x 16 real columns is a product basis (16 x n_lo) times coefficients (n_lo x
 // 16) on v_mfma_f32_16x16x4f32.  Four waves; per step of nbox source boxes a wave locates the
 // item's targets in one box (or reads their records) and writes the products of their Chebyshev
-// values to LDS (ks floats per target).  Then each wave takes one tile of 16 columns and its share of the four blocks of
-// targets, and goes through the distinct cones of each box (2 to 3 for 64 targets), 32 coefficients
-// at a time: the next chunk's (or cone's, or box's) coefficients are loaded while the current
-// ones are multiplied into every block that has targets in the cone, rows of other targets zeroed.
+// values to LDS (ks floats per target).  Then each wave takes one tile of 16 columns and its share
+// of the four blocks of targets, and goes through the distinct cones of each box (2 to 3 for 64
+// targets), 32 coefficients at a time: the next chunk's (or cone's, or box's) coefficients are
+// loaded while the current ones are multiplied into every block that has targets in the cone,
+// rows of other targets zeroed.
 // The sums of a box times the centre factors are added up in registers.
 // Lane l: g = l / 16, n = l % 16; A[row n], B[column n] at coefficient 8 c + 2 g + s in step s of
 // chunk c (one 8-byte LDS read gives A for two steps), C[row 4 g + i][column n] in element i;
@@ -509,7 +708,9 @@ typedef float mf4 __attribute__((ext_vector_type(4)));
 // Bound by the waits for coefficients and LDS, not by the matrix rate: 32 columns, 262,144 points,
 // (2,3,3), far phase 27 -> 11.9 ms (16.2 ms with
 // k_far_cols); 5 columns, 49,999 points, (3,3,3): 2.6 -> 1.65 ms against k_far_cols.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_far_mfma(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(4)))
+void k_far_mfma(
     const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const float* __restrict__ F,
@@ -834,10 +1035,67 @@ void launch_transform_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int
         c0, xsz, D.cones, V, F, static_cast<const R*>(D.wmat), nc, cw, nch, kp);
 }
 
+// k_far_rec_cols for a call of at most FEW_COLUMNS columns, where the plan has pair records and a
+// cone's coefficients for five columns fit the LDS; false otherwise
+template <typename R>
+static bool launch_far_rec_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
+                                const Cx<R>* F, Cx<R>* far_res, int nc)
+{
+    constexpr size_t CX = sizeof(Cx<R>);
+    if (!D.far_rec || (size_t(D.n_lo) * 5 + 2) * CX > size_t(64) * 1024)
+        return false;
+    const DevicePlan::FarGroup& G = D.far_steps[step];
+    const int64_t n = G.item1 - G.item0;
+    // waves per item: as many for every number of columns, so that a column's sum does not depend
+    // on the others; at most 128 KB of LDS
+    int w = far_split(n);
+    while (w > 1 && std::max<size_t>(12 * 1024, (size_t(D.n_lo) * 5 + 2) * CX) * w > 128 * 1024)
+        w /= 2;
+    // groups of at most five columns, as equal as they go
+    const int gy = (nc + 4) / 5;
+    auto go = [&](auto o0, auto ncc)
+    {
+        constexpr int O0 = decltype(o0)::value, NC = decltype(ncc)::value;
+        // 16-byte words, an odd number of them, so that the cones start in different banks
+        const int stride = sizeof(R) == 4 ? (((D.n_lo * NC + 1) / 2) | 1) * 2 : (D.n_lo * NC) | 1;
+        const size_t cone = size_t(stride) * CX;
+        const int most = int(std::min<size_t>(4, std::max<size_t>(1, size_t(12) * 1024 / cone)));
+        const size_t lds = std::max(cone * most * w, w > 1 ? size_t(w) * 64 * NC * CX : 0);
+        if (lds > size_t(64) * 1024)
+            HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_far_rec_cols<R, O0, NC>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        k_far_rec_cols<R, O0, NC><<<dim3(unsigned(n), unsigned(gy)), dim3(64 * w), lds, st>>>(
+            D.far_items + G.item0, D.far_srange + 2 * G.item0, D.far_rec_off + G.item0,
+            static_cast<const FarRec<R>*>(D.far_rec), static_cast<const Cx<R>*>(D.far_cf), F, nc,
+            most, stride, D.ntgt, far_res, kp);
+    };
+    auto cols = [&](auto o0)
+    {
+        switch ((nc + gy - 1) / gy)
+        {
+        case 5: go(o0, std::integral_constant<int, 5>()); break;
+        case 4: go(o0, std::integral_constant<int, 4>()); break;
+        default: go(o0, std::integral_constant<int, 3>()); break;
+        }
+    };
+    switch (D.lo[0])
+    {
+    case 1: cols(std::integral_constant<int, 1>()); break;
+    case 2: cols(std::integral_constant<int, 2>()); break;
+    case 3: cols(std::integral_constant<int, 3>()); break;
+    case 4: cols(std::integral_constant<int, 4>()); break;
+    case 5: cols(std::integral_constant<int, 5>()); break;
+    default: cols(std::integral_constant<int, 0>()); break;
+    }
+    return true;
+}
+
 template <typename R>
 void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step, const Cx<R>* F,
-                     Cx<R>* far_res, int nc)
+                     Cx<R>* far_res, int nc, bool few)
 {
+    if (few && launch_far_rec_cols<R>(D, st, kp, step, F, far_res, nc))
+        return;
     const DevicePlan::FarGroup& G = D.far_steps[step];
     const int64_t n = G.item1 - G.item0;
     const WorkItem* items = D.far_items + G.item0;
@@ -896,7 +1154,7 @@ void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
     template void launch_transform_cols<R>(DevicePlan&, hipStream_t, const KParams&, int64_t,   \
                                            int64_t, const Cx<R>*, Cx<R>*, int);                 \
     template void launch_far_cols<R>(DevicePlan&, hipStream_t, const KParams&, int,             \
-                                     const Cx<R>*, Cx<R>*, int);
+                                     const Cx<R>*, Cx<R>*, int, bool);
 IFGF_COLS(float)
 IFGF_COLS(double)
 #undef IFGF_COLS

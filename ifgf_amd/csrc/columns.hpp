@@ -21,6 +21,6 @@ void launch_transform_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int
 // far launch `step` (of far_steps): added to the far results of its targets' levels
 template <typename R>
 void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step, const Cx<R>* F,
-                     Cx<R>* far_res, int nc);
+                     Cx<R>* far_res, int nc, bool few);
 } // namespace dev
 } // namespace ifgf

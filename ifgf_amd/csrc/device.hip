@@ -1489,7 +1489,8 @@ void device_free(DevicePlan& D)
                     D.src_end, D.child, D.geo, D.cones, D.ctab, D.ho_nodes, D.trig_th,
                     D.trig_ph, D.fine_ang, D.wmat, D.up_grp, D.up_tl_desc, D.tr_list,
                     D.leaf_cones, D.leaf_boxes, D.up_cones, D.far_srange, D.far_src,
-                    D.near_off, D.near_run, D.near_pts, D.far_items, D.near_items, D.wsorted, D.result, D.far_res, D.far_rec_off, D.far_rec, D.far_cf, D.V,
+                    D.near_off, D.near_run, D.near_pts, D.far_items, D.near_items, D.wsorted,
+                    D.result, D.far_res, D.far_rec_off, D.far_rec, D.far_cf, D.V,
                     D.F, D.F_bank[0], D.F_bank[1], D.b_ws, D.b_res, D.b_V, D.b_F, D.b_in,
                     D.b_out, D.h_in, D.h_out};
     for (void* p : ptrs)
@@ -2186,9 +2187,8 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
             }
         }
         // several columns: the batched pipeline, in as few equal passes as the shape's most
-        // columns per pass and the device memory allow.  Two columns are faster one by one (mixed
-        // form, 262,144 points order 6: 5.4 against 8.0 ms; FP64, 50,000 points: 6.5 against 6.6),
-        // three about even (8.1 against 8.6 ms; 20,000 points: 1.16 against 1.00)
+        // columns per pass and the device memory allow.  At 262,144 points, order 6: one column 1.7
+        // ms, three together 4.1; two go one by one
         if (nrhs >= 3 && !D.ring && std::getenv("IFGF_NO_BATCH") == nullptr)
         {
             auto equal = [&](int most)
@@ -2204,6 +2204,8 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                 rb = have >= 2 ? equal(have) : 0;
             if (rb >= 2)
             {
+                // by the columns of the call, not of a pass: results do not depend on the passes
+                const bool few = nrhs <= FEW_COLUMNS;
                 for (int64_t c = 0; c < nrhs; c += rb)
                 {
                     const int ncol = int(std::min<int64_t>(rb, nrhs - c));
@@ -2211,12 +2213,12 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                     double* oc = static_cast<double*>(out) + 2 * c * D.ntgt;
                     if (device_ptrs)
                     {
-                        mult_batched(D, wc, oc, ncol, st, io, graph && !timed);
+                        mult_batched(D, wc, oc, ncol, st, io, graph && !timed, few);
                         continue;
                     }
                     HIP_OK(hipMemcpyAsync(D.b_in, wc, 16 * size_t(ncol) * size_t(D.nsrc),
                                           hipMemcpyHostToDevice, st));
-                    mult_batched(D, D.b_in, D.b_out, ncol, st, io, graph && !timed);
+                    mult_batched(D, D.b_in, D.b_out, ncol, st, io, graph && !timed, few);
                     HIP_OK(hipMemcpyAsync(oc, D.b_out, 16 * size_t(ncol) * size_t(D.ntgt),
                                           hipMemcpyDeviceToHost, st));
                 }

@@ -220,7 +220,8 @@ struct DevicePlan
 
     // the single-column mult's core captured as a graph (on first use with graphs enabled),
     // and the batched mult's core for the current batch buffers, per number of columns (at most
-    // MAX_COLUMNS of them): hipGraph_t, hipGraphExec_t
+    // MAX_COLUMNS of them; as -columns those of calls of at most FEW_COLUMNS columns):
+    // hipGraph_t, hipGraphExec_t
     void* graph = nullptr;
     void* graph_exec = nullptr;
     std::map<int, std::pair<void*, void*>> b_graphs;
@@ -258,8 +259,14 @@ void device_free(DevicePlan& D);
 int64_t device_transform_cones(const DevicePlan& D);
 // batched mult (batched.hip): ncol <= b_rb columns of device densities
 constexpr int MAX_COLUMNS = 32;
+// calls of at most this many columns take the far field by groups of columns (k_far_rec_cols), the
+// others 16 real columns at a time.  Whole mult of 8, 12 and 16 columns by groups / by tiles:
+// 7.9 / 10.2, 11.9 / 14.6 and 16.4 / 16.1 ms at (2,3,3), 262,144 points; 7.3 / 8.6, 11.5 / 11.6 and
+// 15.0 / 13.3 at (3,5,4), 100,000 points; FP64 at (3,5,4), 50,000 points, 11.6 / 12.3, 17.2 / 17.3
+// and 21.8 / 19.9.
+constexpr int FEW_COLUMNS = 12;
 void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int ncol, void* stream,
-                  int io, bool graph = false);
+                  int io, bool graph, bool few);
 // w: complex128 (host or device), out: complex128 (host or device); nrhs columns of length
 // N / M stored one after another.  io: IO_* bits applied while the densities are gathered and
 // the results scattered (conjugations and a sign, for adjoint products).

@@ -32,7 +32,9 @@ using namespace dev;
 // chunk was read ahead past the last one; at (2,3,3) and (2,5,5) within 2% of k_up_grp without
 // its transform.
 template <typename R, int O0, int O1, bool SEQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 20 ? 4 : 3) : 2))) void k_up_rows(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 20 ? 4 : 3) : 2)))
+void k_up_rows(
     const UpDesc* __restrict__ desc, int64_t n, int K, const CellRef* __restrict__ ctab,
     const UpGrpOf<R>* __restrict__ grp, const Cx<R>* __restrict__ F, Cx<R>* __restrict__ V,
     KParams kp)
@@ -202,7 +204,9 @@ __device__ __forceinline__ void stage_cones(const Cx<R>* __restrict__ F, int c0,
 // (5,5,5), combined field on a torus, 131,072 points; with a read-ahead in two buffers instead
 // 27 registers spilled at (2,5,*).
 template <typename R, int O0, int O1, bool FAST>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : (O0 * O1 > 24 ? 1 : 2)))) void k_far_rows(
+__global__ __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : (O0 * O1 > 24 ? 1 : 2))))
+void k_far_rows(
     const WorkItem* __restrict__ items, int64_t nitems, const int32_t* __restrict__ srange,
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
     const CellRef* __restrict__ ctab, const Cx<R>* __restrict__ F,
@@ -457,7 +461,9 @@ __global__ __launch_bounds__(64) void k_far_record(
 // at (3,6,4), 1M points; 3.7 -> 2.4 ms at (2,3,3), 1M points; FP64 at (3,5,4), 99,991 points,
 // 1.6 -> 0.63 ms.
 template <typename R, int O0, int O1>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 9 ? 7 : 5) : 3))) void k_far_rec(
+__global__ __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? (O0 * O1 <= 9 ? 7 : 5) : 3)))
+void k_far_rec(
     const WorkItem* __restrict__ items, int64_t nitems, const int32_t* __restrict__ srange,
     const int64_t* __restrict__ rec_off, const FarRec<R>* __restrict__ rec,
     const Cx<R>* __restrict__ cfs, const Cx<R>* __restrict__ F, int stage, int stride, int split,

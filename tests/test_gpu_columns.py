@@ -1,6 +1,6 @@
 """Several density columns in one pass against the same columns one by one, where the kernels of
-columns.hip change form: numbers of columns at the edges of the 16-wide column tiles and of the
-register instances, few and many fine coefficients (source boxes per step, products too large
+columns.hip change form: numbers of columns at the edges of the groups of up to five columns, of
+the 16-wide column tiles and of the register instances, few and many fine coefficients (source boxes per step, products too large
 for LDS), fine factor 1, targets other than the sources, passes of unequal width."""
 import os
 
@@ -29,7 +29,7 @@ def _check(op, W, prec):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
-@pytest.mark.parametrize("ncol", [3, 4, 5, 8, 9, 16, 17, 25, 32, 33])
+@pytest.mark.parametrize("ncol", [3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 16, 17, 25, 32, 33])
 def test_numbers_of_columns(gpu, ncol, prec):
     x, y = spheroid(3000, 81), sphere(1111, 82) * 1.5
     W = np.stack([cdens(3000, 200 + c) for c in range(ncol)], axis=1)
@@ -47,13 +47,14 @@ def test_numbers_of_columns(gpu, ncol, prec):
     ("modhelmholtz", 13, 900),  # 700, no compiled first order, fine factor 1
     ("modhelmholtz", 8, 2500),
 ])
-def test_orders_of_columns(gpu, kind, order, n, prec):
+@pytest.mark.parametrize("ncol", [6, 13])  # far field by groups of columns, by 16-wide tiles
+def test_orders_of_columns(gpu, kind, order, n, prec, ncol):
     x = spheroid(n, 83)
     if kind == "laplace":
         op = ifgf_amd.LaplaceIfgfOperator(20, order, 1, -1, precision=prec)
-        W = np.stack([cdens(n, 300 + c).real for c in range(6)], axis=1)
+        W = np.stack([cdens(n, 300 + c).real for c in range(ncol)], axis=1)
     else:
         op = ifgf_amd.MofifiedHelmholtzIfgfOperator(0.5 - 6.0j, 20, order, 1, -1, precision=prec)
-        W = np.stack([cdens(n, 300 + c) for c in range(6)], axis=1)
+        W = np.stack([cdens(n, 300 + c) for c in range(ncol)], axis=1)
     op.init(x.T, x.T)
     _check(op, W, prec)

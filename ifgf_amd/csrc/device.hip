@@ -2113,13 +2113,36 @@ static size_t batch_bytes(const DevicePlan& D, int rb, bool host_io, size_t n[4]
     return n[0] + n[1] + n[2] + n[3] + (host_io ? 16 * size_t(rb) * size_t(D.nsrc + D.ntgt) : 0);
 }
 
-// Batch buffers for up to want columns; the number of columns they hold (as many as leave half of
-// the free memory and 1 GiB of it; below 2: none).  Buffers that hold enough are kept.
+// Columns that batch buffers may hold of `want` with avail bytes of device memory free: as many as
+// take at most half of them less 1 GiB; below 2: none
+static int batch_columns(const DevicePlan& D, int want, bool host_io, size_t avail)
+{
+    size_t n[4];
+    int rb = want;
+    while (rb >= 2 && 2 * batch_bytes(D, rb, host_io, n) + (size_t(2) << 30) > avail)
+        rb = rb > 8 ? (rb + 1) / 2 : rb - 1;
+    return rb < 2 ? 0 : rb;
+}
+
+// Batch buffers for up to want columns; the number of columns they hold (batch_columns).  Buffers
+// that hold enough are kept, and so are those that hold as many as the memory allowed when as
+// many columns were asked for before: captured graphs go with the buffers, and memory that
+// others have taken since must not narrow them.  They are laid down again once the memory allows
+// twice the columns, or all of them.
 static int ensure_batch(DevicePlan& D, int want, bool host_io)
 {
     if (D.b_rb >= want && (!host_io || D.b_in))
         return want;
-    want = std::max(want, D.b_rb);
+    const bool asked = want <= D.b_asked && (!host_io || D.b_asked_host);
+    D.b_asked = want = std::max(want, D.b_asked);
+    D.b_asked_host = host_io = host_io || D.b_asked_host;
+    const int have = !host_io || D.b_in ? D.b_rb : 0;
+    size_t free_b = 0, total_b = 0, n[4];
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
+        return have;
+    const int rb = batch_columns(D, want, host_io, free_b + size_t(D.b_bytes));
+    if (have > 0 ? rb <= have || (asked && rb < std::min(want, 2 * have)) : rb < 2)
+        return have;
     drop_batch_graphs(D); // captured graphs hold the old buffers
     for (void* p : {D.b_ws, D.b_res, D.b_V, D.b_F, static_cast<void*>(D.b_in),
                     static_cast<void*>(D.b_out)})
@@ -2129,14 +2152,6 @@ static int ensure_batch(DevicePlan& D, int want, bool host_io)
     D.b_in = D.b_out = nullptr;
     D.b_rb = 0;
     D.b_bytes = 0;
-    size_t free_b = 0, total_b = 0, n[4];
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
-        return 0;
-    int rb = want;
-    while (rb >= 2 && 2 * batch_bytes(D, rb, host_io, n) + (size_t(2) << 30) > free_b)
-        rb = rb > 8 ? (rb + 1) / 2 : rb - 1;
-    if (rb < 2)
-        return 0;
     const size_t need = batch_bytes(D, rb, host_io, n);
     HIP_OK(hipMalloc(&D.b_ws, n[0]));
     HIP_OK(hipMalloc(&D.b_res, n[1]));

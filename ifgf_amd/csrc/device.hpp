@@ -248,6 +248,10 @@ struct DevicePlan
     void *b_ws = nullptr, *b_res = nullptr, *b_V = nullptr, *b_F = nullptr;
     double *b_in = nullptr, *b_out = nullptr;
     int64_t b_bytes = 0;
+    // the most columns asked for so far, and whether with host densities: memory may have allowed
+    // fewer (ensure_batch)
+    int b_asked = 0;
+    bool b_asked_host = false;
 };
 
 // ring: 0 = every level resident when it fits the device memory, else level storage;

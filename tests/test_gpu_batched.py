@@ -428,3 +428,41 @@ def test_configuration3_one_operator(gpu):
     d = rel(res["mixed"], res["fp64"])
     print(f"configuration 3 one operator: mixed vs fp64 {d:.2e}", flush=True)
     assert d < 2e-5
+
+
+def test_batch_buffers_that_memory_narrowed_stay(gpu):
+    """32 columns where the free memory holds buffers for 16: two passes with the results of one.
+    A second such call keeps its buffers, also when others have taken most of the memory left, and
+    with the memory given back a call widens them."""
+    import torch
+    GiB = 1 << 30
+    x = spheroid(50000, 210)
+    W = torch.as_tensor(np.stack([cdens(50000, 211 + i) for i in range(32)], 1), device="cuda:0")
+    free = lambda: (torch.cuda.synchronize(), torch.cuda.empty_cache(),
+                    torch.cuda.mem_get_info()[0])[2]
+
+    def take(left):
+        return torch.empty(free() - left, dtype=torch.uint8, device="cuda:0")
+
+    def mult(op):
+        f = free()
+        u = op.mult(W).cpu()
+        return u, f - free()
+
+    wide, narrow = (ifgf_amd.HelmholtzIfgfOperator(20.0, 64, 6, 1, -1) for _ in range(2))
+    wide.init(x.T, x.T)
+    U, need = mult(wide)
+    print(f"batch buffers of 32 columns: {need / GiB:.2f} GiB", flush=True)
+    assert need > GiB
+    del wide
+    narrow.init(x.T, x.T)
+    filler = take(2 * GiB + 3 * need // 2)
+    u, got = mult(narrow)
+    print(f"narrowed: {got / GiB:.2f} GiB", flush=True)
+    assert need // 4 < got < 3 * need // 4 and torch.equal(u, U)
+    more = take(2 * GiB + need // 4)
+    u, got = mult(narrow)
+    assert abs(got) < GiB // 4 and torch.equal(u, U), got / GiB
+    del filler, more
+    u, got = mult(narrow)
+    assert got > need // 4 and torch.equal(u, U)

@@ -10,7 +10,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <cstdint>
 #include <stdexcept>
 #include <vector>
@@ -275,7 +274,7 @@ __device__ __forceinline__ void lds_fence()
 // another order), and slower than it on the 32-column spheroid (8.5 against 6.7 ms per mult):
 // the pass moves 19 GB (values read, coefficients of the active sub-cones written) and the
 // arithmetic is not what bounds it. Kept for that comparison: it runs only when the
-// environment variable IFGF_TRANSFORM_MFMA is set when a batched pass is enqueued or captured.
+// environment variable IFGF_TRANSFORM_MFMA is set at the call (device_mult).
 __global__ __launch_bounds__(64) void k_transform_mf(int64_t c0, int64_t c1, int NC,
                                                      const ConeDev* __restrict__ cones,
                                                      const float* __restrict__ V,
@@ -379,17 +378,11 @@ __global__ __launch_bounds__(64) void k_transform_mf(int64_t c0, int64_t c1, int
     }
 }
 
-// the transform on MFMA tiles was asked for and the orders and form have it
-template <typename R> bool use_mfma(const DevicePlan& D)
-{
-    return sizeof(R) == 4 && order_class(D) == 1 && std::getenv("IFGF_TRANSFORM_MFMA") != nullptr;
-}
-
 // everything of a batched mult between the gather of the densities and the scatter of the
 // results: it reads and writes only the batch buffers, so one captured graph per number of
-// columns serves every call with these buffers
+// columns and form (few, tiles) serves every call with these buffers
 template <int KIND, typename R, int RB>
-void run_batched_core(DevicePlan& D, hipStream_t st, int nc, bool few)
+void run_batched_core(DevicePlan& D, hipStream_t st, int nc, bool few, bool tiles)
 {
     const KParams kp = kparams(D);
     const NodeTabs tabs{D.ho_nodes, D.trig_th, D.trig_ph};
@@ -426,7 +419,7 @@ void run_batched_core(DevicePlan& D, hipStream_t st, int nc, bool few)
         {
             bool done = false;
             if constexpr (sizeof(R) == 4)
-                if (use_mfma<R>(D) && nc % 8 == 0)
+                if (tiles && nc % 8 == 0)
                 {
                     k_transform_mf<<<dim3(unsigned((c1 - c0) * (nc / 8))), dim3(64), 0, st>>>(
                         c0, c1, 2 * nc, D.cones, reinterpret_cast<const float*>(V),
@@ -444,10 +437,10 @@ void run_batched_core(DevicePlan& D, hipStream_t st, int nc, bool few)
 }
 
 // one batched mult: gather, the core (eagerly, or as the captured graph of this number of
-// columns), scatter
+// columns and form), scatter
 template <int KIND, typename R, int RB>
 void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, int ncol,
-                 hipStream_t st, int io, bool graph, bool few)
+                 hipStream_t st, int io, bool graph, bool few, bool tiles)
 {
     Cx<R>* ws = static_cast<Cx<R>*>(D.b_ws);
     Cx<R>* res = static_cast<Cx<R>*>(D.b_res);
@@ -459,7 +452,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
         w_dev, D.src_perm, ws, D.nsrc, nc, ncol, in_im);
     if (graph)
     {
-        auto& g = D.b_graphs[few ? -nc : nc];
+        auto& g = D.b_graphs[nc | (few ? 64 : 0) | (tiles ? 128 : 0)]; // nc <= 32
         if (!g.second)
         {
             // captured on the plan's capture stream (the caller's may be the null stream,
@@ -472,7 +465,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
             }
             hipStream_t cs = static_cast<hipStream_t>(D.cap_stream);
             HIP_OK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-            run_batched_core<KIND, R, RB>(D, cs, nc, few);
+            run_batched_core<KIND, R, RB>(D, cs, nc, few, tiles);
             hipGraph_t gr = nullptr;
             HIP_OK(hipStreamEndCapture(cs, &gr));
             hipGraphExec_t ex = nullptr;
@@ -482,7 +475,7 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
         HIP_OK(hipGraphLaunch(static_cast<hipGraphExec_t>(g.second), st));
     }
     else
-        run_batched_core<KIND, R, RB>(D, st, nc, few);
+        run_batched_core<KIND, R, RB>(D, st, nc, few, tiles);
     k_scatter_b<R><<<dim3(unsigned((nt + 255) / 256)), dim3(256), 0, st>>>(
         res, res + nt, D.n_far_lvls, D.tgt_perm, out_dev, D.ntgt, nc, ncol, out_re, out_im);
     HIP_OK(hipGetLastError());
@@ -490,55 +483,55 @@ void run_batched(DevicePlan& D, const double* w_dev, double* out_dev, int nc, in
 
 template <typename R, int RB>
 void run_kind(DevicePlan& D, const double* w, double* o, int nc, int ncol, hipStream_t st, int io,
-              bool graph, bool few)
+              bool graph, bool few, bool tiles)
 {
     switch (D.kind)
     {
     case KIND_HELMHOLTZ:
-        return run_batched<KH, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KH, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     case KIND_MODHELMHOLTZ:
-        return run_batched<KM, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KM, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     case KIND_LAPLACE:
-        return run_batched<KL, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KL, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     case KIND_DOUBLELAYER:
-        return run_batched<KD, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KD, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     case KIND_COMBINED:
-        return run_batched<KC, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KC, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     case KIND_GRAD:
-        return run_batched<KG, R, RB>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_batched<KG, R, RB>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     }
     throw std::runtime_error("unknown kernel kind");
 }
 
 template <typename R>
 void run_width(DevicePlan& D, const double* w, double* o, int ncol, hipStream_t st, int io,
-               bool graph, bool few)
+               bool graph, bool few, bool tiles)
 {
     // the MFMA tiles take 8 columns at a time: zero columns fill the last
-    int nc = use_mfma<R>(D) ? (ncol + 7) / 8 * 8 : ncol;
+    int nc = tiles ? (ncol + 7) / 8 * 8 : ncol;
     if (nc > D.b_rb)
         nc = ncol;
     if (nc <= 2)
-        return run_kind<R, 2>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_kind<R, 2>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     if (nc <= 4)
-        return run_kind<R, 4>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_kind<R, 4>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     if (nc <= 8)
-        return run_kind<R, 8>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_kind<R, 8>(D, w, o, nc, ncol, st, io, graph, few, tiles);
     if (nc <= 16)
-        return run_kind<R, 16>(D, w, o, nc, ncol, st, io, graph, few);
-    run_kind<R, 32>(D, w, o, nc, ncol, st, io, graph, few);
+        return run_kind<R, 16>(D, w, o, nc, ncol, st, io, graph, few, tiles);
+    run_kind<R, 32>(D, w, o, nc, ncol, st, io, graph, few, tiles);
 }
 } // namespace
 
 void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int ncol, void* stream,
-                  int io, bool graph, bool few)
+                  int io, bool graph, bool few, bool tiles)
 {
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (ncol < 1 || ncol > D.b_rb || ncol > MAX_COLUMNS)
         throw std::runtime_error("mult_batched: column count or buffers");
     if (D.prec == PREC_FP64)
-        run_width<double>(D, w_dev, out_dev, ncol, st, io, graph, few);
+        run_width<double>(D, w_dev, out_dev, ncol, st, io, graph, few, tiles);
     else
-        run_width<float>(D, w_dev, out_dev, ncol, st, io, graph, few);
+        run_width<float>(D, w_dev, out_dev, ncol, st, io, graph, few, tiles);
 }
 } // namespace ifgf

@@ -2212,8 +2212,10 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                 return int((nrhs + passes - 1) / passes);
             };
             int rb = equal(D.shape.rb > 0 ? D.shape.rb : MAX_COLUMNS);
-            // (the MFMA transform pads a pass to whole tiles of 8 columns)
-            const bool tiles = std::getenv("IFGF_TRANSFORM_MFMA") != nullptr;
+            // (the MFMA transform, where it was asked for and the orders and form have it, pads a
+            // pass to whole tiles of 8 columns)
+            const bool tiles = D.prec == PREC_MIXED && order_class(D) == 1 &&
+                               std::getenv("IFGF_TRANSFORM_MFMA") != nullptr;
             const int have = ensure_batch(D, tiles ? (rb + 7) / 8 * 8 : rb, !device_ptrs);
             if (have < rb)
                 rb = have >= 2 ? equal(have) : 0;
@@ -2228,12 +2230,12 @@ std::string device_mult(DevicePlan& D, const void* w, void* out, int64_t nrhs, b
                     double* oc = static_cast<double*>(out) + 2 * c * D.ntgt;
                     if (device_ptrs)
                     {
-                        mult_batched(D, wc, oc, ncol, st, io, graph && !timed, few);
+                        mult_batched(D, wc, oc, ncol, st, io, graph && !timed, few, tiles);
                         continue;
                     }
                     HIP_OK(hipMemcpyAsync(D.b_in, wc, 16 * size_t(ncol) * size_t(D.nsrc),
                                           hipMemcpyHostToDevice, st));
-                    mult_batched(D, D.b_in, D.b_out, ncol, st, io, graph && !timed, few);
+                    mult_batched(D, D.b_in, D.b_out, ncol, st, io, graph && !timed, few, tiles);
                     HIP_OK(hipMemcpyAsync(oc, D.b_out, 16 * size_t(ncol) * size_t(D.ntgt),
                                           hipMemcpyDeviceToHost, st));
                 }

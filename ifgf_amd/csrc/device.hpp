@@ -220,8 +220,7 @@ struct DevicePlan
 
     // the single-column mult's core captured as a graph (on first use with graphs enabled),
     // and the batched mult's core for the current batch buffers, per number of columns (at most
-    // MAX_COLUMNS of them; as -columns those of calls of at most FEW_COLUMNS columns):
-    // hipGraph_t, hipGraphExec_t
+    // MAX_COLUMNS) and the forms of mult_batched: hipGraph_t, hipGraphExec_t
     void* graph = nullptr;
     void* graph_exec = nullptr;
     std::map<int, std::pair<void*, void*>> b_graphs;
@@ -269,8 +268,9 @@ constexpr int MAX_COLUMNS = 32;
 // 15.0 / 13.3 at (3,5,4), 100,000 points; FP64 at (3,5,4), 50,000 points, 11.6 / 12.3, 17.2 / 17.3
 // and 21.8 / 19.9.
 constexpr int FEW_COLUMNS = 12;
+// few: of a call of at most FEW_COLUMNS; tiles: the transform on MFMA tiles
 void mult_batched(DevicePlan& D, const double* w_dev, double* out_dev, int ncol, void* stream,
-                  int io, bool graph, bool few);
+                  int io, bool graph, bool few, bool tiles);
 // w: complex128 (host or device), out: complex128 (host or device); nrhs columns of length
 // N / M stored one after another.  io: IO_* bits applied while the densities are gathered and
 // the results scattered (conjugations and a sign, for adjoint products).

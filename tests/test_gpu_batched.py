@@ -466,3 +466,27 @@ def test_batch_buffers_that_memory_narrowed_stay(gpu):
     del filler, more
     u, got = mult(narrow)
     assert got > need // 4 and torch.equal(u, U)
+
+
+def test_graph_replays_follow_the_transform_form(gpu):
+    """Graph replays of 16 columns after the transform's form was changed by its environment
+    variable: each replay equals the eager mult of the form in force, which differs from the
+    other's by rounding."""
+    import torch
+    x = spheroid(6000, 220)
+    W = torch.as_tensor(np.stack([cdens(6000, 221 + i) for i in range(16)], 1), device="cuda:0")
+    op = ifgf_amd.HelmholtzIfgfOperator(9.0, 64, 6, 1, -1)
+    op.init(x.T, x.T)
+    eager = {}
+    try:
+        for graph in (False, True, True):
+            op.use_graph = graph
+            for mfma in (False, True):
+                os.environ.pop("IFGF_TRANSFORM_MFMA", None)
+                if mfma:
+                    os.environ["IFGF_TRANSFORM_MFMA"] = "1"
+                u = op.mult(W).cpu()
+                assert torch.equal(u, eager.setdefault(mfma, u)), (graph, mfma)
+    finally:
+        os.environ.pop("IFGF_TRANSFORM_MFMA", None)
+    assert not torch.equal(eager[False], eager[True])

@@ -31,6 +31,7 @@ struct ifgf_operator
     bool same_points = false;
     bool merged = false; // several geometries (ifgf_merge)
     bool host_plan = false; // octrees and cone marking on the host (IFGF_INIT_HOST_PLAN)
+    bool pair_records = true; // unless IFGF_INIT_NO_PAIR_RECORDS
     ifgf_cutoff_fn cutoff = nullptr;
     void* cutoff_ctx = nullptr;
     // the plan was read from a file and built with a cutOff callback that did not travel:
@@ -128,6 +129,7 @@ extern "C"
             if (cutoff)
                 cb = [cutoff, cutoff_ctx](double d) { return cutoff(d, cutoff_ctx) != 0; };
             op->host_plan = plan_only || (flags & IFGF_INIT_HOST_PLAN) != 0;
+            op->pair_records = (flags & IFGF_INIT_NO_PAIR_RECORDS) == 0;
             std::string e =
                 build_plan(op->plan, srcs, n_src, tgts, n_tgt, normals, op->leaf, op->order,
                            op->n_elem, cb, default_threads(),
@@ -138,7 +140,7 @@ extern "C"
             if (plan_only)
                 return IFGF_OK;
             e = device_upload(op->plan, op->precision, op->dev,
-                              (flags & IFGF_INIT_LEVEL_RING) ? 1 : 0);
+                              (flags & IFGF_INIT_LEVEL_RING) ? 1 : 0, op->pair_records);
             if (!e.empty())
                 return fail(op, IFGF_EINTERNAL, e);
             op->on_device = true;
@@ -217,6 +219,7 @@ extern "C"
             op->same_points = info.same_points != 0;
             op->merged = info.merged != 0;
             op->host_plan = info.host_plan != 0;
+            op->pair_records = (flags & IFGF_INIT_NO_PAIR_RECORDS) == 0;
             op->cutoff = nullptr;
             op->cutoff_ctx = nullptr;
             op->cutoff_lost = info.had_cutoff != 0;
@@ -224,7 +227,7 @@ extern "C"
             if (plan_only)
                 return IFGF_OK;
             e = device_upload(op->plan, op->precision, op->dev,
-                              (flags & IFGF_INIT_LEVEL_RING) ? 1 : 0);
+                              (flags & IFGF_INIT_LEVEL_RING) ? 1 : 0, op->pair_records);
             if (!e.empty())
                 return fail(op, IFGF_EINTERNAL, e);
             op->on_device = true;
@@ -332,6 +335,7 @@ extern "C"
                         cb = [f, ctx](double d) { return f(d, ctx) != 0; };
                     }
                     a->host_plan = op->host_plan;
+                    a->pair_records = op->pair_records;
                     std::string e =
                         build_plan(a->plan, ys.data(), T.n, xs.data(), S.n, nullptr, a->leaf,
                                    a->order, a->n_elem, cb, default_threads(),
@@ -339,7 +343,7 @@ extern "C"
                     if (!e.empty())
                         return fail(op, IFGF_EINTERNAL, "adjoint plan: " + e);
                     a->planned = true;
-                    e = device_upload(a->plan, a->precision, a->dev);
+                    e = device_upload(a->plan, a->precision, a->dev, 0, a->pair_records);
                     if (!e.empty())
                         return fail(op, IFGF_EINTERNAL, "adjoint upload: " + e);
                     a->on_device = true;
@@ -387,6 +391,7 @@ extern "C"
         m->n_elem = o0.n_elem;
         m->precision = o0.precision;
         m->merged = true;
+    m->pair_records = (flags & IFGF_INIT_NO_PAIR_RECORDS) == 0;
         m->same_points = same;
         try
         {
@@ -399,7 +404,7 @@ extern "C"
             m->planned = true;
             if (!plan_only)
             {
-                e = device_upload(m->plan, m->precision, m->dev);
+                e = device_upload(m->plan, m->precision, m->dev, 0, m->pair_records);
                 if (!e.empty())
                 {
                     ops[0]->err = e;

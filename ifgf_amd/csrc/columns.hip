@@ -482,7 +482,7 @@ void k_far_cols(
 #pragma unroll
                 for (int j = 0; j < TM; j++)
                     if ((m >> j) & 1u)
-                        acc[j] = cadd(acc[j], cmul(val[j], s_cf[b][tgt0 + j]));
+                        acc[j] = cmul_add(acc[j], val[j], s_cf[b][tgt0 + j]);
             }
         }
         __syncthreads();
@@ -652,7 +652,7 @@ void k_far_rec_cols(const WorkItem* __restrict__ items, const int32_t* __restric
                 }
 #pragma unroll
                 for (int r = 0; r < NC; r++)
-                    acc[r] = cadd(acc[r], cmul(p[r], cc));
+                    acc[r] = cmul_add(acc[r], p[r], cc);
             }
         }
     }

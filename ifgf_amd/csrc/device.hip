@@ -1518,7 +1518,7 @@ void device_free(DevicePlan& D)
     D = DevicePlan();
 }
 
-std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
+std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring, bool records)
 {
     try
     {
@@ -2077,7 +2077,7 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring)
             const size_t pairs = size_t(roff.back());
             const size_t rs = precision == PREC_FP64 ? sizeof(FarRec<double>) : sizeof(FarRec<float>);
             HIP_OK(hipMemGetInfo(&free_b, &total_b));
-            if (pairs > 0 && (rs + cs) * pairs <= free_b / 4)
+            if (records && pairs > 0 && (rs + cs) * pairs <= free_b / 4)
             {
                 D.far_rec_off = dupload(roff, tot);
                 D.far_rec = dalloc<unsigned char>(rs * pairs, tot);

@@ -254,8 +254,8 @@ struct DevicePlan
 };
 
 // ring: 0 = every level resident when it fits the device memory, else level storage;
-// 1 = level storage (DevicePlan::ring)
-std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring = 0);
+// 1 = level storage (DevicePlan::ring).  records: lay down the far pair records where memory allows
+std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring, bool records);
 void device_free(DevicePlan& D);
 // coarse cones of one mult's standalone values -> coefficients transform (all of them unless
 // leaf sampling and the grouped upward kernel transform their own)

@@ -334,7 +334,7 @@ void k_far_rows(
             cf = {R(INV_4PI_D * rinv), R(0)};
         else
             cf = cscale(expmk_far<R>(B.k_re, B.k_im, r), R(INV_4PI_D * rinv));
-        acc = cadd(acc, cmul(val[0], cf));
+        acc = cmul_add(acc, val[0], cf);
     };
     // the next source box's index is loaded one box ahead, so that its geometry loads do not
     // wait for it
@@ -553,7 +553,7 @@ void k_far_rec(
                         const R y0[1] = {x0}, y1[1] = {x1}, y2[1] = {x2};
                         eval_any<R, 1>(l, kp.lo0, kp.lo1, kp.lo2, y0, y1, y2, v);
                     }
-                    acc = cadd(acc, cmul(v[0], c0));
+                    acc = cmul_add(acc, v[0], c0);
                 }
                 // the next step's staging writes stay behind this step's LDS reads
                 asm volatile("" ::: "memory");
@@ -569,7 +569,7 @@ void k_far_rec(
                 const R y0[1] = {x0}, y1[1] = {x1}, y2[1] = {x2};
                 eval_any<R, 1>(c, kp.lo0, kp.lo1, kp.lo2, y0, y1, y2, v);
             }
-            acc = cadd(acc, cmul(v[0], c0));
+            acc = cmul_add(acc, v[0], c0);
         }
     }
     for (int m = Tp; m < 64; m <<= 1)

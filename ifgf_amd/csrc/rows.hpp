@@ -15,6 +15,13 @@ namespace dev
 __device__ __forceinline__ float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double fma_r(double a, double b, double c) { return fma(a, b, c); }
 
+// acc + a b, each rounding in its place: left to the compiler, the far field from the pair records and
+// the one that locates the pairs fused different products of a b, and their results differed
+template <typename R> __device__ __forceinline__ Cx<R> cmul_add(Cx<R> acc, Cx<R> a, Cx<R> b)
+{
+    return {acc.x + fma_r(a.x, b.x, -(a.y * b.y)), acc.y + fma_r(a.x, b.y, a.y * b.x)};
+}
+
 // A cone's coefficients are read a chunk ahead of the arithmetic, in two buffers of at most
 // CHUNK complex values (48 bytes of registers each): whole axis-2 planes where one or more fit,
 // else a plane's rows in equal parts

@@ -75,7 +75,7 @@ class _IfgfOperator:
 
     # IfgfOperator::init (ifgfoperator.hpp:65-106)
     def init(self, srcs, targets, cutOff=None, normals=None, *, plan_only=False,
-             host_plan=False, level_ring=False):
+             host_plan=False, level_ring=False, pair_records=True):
         s = _points(srcs, "srcs")
         t = _points(targets, "targets")
         n = None if normals is None else _points(normals, "normals")
@@ -86,7 +86,8 @@ class _IfgfOperator:
                              None if n is None else n.ctypes.data, cb, None,
                              (_lib.INIT_PLAN_ONLY if plan_only else 0)
                              | (_lib.INIT_HOST_PLAN if host_plan else 0)
-                             | (_lib.INIT_LEVEL_RING if level_ring else 0))
+                             | (_lib.INIT_LEVEL_RING if level_ring else 0)
+                             | (0 if pair_records else _lib.INIT_NO_PAIR_RECORDS))
         check(rc, self._h, "init")
         self._n, self._m = s.shape[0], t.shape[0]
 
@@ -96,13 +97,14 @@ class _IfgfOperator:
         them every time)."""
         check(lib().ifgf_plan_save(self._h, os.fsencode(path)), self._h, "save_plan")
 
-    def load_plan(self, path, *, plan_only=False, level_ring=False):
+    def load_plan(self, path, *, plan_only=False, level_ring=False, pair_records=True):
         """init from a file written by save_plan, for an operator of the same kernel,
         wavenumber, leaf size, order, n_elem and tolerance: the same results, bit for bit,
         without rebuilding the plan."""
         rc = lib().ifgf_init_from_plan(self._h, os.fsencode(path),
                                        (_lib.INIT_PLAN_ONLY if plan_only else 0)
-                                       | (_lib.INIT_LEVEL_RING if level_ring else 0))
+                                       | (_lib.INIT_LEVEL_RING if level_ring else 0)
+                                       | (0 if pair_records else _lib.INIT_NO_PAIR_RECORDS))
         check(rc, self._h, "load_plan")
         n_src, n_tgt = ctypes.c_int64(), ctypes.c_int64()
         check(lib().ifgf_sizes(self._h, ctypes.byref(n_src), ctypes.byref(n_tgt)), self._h,
@@ -264,13 +266,15 @@ class MergedIfgfOperator(_IfgfOperator):
     every phase of mult runs one launch per level for all geometries.  mult takes the parts'
     densities concatenated (or a list of them, returning a list of results)."""
 
-    def __init__(self, ops, *, plan_only=False):
+    def __init__(self, ops, *, plan_only=False, pair_records=True):
         ops = list(ops)
         if not ops or any(getattr(o, "_n", None) is None for o in ops):
             raise _lib.IfgfError("merge needs initialised operators")
         arr = (ctypes.c_void_p * len(ops))(*[o._h.value for o in ops])
         h = ctypes.c_void_p()
-        rc = lib().ifgf_merge(arr, len(ops), _lib.INIT_PLAN_ONLY if plan_only else 0,
+        rc = lib().ifgf_merge(arr, len(ops),
+                              (_lib.INIT_PLAN_ONLY if plan_only else 0)
+                              | (0 if pair_records else _lib.INIT_NO_PAIR_RECORDS),
                               ctypes.byref(h))
         check(rc, ops[0]._h, "merge")
         self._h = h
@@ -293,9 +297,9 @@ class MergedIfgfOperator(_IfgfOperator):
         return super().mult(weights)
 
 
-def merge(ops, *, plan_only=False):
+def merge(ops, *, plan_only=False, pair_records=True):
     """One operator for several initialised operators of one class and one set of orders."""
-    return MergedIfgfOperator(ops, plan_only=plan_only)
+    return MergedIfgfOperator(ops, plan_only=plan_only, pair_records=pair_records)
 
 
 class HelmholtzIfgfOperator(_IfgfOperator):

@@ -47,6 +47,10 @@ extern "C" {
                                   as its coefficients are written, and mults of several columns
                                   run one column at a time).  Chosen by init when every level's
                                   do not fit the free device memory. */
+#define IFGF_INIT_NO_PAIR_RECORDS 8 /* lay down no records of where each target lies in each of its
+                                  far source boxes (24 bytes a pair, FP64 48; by default init
+                                  does where device memory allows): the far field then locates
+                                  the targets in every mult, for the same results */
 
 /* ifgf_mult flags */
 #define IFGF_DEVICE_POINTERS 1 /* w and out are device pointers; work is enqueued on stream */
@@ -86,8 +90,8 @@ int ifgf_init(ifgf_operator* op, const double* srcs, int64_t n_src, const double
  * upward tables, the geometries of a merged operator) and its launch shape to a file.
  * ifgf_init_from_plan reads one into an operator created with the same kernel, wavenumber,
  * leaf size, order, n_elem and tolerance (IFGF_EINVAL otherwise), then uploads it as
- * ifgf_init does (flags: IFGF_INIT_PLAN_ONLY, IFGF_INIT_LEVEL_RING) and applies the saved
- * launch shape; the gradient direction stays the operator's (ifgf_set_dx).  Results equal
+ * ifgf_init does (flags: IFGF_INIT_PLAN_ONLY, IFGF_INIT_LEVEL_RING,
+ * IFGF_INIT_NO_PAIR_RECORDS) and applies the saved launch shape; the gradient direction stays the operator's (ifgf_set_dx).  Results equal
  * those of the operator that wrote the file, bit for bit.  The file is checked (format,
  * version, byte order, length, a 64-bit checksum, array sizes and indices); a damaged or
  * foreign file gives IFGF_EINVAL and leaves the operator as it was.  Load only files this
@@ -134,7 +138,7 @@ int ifgf_mult_adjoint(ifgf_operator* op, const double* g, int64_t nrhs, double* 
  * wavenumber and points.  Precision and kernel family are those of ops[0].  No counterpart in
  * the reference (one geometry per IfgfOperator); for batches of many geometries.  The parts
  * stay the caller's; errors are reported on ops[0].  flags: IFGF_INIT_PLAN_ONLY merges the
- * host plans only (introspection). */
+ * host plans only (introspection); IFGF_INIT_NO_PAIR_RECORDS. */
 int ifgf_merge(ifgf_operator* const* ops, int n_ops, int flags, ifgf_operator** out);
 
 /* Numbers of sources and targets of a planned operator (a merged one: the sums). */

@@ -497,19 +497,25 @@ void k_far_cols(
 }
 typedef float mf4 __attribute__((ext_vector_type(4)));
 
-// Far field from the pair records for NC of the nc columns (blockIdx.y picks which), any orders: a
-// workgroup per item, its waves sharing the item's sources; lanes = (target, run of sources) as in
-// k_far_rec.  Per step the wave copies its lanes' distinct cones (up to most at a time, the NC
+// Far field for NC of the nc columns (blockIdx.y picks which), any orders: a workgroup per item, its
+// waves sharing the item's sources; lanes = (target, run of sources) as in k_far_rec.  PLACE: where
+// the pairs lie, read from their records (0) or, without those, located by locate_fast (1) or
+// locate (2), so that the results do not depend on the room for records.  Per step the wave copies its lanes' distinct cones (up to most at a time, the NC
 // columns' coefficients next to one another) to LDS and each lane adds coefficient times
 // Chebyshev product for its target, one product for the columns.  Bound by the LDS reads (8 NC
 // bytes per lane and coefficient).  Whole mult of 3 and 5 columns, with the kernels that evaluate
 // 16 columns at a time -> with this one: 8.0 -> 4.1 and 9.1 -> 5.3 ms at (2,3,3), 262,144 points;
 // 6.8 -> 3.3 and 7.7 -> 4.8 at (3,5,4), 100,000 points; FP64 at (3,5,4), 50,000 points, 6.9 -> 4.9
 // and 10.3 -> 8.3.  NC of 8 and 16 instead (fewer groups, more registers and LDS per wave): 12
-// columns 12.4 and 17.9 ms against 11.9.
-template <typename R, int O0, int NC>
+// columns 12.4 and 17.9 ms against 11.9.  Without records, where every group of columns locates
+// the pairs: 3, 5 and 12 columns at (2,3,3) 8.6 -> 5.5, 9.8 -> 6.8 and 15.1 -> 14.4 ms, FP64 at
+// (3,5,4), 50,000 points, 7.5 -> 6.0, 10.8 -> 10.0 and, slower, 18.0 -> 21.5.
+template <typename R, int O0, int NC, int PLACE>
 __global__ __launch_bounds__(512)
-void k_far_rec_cols(const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
+void k_far_few_cols(const WorkItem* __restrict__ items, const int32_t* __restrict__ srange,
+                    const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,
+                    const CellRef* __restrict__ ctab, const double* __restrict__ tpts,
+                    const double* __restrict__ ang, int ang_base, int phase,
                     const int64_t* __restrict__ rec_off, const FarRec<R>* __restrict__ rec,
                     const Cx<R>* __restrict__ cfs, const Cx<R>* __restrict__ F, int nc, int most,
                     int stride, int64_t ntgt, Cx<R>* __restrict__ far_res, KParams kp)
@@ -526,10 +532,23 @@ void k_far_rec_cols(const WorkItem* __restrict__ items, const int32_t* __restric
     const int ti = lane & (Tp - 1);
     const int grp = lane / Tp, ngrp = 64 / Tp;
     const bool valid = ti < wi.count;
-    const int32_t n = srange[2 * it + 1] - srange[2 * it];
+    const int32_t j0 = srange[2 * it], n = srange[2 * it + 1] - j0;
     const int32_t ja = n * wave / wpb, jb = n * (wave + 1) / wpb;
-    const FarRec<R>* rp = rec + rec_off[it] + ti;
-    const Cx<R>* cp = cfs + rec_off[it] + ti;
+    const FarRec<R>* rp = nullptr;
+    const Cx<R>* cp = nullptr;
+    double y0 = 0, y1 = 0, y2 = 0;
+    if constexpr (PLACE == 0)
+    {
+        rp = rec + rec_off[it] + ti;
+        cp = cfs + rec_off[it] + ti;
+    }
+    else if (valid)
+    {
+        const int64_t t = int64_t(wi.first) + ti;
+        y0 = tpts[3 * t];
+        y1 = tpts[3 * t + 1];
+        y2 = tpts[3 * t + 2];
+    }
     constexpr int ROWS = 64 / NC; // rows of NC columns the wave copies at a time
     const int n_lo = kp.n_lo;
     const int col = lane % NC, row0 = lane < ROWS * NC ? lane / NC : 4 * n_lo;
@@ -545,13 +564,20 @@ void k_far_rec_cols(const WorkItem* __restrict__ items, const int32_t* __restric
         qs = -1;
         if (valid && j + grp < jb)
         {
-            const int64_t e = int64_t(j + grp) * wi.count;
-            const FarRec<R> q = rp[e];
+            FarRec<R> q;
+            if constexpr (PLACE == 0)
+            {
+                const int64_t e = int64_t(j + grp) * wi.count;
+                q = rp[e];
+                cf = cp[e];
+            }
+            else
+                place_pair<R, PLACE == 1>(geo[far_src[j0 + j + grp]], ctab, ang + ang_base, ang_base,
+                                          y0, y1, y2, phase, kp, q, cf);
             qs = q.slot;
             q0 = q.x0;
             q1 = q.x1;
             q2 = q.x2;
-            cf = cp[e];
         }
     };
     fetch(ja);
@@ -1035,14 +1061,14 @@ void launch_transform_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int
         c0, xsz, D.cones, V, F, static_cast<const R*>(D.wmat), nc, cw, nch, kp);
 }
 
-// k_far_rec_cols for a call of at most FEW_COLUMNS columns, where the plan has pair records and a
-// cone's coefficients for five columns fit the LDS; false otherwise
+// k_far_few_cols for a call of at most FEW_COLUMNS columns, where a cone's coefficients for five
+// columns fit the LDS; false otherwise
 template <typename R>
-static bool launch_far_rec_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
+static bool launch_far_few_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step,
                                 const Cx<R>* F, Cx<R>* far_res, int nc)
 {
     constexpr size_t CX = sizeof(Cx<R>);
-    if (!D.far_rec || (size_t(D.n_lo) * 5 + 2) * CX > size_t(64) * 1024)
+    if ((size_t(D.n_lo) * 5 + 2) * CX > size_t(64) * 1024)
         return false;
     const DevicePlan::FarGroup& G = D.far_steps[step];
     const int64_t n = G.item1 - G.item0;
@@ -1053,30 +1079,42 @@ static bool launch_far_rec_cols(DevicePlan& D, hipStream_t st, const KParams& kp
         w /= 2;
     // groups of at most five columns, as equal as they go
     const int gy = (nc + 4) / 5;
-    auto go = [&](auto o0, auto ncc)
+    auto go = [&](auto o0, auto ncc, auto place)
     {
         constexpr int O0 = decltype(o0)::value, NC = decltype(ncc)::value;
+        constexpr int PLACE = decltype(place)::value;
         // 16-byte words, an odd number of them, so that the cones start in different banks
         const int stride = sizeof(R) == 4 ? (((D.n_lo * NC + 1) / 2) | 1) * 2 : (D.n_lo * NC) | 1;
         const size_t cone = size_t(stride) * CX;
         const int most = int(std::min<size_t>(4, std::max<size_t>(1, size_t(12) * 1024 / cone)));
         const size_t lds = std::max(cone * most * w, w > 1 ? size_t(w) * 64 * NC * CX : 0);
         if (lds > size_t(64) * 1024)
-            HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_far_rec_cols<R, O0, NC>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-        k_far_rec_cols<R, O0, NC><<<dim3(unsigned(n), unsigned(gy)), dim3(64 * w), lds, st>>>(
-            D.far_items + G.item0, D.far_srange + 2 * G.item0, D.far_rec_off + G.item0,
+            HIP_OK(hipFuncSetAttribute(
+                reinterpret_cast<const void*>(&k_far_few_cols<R, O0, NC, PLACE>),
+                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        k_far_few_cols<R, O0, NC, PLACE><<<dim3(unsigned(n), unsigned(gy)), dim3(64 * w), lds, st>>>(
+            D.far_items + G.item0, D.far_srange + 2 * G.item0, D.far_src, D.geo, D.ctab, D.tgt_pts,
+            D.fine_ang, G.ang_base, D.kind != KL, D.far_rec ? D.far_rec_off + G.item0 : nullptr,
             static_cast<const FarRec<R>*>(D.far_rec), static_cast<const Cx<R>*>(D.far_cf), F, nc,
             most, stride, D.ntgt, far_res, kp);
     };
-    auto cols = [&](auto o0)
+    auto width = [&](auto o0, auto place)
     {
         switch ((nc + gy - 1) / gy)
         {
-        case 5: go(o0, std::integral_constant<int, 5>()); break;
-        case 4: go(o0, std::integral_constant<int, 4>()); break;
-        default: go(o0, std::integral_constant<int, 3>()); break;
+        case 5: go(o0, std::integral_constant<int, 5>(), place); break;
+        case 4: go(o0, std::integral_constant<int, 4>(), place); break;
+        default: go(o0, std::integral_constant<int, 3>(), place); break;
         }
+    };
+    auto cols = [&](auto o0)
+    {
+        if (D.far_rec)
+            return width(o0, std::integral_constant<int, 0>());
+        if constexpr (sizeof(R) == 4)
+            if (G.ang_n > 0)
+                return width(o0, std::integral_constant<int, 1>());
+        width(o0, std::integral_constant<int, 2>());
     };
     switch (D.lo[0])
     {
@@ -1094,7 +1132,7 @@ template <typename R>
 void launch_far_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int step, const Cx<R>* F,
                      Cx<R>* far_res, int nc, bool few)
 {
-    if (few && launch_far_rec_cols<R>(D, st, kp, step, F, far_res, nc))
+    if (few && launch_far_few_cols<R>(D, st, kp, step, F, far_res, nc))
         return;
     const DevicePlan::FarGroup& G = D.far_steps[step];
     const int64_t n = G.item1 - G.item0;

@@ -262,7 +262,7 @@ void device_free(DevicePlan& D);
 int64_t device_transform_cones(const DevicePlan& D);
 // batched mult (batched.hip): ncol <= b_rb columns of device densities
 constexpr int MAX_COLUMNS = 32;
-// calls of at most this many columns take the far field by groups of columns (k_far_rec_cols), the
+// calls of at most this many columns take the far field by groups of columns (k_far_few_cols), the
 // others 16 real columns at a time.  Whole mult of 8, 12 and 16 columns by groups / by tiles:
 // 7.9 / 10.2, 11.9 / 14.6 and 16.4 / 16.1 ms at (2,3,3), 262,144 points; 7.3 / 8.6, 11.5 / 11.6 and
 // 15.0 / 13.3 at (3,5,4), 100,000 points; FP64 at (3,5,4), 50,000 points, 11.6 / 12.3, 17.2 / 17.3

@@ -407,47 +407,10 @@ __global__ __launch_bounds__(64) void k_far_record(
     {
         const int j = e / wi.count;
         const int64_t t = int64_t(wi.first) + (e - j * wi.count);
-        const BoxGeo& B = geo[far_src[j0 + j]];
-        const double v0 = tpts[3 * t] - B.ctr[0], v1 = tpts[3 * t + 1] - B.ctr[1],
-                     v2 = tpts[3 * t + 2] - B.ctr[2];
-        FarRec<R> q{};
-        q.slot = -1;
-        Cx<R> cf = {R(0), R(0)};
-        double r = 1, ri = 1;
-        bool ok;
-        if constexpr (FAST)
-        {
-            LocF L;
-            ok = locate_fast(B, rec_ang + (2 * B.fth_off - ang_base),
-                             rec_ang + (2 * B.fph_off - ang_base), ctab, v0, v1, v2, kp.f0, kp.f1,
-                             kp.f2, L);
-            if (ok)
-            {
-                q.slot = L.fine;
-                q.x0 = R(L.xi[0]);
-                q.x1 = R(L.xi[1]);
-                q.x2 = R(L.xi[2]);
-                r = L.r;
-                ri = L.rinv;
-            }
-        }
-        else
-        {
-            Loc L;
-            ok = locate(B, ctab, v0, v1, v2, kp.f0, kp.f1, kp.f2, L);
-            if (ok)
-            {
-                q.slot = L.fine;
-                q.x0 = R(L.xi[0]);
-                q.x1 = R(L.xi[1]);
-                q.x2 = R(L.xi[2]);
-                r = L.r;
-                ri = 1.0 / L.r;
-            }
-        }
-        if (ok)
-            cf = phase ? cscale(expmk_far<R>(B.k_re, B.k_im, r), R(INV_4PI_D * ri))
-                       : Cx<R>{R(INV_4PI_D * ri), R(0)};
+        FarRec<R> q;
+        Cx<R> cf;
+        place_pair<R, FAST>(geo[far_src[j0 + j]], ctab, FAST ? rec_ang : nullptr, ang_base,
+                            tpts[3 * t], tpts[3 * t + 1], tpts[3 * t + 2], phase, kp, q, cf);
         rec[off + e] = q;
         cfs[off + e] = cf;
     }

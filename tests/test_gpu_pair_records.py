@@ -63,7 +63,7 @@ def _make(kind, order, tol, k, prec):
 def test_orders_and_columns(gpu, kind, order, tol, n, k, prec):
     x = spheroid(n, 501) if tol < 0 else sphere(n, 100 + n % 97)
     a, b = _pair(_make(kind, order, tol, k, prec), x, x)
-    for ncol in (1, 13, 32):
+    for ncol in (1, 4, 5, 12, 13, 32):
         print(f"{kind} order {order} prec={prec} columns={ncol}", flush=True)
         W = _columns(n, ncol)
         _same(a, b, W.real.copy() if kind == "laplace" else W)
@@ -87,7 +87,7 @@ def test_other_targets_adjoint_level_storage_and_merged(gpu, prec, tmp_path):
     x, y = spheroid(4000, 506), sphere(2500, 507) * 1.4
     make = lambda: ifgf_amd.HelmholtzIfgfOperator(9.0, 30, 6, 1, -1, precision=prec)
     a, b = _pair(make, x, y)
-    for ncol in (1, 16):
+    for ncol in (1, 5, 16):
         _same(a, b, _columns(4000, ncol))
         g = _columns(2500, ncol)
         assert np.array_equal(a.mult_adjoint(g), b.mult_adjoint(g))
@@ -106,5 +106,5 @@ def test_other_targets_adjoint_level_storage_and_merged(gpu, prec, tmp_path):
         parts.append(op)
     ma, mb = ifgf_amd.merge(parts), ifgf_amd.merge(parts, pair_records=False)
     assert mb.plan_counts()["device_bytes"] < ma.plan_counts()["device_bytes"]
-    for ncol in (1, 14):
+    for ncol in (1, 4, 14):
         _same(ma, mb, _columns(5000, ncol))

@@ -202,10 +202,13 @@ __device__ __forceinline__ void stage_cones(const Cx<R>* __restrict__ F, int c0,
 // coefficients are not all in registers (eval_point).  Far phase against the kernel that read each
 // coefficient from memory in Clenshaw order: 24.8 -> 8.8 ms at (3,6,4), 1M points; 26 -> 6.8 ms at
 // (5,5,5), combined field on a torus, 131,072 points; with a read-ahead in two buffers instead
-// 27 registers spilled at (2,5,*).
+// 27 registers spilled at (2,5,*).  At six coefficients a plane 8 waves per SIMD (4 registers
+// spilled at (2,3)) against 7: far phase 4.74 -> 4.63 ms, whole mult 8.65 -> 8.43 at (2,3,3), 1M
+// points; with fewer, slower (2.33 -> 2.38 at (2,2,2), 400,000 points).
 template <typename R, int O0, int O1, bool FAST>
 __global__ __launch_bounds__(512)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : (O0 * O1 > 24 ? 1 : 2))))
+__attribute__((amdgpu_waves_per_eu(
+    sizeof(R) == 4 ? (O0 * O1 == 6 ? 8 : 4) : (O0 * O1 > 24 ? 1 : 2))))
 void k_far_rows(
     const WorkItem* __restrict__ items, int64_t nitems, const int32_t* __restrict__ srange,
     const int32_t* __restrict__ far_src, const BoxGeo* __restrict__ geo,

@@ -20,13 +20,14 @@
 #include <map>
 #include <mutex>
 #include <stdexcept>
-#include <thread>
 #include <type_traits>
 #include <utility>
 
 #include "dev_common.hpp"
 #include "device.hpp"
+#include "jobs.hpp"
 #include "orders.hpp"
+#include "up_groups.hpp"
 
 namespace ifgf
 {
@@ -843,147 +844,6 @@ static std::vector<WorkItem> make_items(const std::vector<int32_t>& boxes, const
             out.push_back({b, int32_t(f), int32_t(std::min<int64_t>(64, e - f)), 0});
     }
     return out;
-}
-
-// The upward tables regrouped by child cone: per (cell, octant) row the distinct child fine
-// cones (cf, sub) its nodes fall into, in order of first appearance, and per child cone its
-// nodes (ascending) in records of at most Rec::N.  Row r's cones are dkey[2 doff[r] ..], its
-// records [goff[r], goff[r + 1]).
-template <class Rec> struct GroupTables
-{
-    std::vector<Rec> grp;
-    std::vector<int32_t> goff, doff, dkey;
-};
-// the rows of cells [c0, c1) of one part, appended to T
-template <class Rec>
-void group_cells(const UpLevel& U, int n_hi, int64_t c0, int64_t c1, GroupTables<Rec>& T)
-{
-    std::vector<int32_t> gcnt, gnode, nd(n_hi);
-    for (int64_t cell = c0; cell < c1; cell++)
-        for (int c = 0; c < 8; c++)
-        {
-            const UpEntry* row = &U.entries[size_t(cell) * n_hi * 8 + c]; // node q: row[8 q]
-            const size_t k0 = T.dkey.size() / 2;
-            T.doff.push_back(int32_t(k0));
-            T.goff.push_back(int32_t(T.grp.size()));
-            int last = -1; // neighbouring nodes mostly share the last cone found
-            for (int q = 0; q < n_hi; q++)
-            {
-                const UpEntry& E = row[8 * q];
-                nd[q] = -1;
-                if (E.cf < 0)
-                    continue;
-                const int nk = int(T.dkey.size() / 2 - k0);
-                auto is = [&](int i)
-                { return T.dkey[2 * (k0 + i)] == E.cf && T.dkey[2 * (k0 + i) + 1] == E.sub; };
-                int d = (last >= 0 && is(last)) ? last : -1;
-                for (int i = 0; d < 0 && i < nk; i++)
-                    if (is(i))
-                        d = i;
-                if (d < 0)
-                {
-                    d = nk;
-                    T.dkey.push_back(E.cf);
-                    T.dkey.push_back(E.sub);
-                }
-                nd[q] = last = d;
-            }
-            const int nk = int(T.dkey.size() / 2 - k0);
-            gcnt.assign(size_t(nk) + 1, 0);
-            for (int q = 0; q < n_hi; q++)
-                if (nd[q] >= 0)
-                    gcnt[size_t(nd[q]) + 1]++;
-            for (int i = 0; i < nk; i++)
-                gcnt[i + 1] += gcnt[i];
-            gnode.assign(size_t(gcnt[nk]), 0);
-            for (int q = 0; q < n_hi; q++)
-                if (nd[q] >= 0)
-                    gnode[size_t(gcnt[nd[q]]++)] = q;
-            for (size_t i = 0; i < gnode.size();)
-            {
-                const int d = nd[gnode[i]];
-                Rec G{};
-                G.cf = row[8 * gnode[i]].cf;
-                G.subd = row[8 * gnode[i]].sub | (d << 8);
-                uint32_t qs[4] = {0xffffu, 0xffffu, 0xffffu, 0xffffu};
-                for (int g = 0; g < Rec::N && i < gnode.size() && nd[gnode[i]] == d; g++, i++)
-                {
-                    using X = typename std::remove_reference<decltype(G.x0[0])>::type;
-                    const UpEntry& E = row[8 * gnode[i]];
-                    qs[g] = uint32_t(gnode[i]);
-                    G.x0[g] = X(E.xi[0]);
-                    G.x1[g] = X(E.xi[1]);
-                    G.x2[g] = X(E.xi[2]);
-                    G.tr[g] = X(E.tf[0]);
-                    G.ti[g] = X(E.tf[1]);
-                }
-                G.q01 = qs[0] | (qs[1] << 16);
-                if constexpr (Rec::N == 4)
-                    G.q23 = qs[2] | (qs[3] << 16);
-                T.grp.push_back(G);
-            }
-        }
-}
-// every part's rows, by up to 16 threads; part_cell[part]: the part's first cell
-template <class Rec>
-GroupTables<Rec> group_tables(const std::vector<const UpLevel*>& parts, int n_hi,
-                              std::vector<int64_t>& part_cell)
-{
-    struct Job
-    {
-        const UpLevel* U;
-        int64_t c0, c1;
-    };
-    std::vector<Job> jobs;
-    int64_t cells = 0;
-    for (const UpLevel* U : parts)
-    {
-        part_cell.push_back(cells);
-        const int64_t n = int64_t(U->entries.size()) / (int64_t(n_hi) * 8);
-        for (int64_t c = 0; c < n; c += 64)
-            jobs.push_back({U, c, std::min<int64_t>(n, c + 64)});
-        cells += n;
-    }
-    std::vector<GroupTables<Rec>> out(jobs.size());
-    const size_t nth = std::min<size_t>(16, std::max<size_t>(1, jobs.size()));
-    auto work = [&](size_t t)
-    {
-        for (size_t j = t; j < jobs.size(); j += nth)
-            group_cells(*jobs[j].U, n_hi, jobs[j].c0, jobs[j].c1, out[j]);
-    };
-    std::vector<std::thread> pool;
-    for (size_t t = 1; t < nth; t++)
-        pool.emplace_back(work, t);
-    work(0);
-    for (auto& th : pool)
-        th.join();
-    GroupTables<Rec> T;
-    size_t ng = 0, nk = 0;
-    for (const auto& o : out)
-    {
-        ng += o.grp.size();
-        nk += o.dkey.size();
-    }
-    if (nk / 2 > size_t(INT32_MAX))
-        throw std::runtime_error("upward tables: too many distinct child cones");
-    if (ng > size_t(INT32_MAX))
-        throw std::runtime_error("upward tables: too many node groups");
-    T.grp.reserve(ng);
-    T.dkey.reserve(nk);
-    for (auto& o : out)
-    {
-        const int32_t g0 = int32_t(T.grp.size()), k0 = int32_t(T.dkey.size() / 2);
-        for (int32_t v : o.goff)
-            T.goff.push_back(g0 + v);
-        for (int32_t v : o.doff)
-            T.doff.push_back(k0 + v);
-        T.grp.insert(T.grp.end(), o.grp.begin(), o.grp.end());
-        T.dkey.insert(T.dkey.end(), o.dkey.begin(), o.dkey.end());
-        o = GroupTables<Rec>();
-    }
-    T.goff.push_back(int32_t(T.grp.size()));
-    T.doff.push_back(int32_t(T.dkey.size() / 2));
-    return T;
 }
 
 // the upward pass into parent level `level`: cones with a table, then cones a .. b of the others
@@ -1852,13 +1712,8 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring,
                 }
             };
             const size_t n = desc.size();
-            const size_t nth = std::min<size_t>(16, std::max<size_t>(1, n / 4096));
-            std::vector<std::thread> pool;
-            for (size_t t = 1; t < nth; t++)
-                pool.emplace_back(fill, n * t / nth, n * (t + 1) / nth);
-            fill(0, n / nth);
-            for (auto& th : pool)
-                th.join();
+            const size_t nj = std::max<size_t>(1, n / 4096);
+            run_jobs(nj, 16, [&](size_t j) { fill(n * j / nj, n * (j + 1) / nj); });
             D.up_tl_desc = dupload(desc, tot);
         }
         D.tr_list_off[D.levels] = int64_t(tr_list.size());

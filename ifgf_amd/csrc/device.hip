@@ -1931,12 +1931,20 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring,
                 roff[i + 1] = roff[i] + int64_t(fitems[i].count) * (frange[2 * i + 1] - frange[2 * i]);
             const size_t pairs = size_t(roff.back());
             const size_t rs = precision == PREC_FP64 ? sizeof(FarRec<double>) : sizeof(FarRec<float>);
+            const size_t bytes = (rs + cs) * pairs + sizeof(int64_t) * roff.size();
             HIP_OK(hipMemGetInfo(&free_b, &total_b));
-            if (records && pairs > 0 && (rs + cs) * pairs <= free_b / 4)
+            // at most a quarter of the free memory; the far field does without them where another
+            // program was faster to take it
+            void* off = nullptr;
+            if (records && pairs > 0 && 4 * bytes <= free_b &&
+                device_alloc_all({{&off, sizeof(int64_t) * roff.size()},
+                                  {&D.far_rec, rs * pairs},
+                                  {&D.far_cf, cs * pairs}}))
             {
-                D.far_rec_off = dupload(roff, tot);
-                D.far_rec = dalloc<unsigned char>(rs * pairs, tot);
-                D.far_cf = dalloc<unsigned char>(cs * pairs, tot);
+                D.far_rec_off = static_cast<int64_t*>(off);
+                tot += int64_t(bytes);
+                HIP_OK(hipMemcpy(off, roff.data(), sizeof(int64_t) * roff.size(),
+                                 hipMemcpyHostToDevice));
                 if (precision == PREC_FP64)
                     record_far<double>(D);
                 else

@@ -6,8 +6,10 @@
 
 #include <algorithm>
 #include <cstddef>
+#include <initializer_list>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #define HIP_OK(x)                                                                          \
@@ -20,6 +22,25 @@
 
 namespace ifgf
 {
+// device memory for several arrays (pointer, bytes): all of them, or none and false
+inline bool device_alloc_all(std::initializer_list<std::pair<void**, size_t>> arrays)
+{
+    for (auto a = arrays.begin(); a != arrays.end(); ++a)
+        if (hipMalloc(a->first, a->second) != hipSuccess)
+        {
+            *a->first = nullptr;
+            while (a != arrays.begin())
+            {
+                --a;
+                (void)hipFree(*a->first);
+                *a->first = nullptr;
+            }
+            (void)hipGetLastError(); // handled: not for the next call to report
+            return false;
+        }
+    return true;
+}
+
 // a device allocation freed with its owner; grows geometrically (at least 256 bytes)
 struct DBuf
 {

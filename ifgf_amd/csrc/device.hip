@@ -1933,10 +1933,10 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring,
             const size_t rs = precision == PREC_FP64 ? sizeof(FarRec<double>) : sizeof(FarRec<float>);
             const size_t bytes = (rs + cs) * pairs + sizeof(int64_t) * roff.size();
             HIP_OK(hipMemGetInfo(&free_b, &total_b));
-            // at most a quarter of the free memory; the far field does without them where another
-            // program was faster to take it
+            // at most a quarter of the memory beyond the margin; the far field does without them
+            // where another program was faster to take it
             void* off = nullptr;
-            if (records && pairs > 0 && 4 * bytes <= free_b &&
+            if (records && pairs > 0 && 4 * bytes + margin <= free_b &&
                 device_alloc_all({{&off, sizeof(int64_t) * roff.size()},
                                   {&D.far_rec, rs * pairs},
                                   {&D.far_cf, cs * pairs}}))

@@ -192,8 +192,8 @@ struct DevicePlan
     // records from far_rec_off[i] on, its targets fastest): the fine slot and local coordinates
     // (FarRec) and the centre factor.  All from the geometry and the wavenumber, so recorded once
     // at upload by the location the far field would otherwise repeat in every mult; null when
-    // they would take more than a quarter of the free device memory (24 bytes a pair in the mixed
-    // form, 48 in FP64).
+    // they would take more than a quarter of the free device memory less 4 GiB (24 bytes a pair in
+    // the mixed form, 48 in FP64), or were refused.
     int64_t* far_rec_off = nullptr;
     void* far_rec = nullptr; // FarRec<R>
     void* far_cf = nullptr;  // Cx<R>

@@ -108,3 +108,31 @@ def test_other_targets_adjoint_level_storage_and_merged(gpu, prec, tmp_path):
     assert mb.plan_counts()["device_bytes"] < ma.plan_counts()["device_bytes"]
     for ncol in (1, 4, 14):
         _same(ma, mb, _columns(5000, ncol))
+
+
+def test_records_leave_the_margin_free(gpu):
+    """With 4 GiB and twice the records' memory left an operator goes without records (they take at
+    most a quarter of what there is beyond 4 GiB); with the memory given back it has them."""
+    import torch
+    GiB = 1 << 30
+    x, w = sphere(60000, 520), cdens(60000, 521)
+    make = lambda: ifgf_amd.HelmholtzIfgfOperator(20.0, 64, 6, 1, -1)
+    a, b = _pair(make, x, x)
+    u = a.mult(w)
+    have, bare = (op.plan_counts()["device_bytes"] for op in (a, b))
+    rec = have - bare
+    print(f"pair records {rec / GiB:.2f} GiB", flush=True)
+    assert GiB // 4 < rec < 2 * GiB
+    del a, b
+    torch.cuda.empty_cache()
+    left = bare + 4 * GiB + 2 * rec
+    filler = torch.empty(torch.cuda.mem_get_info()[0] - left, dtype=torch.uint8, device="cuda:0")
+    op = make()
+    op.init(x.T, x.T)
+    c = op.plan_counts()
+    assert c["device_bytes"] == bare and c["level_ring"] == 0
+    assert np.array_equal(op.mult(w), u)
+    del filler
+    torch.cuda.empty_cache()
+    op.init(x.T, x.T)
+    assert op.plan_counts()["device_bytes"] == have and np.array_equal(op.mult(w), u)

@@ -47,6 +47,25 @@ static int fail(ifgf_operator* op, int code, const std::string& msg)
     return code;
 }
 
+// the fields of a launch shape in the order of the C ABI
+static void shape_fields(const LaunchShape& s, int* f)
+{
+    const int v[IFGF_LAUNCH_SHAPE_FIELDS] = {s.xcd_log2, s.cpb, s.up_k, s.rb, s.far_waves, s.overlap};
+    std::memcpy(f, v, sizeof(v));
+}
+
+static LaunchShape shape_of(const int* f)
+{
+    LaunchShape s;
+    s.xcd_log2 = f[0];
+    s.cpb = f[1];
+    s.up_k = f[2];
+    s.rb = f[3];
+    s.far_waves = f[4];
+    s.overlap = f[5];
+    return s;
+}
+
 extern "C"
 {
     const char* ifgf_version(void) { return "ifgf_amd 0.1 (gfx950)"; }
@@ -164,9 +183,10 @@ extern "C"
             info.leaf = op->leaf;
             info.order = op->order;
             info.n_elem = op->n_elem;
-            const LaunchShape& s = op->dev.shape;
-            const int sh[6] = {s.xcd_log2, s.cpb, s.up_k, s.rb, s.far_waves, s.overlap};
-            std::memcpy(info.shape, sh, sizeof(sh));
+            // a shape that nobody chose is saved as the defaults: the upload of the load starts from
+            // its own
+            info.shape_chosen = op->dev.shape_chosen;
+            shape_fields(info.shape_chosen ? op->dev.shape : LaunchShape(), info.shape);
             info.same_points = op->same_points;
             info.merged = op->merged;
             info.had_cutoff = op->cutoff != nullptr || op->cutoff_lost;
@@ -231,16 +251,14 @@ extern "C"
             if (!e.empty())
                 return fail(op, IFGF_EINTERNAL, e);
             op->on_device = true;
-            LaunchShape s;
-            s.xcd_log2 = info.shape[0];
-            s.cpb = info.shape[1];
-            s.up_k = info.shape[2];
-            s.rb = info.shape[3];
-            s.far_waves = info.shape[4];
-            s.overlap = info.shape[5];
-            e = device_set_shape(op->dev, s);
-            if (!e.empty())
-                return fail(op, IFGF_EINVAL, std::string(path) + ": launch shape: " + e);
+            int def[6];
+            shape_fields(LaunchShape(), def);
+            if (info.shape_chosen || std::memcmp(info.shape, def, sizeof(def)) != 0)
+            {
+                e = device_set_shape(op->dev, shape_of(info.shape));
+                if (!e.empty())
+                    return fail(op, IFGF_EINVAL, std::string(path) + ": launch shape: " + e);
+            }
         }
         catch (const std::exception& ex)
         {
@@ -636,13 +654,7 @@ extern "C"
     {
         if (!op || !shape)
             return IFGF_EINVAL;
-        const LaunchShape& s = op->dev.shape;
-        shape[0] = s.xcd_log2;
-        shape[1] = s.cpb;
-        shape[2] = s.up_k;
-        shape[3] = s.rb;
-        shape[4] = s.far_waves;
-        shape[5] = s.overlap;
+        shape_fields(op->dev.shape, shape);
         return IFGF_OK;
     }
 
@@ -652,14 +664,7 @@ extern "C"
             return IFGF_EINVAL;
         if (!op->on_device)
             return fail(op, IFGF_ESTATE, "launch shapes need a device init");
-        LaunchShape s;
-        s.xcd_log2 = shape[0];
-        s.cpb = shape[1];
-        s.up_k = shape[2];
-        s.rb = shape[3];
-        s.far_waves = shape[4];
-        s.overlap = shape[5];
-        std::string e = device_set_shape(op->dev, s);
+        std::string e = device_set_shape(op->dev, shape_of(shape));
         if (!e.empty())
             return fail(op, IFGF_EINVAL, e);
         return IFGF_OK;

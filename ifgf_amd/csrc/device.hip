@@ -2207,6 +2207,7 @@ std::string device_set_shape(DevicePlan& D, const LaunchShape& sh)
                          sh.up_k != D.shape.up_k || sh.far_waves != D.shape.far_waves ||
                          sh.overlap != D.shape.overlap;
     D.shape = sh;
+    D.shape_chosen = true;
     if (changed)
         device_drop_graph(D); // the captured kernels have the old shapes
     return "";

@@ -232,6 +232,7 @@ struct DevicePlan
     std::vector<void*> ev_level; // per source level: its coefficients are written
 
     LaunchShape shape;
+    bool shape_chosen = false; // by device_set_shape, not the upload
     // per-phase device times of this operator's last timed mult (ms: near, leaf, upward,
     // transform, far, total); force_timing: time the phases of the next mults (autotuner)
     float last_ms[6] = {0, 0, 0, 0, 0, 0};

@@ -16,7 +16,9 @@ struct PlanFileInfo
     int32_t order = 0, n_elem = 0;
     int32_t shape[6] = {0, 0, 0, 0, 0, 0};
     uint8_t same_points = 0, merged = 0, had_cutoff = 0, host_plan = 0;
-    int32_t reserved = 0;
+    // 1: the shape was set by the caller or the autotuner.  0 (and in files of before): where it equals
+    // the defaults, nobody chose it, and a load keeps the upload's own
+    int32_t shape_chosen = 0;
 };
 static_assert(sizeof(PlanFileInfo) == 48, "file layout");
 

@@ -188,10 +188,12 @@ int ifgf_last_timings(const ifgf_operator* op, double* ms6);
  *         [1] transform cones per workgroup (0 = default; the compiled order classes only)
  *         [2] upward parent cones per workgroup, at most (2, 4, 8, 16; 2 after an init)
  *         [3] batched columns per pass, at most (0 = 32, 8, 32)
- *         [4] mixed far field: waves per workgroup sharing the staged angle tables (1, 2, 4, 8)
+ *         [4] far field: waves per workgroup, sharing the staged angle tables where the pairs are
+ *             located (1, 2, 4, 8; after an init 1, or 2 without pair records)
  *         [5] second stream for the far field beside the upward chain, with the near field
  *             there (1) or first on the main stream (2); 0: one stream
- * Shapes change speed, never results.  ifgf_autotune times the candidates on the operator
+ * Shapes change speed, never results.  A saved plan carries the shape the caller or the tuner
+ * chose; where nobody chose one, a load starts from an init's.  ifgf_autotune times the candidates on the operator
  * itself (synthetic densities, nrhs columns, the fastest of reps mults per candidate), one
  * choice after another, applies the best and returns it; after ifgf_init, not thread-safe
  * with concurrent mults of the same operator. */

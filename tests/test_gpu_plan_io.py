@@ -111,3 +111,33 @@ def test_merged_plan_and_allocation_free_mult(gpu, tmp_path):
     assert rc == _lib.IFGF_OK
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy(), ud.cpu().numpy())
+
+
+def test_launch_shape_that_nobody_chose(gpu, tmp_path):
+    """A plan saved with the launch shape that init or a plan-only init left loads with the shape an
+    init starts from (also without the pair records, which has another); a chosen one, be it the
+    defaults reported before an init, comes back as it was."""
+    x = sphere(3000, 65)
+
+    def op(**kw):
+        o = ifgf_amd.HelmholtzIfgfOperator(8.0, 64, 6, 1, -1)
+        if kw:
+            o.init(x.T, x.T, **kw)
+        return o
+
+    started = {r: op(pair_records=r).launch_shape for r in (True, False)}
+    reported = op().launch_shape
+    assert started[True] != reported and started[True] != started[False]
+    for saver in (op(plan_only=True), op(pair_records=True), op(pair_records=False)):
+        saver.save_plan(tmp_path / "s.plan")
+        for r in (True, False):
+            o = op()
+            o.load_plan(tmp_path / "s.plan", pair_records=r)
+            assert o.launch_shape == started[r]
+    for shape in (reported, dict(started[True], up_cones=8)):
+        saver = op(pair_records=True)
+        saver.launch_shape = shape
+        saver.save_plan(tmp_path / "s.plan")
+        o = op()
+        o.load_plan(tmp_path / "s.plan")
+        assert o.launch_shape == shape

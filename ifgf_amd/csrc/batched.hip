@@ -141,6 +141,9 @@ __global__ __launch_bounds__(64) void k_near_b(const WorkItem* __restrict__ item
                 double xn = 0;
                 if constexpr (NRM)
                     xn = d0 * sn[3 * k] + d1 * sn[3 * k + 1] + d2 * sn[3 * k + 2];
+                // (0 times the density would not do: it need not be finite)
+                if (coincident<KIND>(R(d0) * R(d0) + R(d1) * R(d1) + R(d2) * R(d2)))
+                    continue;
                 const Cx<R> g = p2p<KIND, R>(kb, R(d0), R(d1), R(d2), xn, Cx<R>{1, 0});
 #pragma unroll
                 for (int r = 0; r < RB; r++)

@@ -576,6 +576,16 @@ template <typename R> __device__ __forceinline__ R fdiv_r(R a, R b)
         return a / b;
 }
 
+// a pair that the sum leaves out (G(0) = 0), by its squared distance; the combined field forms its
+// value from what vanishes there
+template <int KIND, typename R> __device__ __forceinline__ bool coincident(R d2)
+{
+    if constexpr (KIND == KG || KIND == KD)
+        return d2 < R(1e-24);
+    else
+        return KIND != KC && d2 == R(0);
+}
+
 template <int KIND, typename R>
 __device__ __forceinline__ Cx<R> p2p(const KParams& kp, R x0, R x1, R x2, double xn, Cx<R> w)
 {
@@ -587,7 +597,7 @@ __device__ __forceinline__ Cx<R> p2p(const KParams& kp, R x0, R x1, R x2, double
     const R inv4pi = R(INV_4PI_D);
     if constexpr (KIND == KH || KIND == KM || (KIND == KG))
     {
-        if (KIND == KG ? (d2 < R(1e-24)) : (d2 == R(0)))
+        if (coincident<KIND>(d2))
             return {0, 0};
         R d, invd;
         dist_inv(d2, d, invd);
@@ -605,7 +615,7 @@ __device__ __forceinline__ Cx<R> p2p(const KParams& kp, R x0, R x1, R x2, double
     }
     else if constexpr (KIND == KL)
     {
-        if (d2 == R(0))
+        if (coincident<KIND>(d2))
             return {0, 0};
         R d, invd;
         dist_inv(d2, d, invd);
@@ -613,7 +623,7 @@ __device__ __forceinline__ Cx<R> p2p(const KParams& kp, R x0, R x1, R x2, double
     }
     else if constexpr (KIND == KD)
     {
-        if (d2 < R(1e-24))
+        if (coincident<KIND>(d2))
             return {0, 0};
         R d, invd;
         dist_inv(d2, d, invd);

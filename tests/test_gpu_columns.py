@@ -58,3 +58,29 @@ def test_orders_of_columns(gpu, kind, order, n, prec, ncol):
         W = np.stack([cdens(n, 300 + c) for c in range(ncol)], axis=1)
     op.init(x.T, x.T)
     _check(op, W, prec)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("ncol", [3, 13])
+@pytest.mark.parametrize("kind", ["helmholtz", "laplace", "grad"])
+def test_densities_that_are_not_finite(gpu, kind, ncol, prec):
+    """A density that is not finite leaves the result at its own point, which the sum leaves out,
+    as finite as a single column does, and the other columns alone."""
+    n = 2000
+    x = spheroid(n, 84)
+    op = {"helmholtz": lambda: ifgf_amd.HelmholtzIfgfOperator(7.0, 20, 7, 1, -1, precision=prec),
+          "laplace": lambda: ifgf_amd.LaplaceIfgfOperator(20, 7, 1, -1, precision=prec),
+          "grad": lambda: ifgf_amd.GradHelmholtzIfgfOperator(0.5 - 6.0j, 20, 8, 1, -1,
+                                                             precision=prec)}[kind]()
+    if kind == "grad":
+        op.setDx(0)
+    op.init(x.T, x.T)
+    W = np.stack([cdens(n, 500 + c) for c in range(ncol)], axis=1)
+    W = W.real.copy() if kind == "laplace" else W
+    good = op.mult(W)
+    W[5, 0], W[6, 1] = np.nan, np.inf
+    U = op.mult(W)
+    assert np.array_equal(U[:, 2:], good[:, 2:])
+    for c in (0, 1):
+        u = op.mult(np.ascontiguousarray(W[:, c]))
+        assert np.array_equal(np.isfinite(U[:, c]), np.isfinite(u)) and np.isfinite(u).any()

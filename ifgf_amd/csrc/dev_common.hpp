@@ -735,29 +735,31 @@ __device__ __forceinline__ int64_t xcd_block(int lg)
     return ((((i >> lg) << 3) + x) << lg) + (i & ((int64_t(1) << lg) - 1));
 }
 
-// The near field and the far groups of a mult on the plan's side stream (host side).  The
-// near field only writes the result (after the zeroing) and the far field adds to it (after
-// the near field), one far group after another (a group: one source level and one target
-// level, deepest source level first), each reading the coefficients of its source level only.
+// The near field and the far launches of a mult on the plan's side stream (host side).  The
+// near field writes the result (after the zeroing); a far launch (one source level, all target
+// levels, deepest source level first) reads the coefficients of its source level only and adds to
+// the far results, an array per target level, which the scatter sums up: the far launches follow
+// one another because they share those arrays, and follow the near field only because that is
+// ready to run before them.
 // mode 1: fork() starts the near field on the side stream (called after the deepest level's
 // transform, so that it runs beside the memory-bound upward kernels rather than the VALU-bound
 // leaf sampling); mode 2: fork() runs it on the main stream (called first).  In both, ready(l),
 // called once the upward chain has written source level l, enqueues on the side stream the far
-// groups of level l (and any deeper ones left), and finish() joins the side stream back.  Mode
-// 0: the near field at fork() and the far groups at finish(), in the same order, on the main
+// launches of level l (and any deeper ones left), and finish() joins the side stream back.  Mode
+// 0: the near field at fork() and the far launches at finish(), in the same order, on the main
 // stream (the sums are the same in every mode).
 template <class NearFn, class FarFn> struct SidePipe
 {
     DevicePlan& D;
     const std::vector<DevicePlan::FarGroup>& groups; // the far launches, deepest source level first
     hipStream_t st;
-    bool on;     // far groups on the side stream (modes 1 and 2)
+    bool on;     // far launches on the side stream (modes 1 and 2)
     bool near_side; // the near field on the side stream (mode 1)
     NearFn near; // near(stream)
     FarFn far;   // far(launch, stream)
     bool forked = false;
-    int next;    // the next far group to enqueue (deepest source level first)
-    // level storage (DevicePlan::ring) on one stream: the far groups of a source level run as
+    int next;    // the next far launch to enqueue (deepest source level first)
+    // level storage (DevicePlan::ring) on one stream: the far launches of a source level run as
     // soon as its coefficients are written, before the level two above overwrites them
     bool inline_far;
     SidePipe(DevicePlan& d, const std::vector<DevicePlan::FarGroup>& g, hipStream_t s, int mode,

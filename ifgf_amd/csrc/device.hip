@@ -1809,7 +1809,7 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring,
         // level, target level), deepest source level first, then deepest target level
         std::vector<WorkItem> fitems;
         std::vector<int32_t> frange;
-        D.far_groups.clear();
+        std::vector<DevicePlan::FarGroup> groups;
         D.far_steps.clear();
         std::vector<std::vector<int32_t>> tb_of_level(P.T.levels);
         for (int32_t t : ftb)
@@ -1856,11 +1856,11 @@ std::string device_upload(const Plan& P, int precision, DevicePlan& D, int ring,
                 // the angle tables of the group's grid classes, staged in LDS by the mixed far
                 // kernel when they fit 48 KB
                 const bool fits = hi > lo && (hi - lo) * int64_t(sizeof(double)) <= 48 * 1024;
-                D.far_groups.push_back({i0, int64_t(fitems.size()), fits ? int(lo) : 0,
-                                        fits ? int(hi - lo) : 0, sl, tl});
+                groups.push_back({i0, int64_t(fitems.size()), fits ? int(lo) : 0,
+                                  fits ? int(hi - lo) : 0, sl});
             }
         // the groups of a source level as one launch where their angle tables fit together
-        for (const auto& G : D.far_groups)
+        for (const auto& G : groups)
         {
             if (!D.far_steps.empty() && D.far_steps.back().src_level == G.src_level &&
                 (D.far_steps.back().ang_n > 0) == (G.ang_n > 0))

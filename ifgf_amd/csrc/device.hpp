@@ -73,9 +73,10 @@ struct LaunchShape
 {
     int xcd_log2 = 4; // work items dealt to the XCDs in runs of 2^xcd_log2 (0: plain order)
     int cpb = 0;      // transform: cones per workgroup (0: the order class's default)
-    int up_k = 16;    // upward: parent cones per workgroup (2, 4, 8 or 16)
+    int up_k = 16;    // upward: parent cones per workgroup, at most (2, 4, 8 or 16)
     int rb = 0;       // batched: most columns per pass (8 or 32; 0: 32)
-    int far_waves = 1; // mixed far field: waves (items) per workgroup sharing the LDS tables
+    int far_waves = 1; // far field: waves (items) per workgroup, sharing the LDS tables of the
+                       // launches that locate the pairs
     int overlap = 1;   // far field on a second stream beside the upward chain, with the near
                        // field there too (1) or first on the main stream (2); 0: one stream
 };
@@ -172,21 +173,18 @@ struct DevicePlan
     PointRun* near_run = nullptr;
     int32_t* near_pts = nullptr;
     WorkItem* far_items = nullptr;
-    // far work in launch groups of one source level and one target level, deepest source level
-    // first: a group can run as soon as its source level's coefficients exist; groups run one
-    // after another (a target point is in boxes of several levels)
+    // the far launches, deepest source level first: the items of one source level (of one target
+    // level each where their angle tables would not fit LDS together); a launch can run as soon
+    // as its source level's coefficients exist.  A target point is in boxes of several levels, so
+    // the items of target level t (WorkItem::pad: its index among the target levels with far
+    // items) add to their own results, far_res[pad * ntgt ..], and the scatter sums the levels in
+    // order.
     struct FarGroup
     {
         int64_t item0, item1; // far_items[item0 .. item1)
         int ang_base, ang_n;  // the sources' angle tables staged in LDS (mixed form; 0: none)
-        int src_level, tgt_level;
+        int src_level;
     };
-    std::vector<FarGroup> far_groups;
-    // the single-column mult's far launches: the groups of one source level together (a group
-    // each where their angle tables would not fit LDS together).  The groups of a launch run
-    // side by side, so the items of target level t (WorkItem::pad: its index among the target
-    // levels with far items) add to their own results, far_res[pad * ntgt ..], and the scatter
-    // sums the levels in order.
     std::vector<FarGroup> far_steps;
     // Where each (target, far source box) pair lies, in the order of the far items (item i's
     // records from far_rec_off[i] on, its targets fastest): the fine slot and local coordinates

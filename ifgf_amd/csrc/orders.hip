@@ -2,10 +2,10 @@
 //
 // The tolerance estimate (ifgfoperator.hpp:108-244) raises each axis' order by itself, so the
 // orders of an operator are any of hundreds of combinations and cannot all be compiled.  These
-// kernels are compiled per first fine order O0 only (the contiguous axis of a fine cone's
-// coefficients) and walk the other two axes in loops: the coefficients of a cone are O1 O2 rows
-// of O0 values, read a chunk of rows ahead of the arithmetic, and the Chebyshev values of the
-// two outer axes come from their recurrence as the rows go by.
+// kernels are compiled per pair of first fine orders (O0 1 to 6, O1 1 to 10; the others run one
+// generic instance) and walk the third axis in a loop: the coefficients of a cone are O2 planes of
+// O1 rows of O0 values, read a chunk ahead of the arithmetic, the Chebyshev values of the
+// first two axes in registers, those of the third from their recurrence as the planes go by.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,8 +27,9 @@ using namespace dev;
 // from child c in part[c n_hi + q], the eight then added in child order.  SEQ = true (n_hi too
 // large for eight copies in LDS): the children one after another, each adding to part[q] (a
 // node is in one group of a child, so no two threads add to the same place): the same sums.
-// Bound by the vector-memory path (each coefficient is read once per group, 64 lanes wide) and
-// the waits for it: at (3,6,4), 1M points, 11.0 ms; 14.7 without the read-ahead, 16 ms when a
+// Bound by the vector-memory path (each coefficient is read once per group, 64 lanes wide): at
+// (3,4,5), 1M points, 29 GB at 4.1 TB/s; at (5,5,5), combined field on a torus, 131,072 points, and in FP64
+// by the waits for it (2.0 and 2.1 TB/s, 348 and 126 vector instructions per ns).  At (3,6,4), 1M points, 11.0 ms; 14.7 without the read-ahead, 16 ms when a
 // chunk was read ahead past the last one; at (2,3,3) and (2,5,5) within 2% of k_up_grp without
 // its transform.
 template <typename R, int O0, int O1, bool SEQ>
@@ -422,7 +423,9 @@ __global__ __launch_bounds__(64) void k_far_record(
 // Far field from the pair records, any orders: as k_far_rows without the cone location.  A step
 // reads the pairs' records (one step ahead), then their cones: with stage > 0 the distinct cones
 // of the wave's lanes copied to LDS by all lanes together, otherwise each lane's from memory.
-// Bound by memory: the records are most of its traffic.  Far phase against locating the cones in
+// Bound by memory at few coefficients, the records most of its traffic (4.0 TB/s at (3,4,5), 1M
+// points); at (5,5,5) by the LDS reads (99 million, 1.3 of 2.4 ms at their rate) and the waits for
+// them (1.9 TB/s, 195 vector instructions per ns).  Far phase against locating the cones in
 // every mult: 7.5 -> 4.5 ms
 // at (3,6,4), 1M points; 3.7 -> 2.4 ms at (2,3,3), 1M points; FP64 at (3,5,4), 99,991 points,
 // 1.6 -> 0.63 ms.
@@ -565,7 +568,8 @@ void k_far_rec(
 // the axis-1 stage; Y: ysz, the axis-0 stage; the axis-2 stage goes to memory).  Each axis has
 // its loop compiled per number of inputs, chosen once by a uniform switch: an input is read from
 // LDS once for all its outputs and the map's entries are scalar operands, where one thread per
-// output read both from LDS for every product.  Bound by LDS and vector issue.
+// output read both from LDS for every product.  Bound by LDS (2 to 4 cycles of bank conflicts per
+// instruction) and vector issue (390 per ns), at 2.7 to 3.0 TB/s.
 // 1M points, (6,9,7)/(3,6,4): 16.8 -> 4.7 ms; torus, 131,072 points, (8,8,8)/(5,5,5): 3.8 ->
 // 0.94 ms.
 template <typename R>

@@ -23,7 +23,7 @@ template <typename R> __device__ __forceinline__ Cx<R> cmul_add(Cx<R> acc, Cx<R>
 }
 
 // A cone's coefficients are read a chunk ahead of the arithmetic, in two buffers of at most
-// CHUNK complex values (48 bytes of registers each): whole axis-2 planes where one or more fit,
+// CHUNK complex values (96 bytes, 24 registers, each): whole axis-2 planes where one or more fit,
 // else a plane's rows in equal parts
 template <typename R> constexpr int CHUNK = sizeof(R) == 4 ? 12 : 6;
 

@@ -104,8 +104,8 @@ __device__ __forceinline__ Cx<R> expmk_far(double kr, double ki, double r)
     R s, c;
     if constexpr (sizeof(R) == 4)
     {
-        double t = ph * INV_2PI_D; // revolutions, reduced exactly in FP64
-        t = t - rint(t);
+        // revolutions, reduced in FP64 (the roundings spelled out: see locate_fast)
+        const double t = fma(ph, INV_2PI_D, -rint(ph * INV_2PI_D));
         s = __builtin_amdgcn_sinf(float(t));
         c = __builtin_amdgcn_cosf(float(t));
     }
@@ -241,40 +241,38 @@ struct LocF
 __device__ __forceinline__ int angle_cell(const double* E, int n, double lo_shift, double inv_h,
                                           double p, double q, float& xi)
 {
+#pragma clang fp contract(off)
     const float cand = atan2_coarse(float(p), float(q)) + float(lo_shift);
     int c = min(max(int(cand * float(inv_h)), 0), n - 1);
     const float sc = float(2.0 * inv_h);
     const double* Cc = E + 2 * (n + 1) + 2 * c;
-    double xr = q * Cc[0] + p * Cc[1], yr = p * Cc[0] - q * Cc[1];
+    double xr = fma(q, Cc[0], p * Cc[1]), yr = fma(p, Cc[0], -(q * Cc[1]));
     xi = atan_small(__fdividef(float(yr), float(xr))) * sc;
     if (fabsf(xi) >= 1.f - 1e-5f)
     {
-        if (c > 0 && !(p * E[2 * c] - q * E[2 * c + 1] >= 0.0))
+        if (c > 0 && !(fma(p, E[2 * c], -(q * E[2 * c + 1])) >= 0.0))
             c--;
-        else if (c < n - 1 && p * E[2 * c + 2] - q * E[2 * c + 3] >= 0.0)
+        else if (c < n - 1 && fma(p, E[2 * c + 2], -(q * E[2 * c + 3])) >= 0.0)
             c++;
         Cc = E + 2 * (n + 1) + 2 * c;
-        xr = q * Cc[0] + p * Cc[1];
-        yr = p * Cc[0] - q * Cc[1];
+        xr = fma(q, Cc[0], p * Cc[1]);
+        yr = fma(p, Cc[0], -(q * Cc[1]));
         xi = atan_small(__fdividef(float(yr), float(xr))) * sc;
     }
     return c;
 }
 
-// FF: the fine/coarse factor of every axis when known at compile time (else f0, f1, f2)
-template <int FF = 0>
+// The kernels that lay down the pair records and those that locate the pairs must come to the same
+// bits, so which products fuse with which sums is spelled out here and in angle_cell: left to the
+// compiler it may differ from one kernel to the next.
 __device__ __forceinline__ bool locate_fast(const BoxGeo& B, const double* eth, const double* eph,
                                             const CellRef* __restrict__ ctab, double v0,
-                                            double v1, double v2, int f0_, int f1_, int f2_,
+                                            double v1, double v2, int f0, int f1, int f2,
                                             LocF& out)
 {
-    const int f0 = FF ? FF : f0_, f1 = FF ? FF : f1_, f2 = FF ? FF : f2_;
-    double a, r2;
-    {
 #pragma clang fp contract(off)
-        a = v0 * v0 + v1 * v1;
-        r2 = a + v2 * v2;
-    }
+    const double a = v0 * v0 + v1 * v1;
+    const double r2 = a + v2 * v2;
     const double rinv = rsq_nr(r2);
     double s = B.H * rinv;
     const double rho = a > 0.0 ? a * rsq_nr(a) : 0.0;
@@ -284,10 +282,10 @@ __device__ __forceinline__ bool locate_fast(const BoxGeo& B, const double* eth, 
     {
         // s decides the domain and the radial cell: near a bound or a cell edge it is
         // recomputed as the plan computes it (correctly rounded sqrt and division)
-        double d = s - B.lo[0];
+        double d = fma(B.H, rinv, -B.lo[0]);
         double t = d * B.inv_hf[0];
         double fl = floor(t);
-        double fr = t - fl;
+        double fr = fma(d, B.inv_hf[0], -fl);
         const double tol = 1e-12 * s;
         if (fabs(s - B.lo[0]) < tol || fabs(s - B.hi[0]) < tol || fr < 1e-9 ||
             fr > 1.0 - 1e-9)
@@ -298,7 +296,7 @@ __device__ __forceinline__ bool locate_fast(const BoxGeo& B, const double* eth, 
             d = s - B.lo[0];
             t = d * B.inv_hf[0];
             fl = floor(t);
-            fr = t - fl;
+            fr = fma(d, B.inv_hf[0], -fl);
             if (fr < 1e-9 || fr > 1.0 - 1e-9)
                 fl = floor(d / B.hf[0]);
         }

@@ -274,7 +274,7 @@ __device__ __forceinline__ void lds_fence()
 // 28% and 42% of a tile). Tile operands: lane l holds A[l % 16][l / 16] (map row, input index)
 // and B[l / 16][l % 16] (input index, column); the result tile row 4 (l / 16) + i, column
 // l % 16 is element i of lane l. The same map as k_transform_cols up to rounding (the axes in
-// another order), and slower than it on the 32-column spheroid (8.9 against 7.5 ms per mult):
+// another order), and slower than it on the 32-column spheroid (9.0 against 6.1 ms per mult):
 // the pass moves 19 GB (values read, coefficients of the active sub-cones written) and the
 // arithmetic is not what bounds it. Kept for that comparison: it runs only when the
 // environment variable IFGF_TRANSFORM_MFMA is set at the call (device_mult).

@@ -166,32 +166,47 @@ __global__ __launch_bounds__(256) void k_up_cols_locate(const int32_t* __restric
 }
 
 // High-order values -> fine coefficients of the active sub-cones (k_transform_rows) of one cone and
-// a chunk of cw columns per workgroup; thread = (pencil, column).  32 columns, 262,144 points,
-// (2,3,3): 7.4 ms, 2.6 TB/s and 328 vector instructions per ns, so by neither alone (with the orders
-// compiled in 6.6 ms).
-template <typename R>
+// a chunk of cw columns per workgroup; thread = (pencil, column).  C: the orders and the chunk's
+// columns as constants (Orders), or run-time values (AnyOrders).
+// 32 columns, 262,144 points, (2,3,3): 6.0 ms, 3.1 TB/s; 7.4 with run-time values, bound by neither
+// memory (2.6 TB/s) nor issue (328 vector instructions per ns) alone.
+struct AnyOrders
+{
+    static constexpr int h0 = 0, h1 = 0, h2 = 0, l0 = 0, l1 = 0, l2 = 0, cw = 0;
+};
+template <int H0, int H1, int H2, int L0, int L1, int L2, int CW> struct Orders // fine factors 3
+{
+    static constexpr int h0 = H0, h1 = H1, h2 = H2, l0 = L0, l1 = L1, l2 = L2, cw = CW;
+};
+template <typename R, class C>
 __global__ __launch_bounds__(256) void k_transform_cols(int64_t c0, int xsz,
                                                         const ConeDev* __restrict__ cones,
                                                         const Cx<R>* __restrict__ V,
                                                         Cx<R>* __restrict__ F,
-                                                        const R* __restrict__ W, int nc, int cw,
+                                                        const R* __restrict__ W, int nc, int cw_,
                                                         int nch, KParams kp)
 {
+    constexpr bool K = C::h0 > 0;
     extern __shared__ __align__(16) unsigned char tr_smem[];
+    const int cw = K ? C::cw : cw_;
     Cx<R>* X = reinterpret_cast<Cx<R>*>(tr_smem);
     Cx<R>* Y = X + xsz * cw;
-    const int h0 = kp.ho0, h1 = kp.ho1, h2 = kp.ho2, nh = kp.n_hi;
-    const int l0 = kp.lo0, l1 = kp.lo1, l2 = kp.lo2;
-    const int m0 = kp.f0 * l0, m1 = kp.f1 * l1;
+    const int h0 = K ? C::h0 : kp.ho0, h1 = K ? C::h1 : kp.ho1, h2 = K ? C::h2 : kp.ho2;
+    const int l0 = K ? C::l0 : kp.lo0, l1 = K ? C::l1 : kp.lo1, l2 = K ? C::l2 : kp.lo2;
+    const int f0 = K ? 3 : kp.f0, f1 = K ? 3 : kp.f1, f2 = K ? 3 : kp.f2;
+    const int nh = h0 * h1 * h2, nlo = l0 * l1 * l2;
+    const int m0 = f0 * l0, m1 = f1 * l1;
     const int64_t it = xcd_block(kp.xlg);
     const int64_t k = it / nch;
-    const int col0 = int(it - k * nch) * cw, cn = min(cw, nc - col0);
+    const int col0 = int(it - k * nch) * cw, cn = K ? C::cw : min(cw, nc - col0);
     const int64_t cone = c0 + k;
     const int tid = threadIdx.x;
+    // e / n (inv = 1 / n), by the constant where there is one
+    auto div = [](int e, int n, float inv) { return K ? e / n : div_small(e, inv); };
     const float icn = 1.0f / float(cn);
     for (int e = tid; e < nh * cn; e += 256)
     {
-        const int i = div_small(e, icn), r = e - i * cn;
+        const int i = div(e, cn, icn), r = e - i * cn;
         X[i * cw + r] = V[(cone * nh + i) * nc + col0 + r];
     }
     __syncthreads();
@@ -201,7 +216,7 @@ __global__ __launch_bounds__(256) void k_transform_cols(int64_t c0, int xsz,
                     {
                         for (int e = tid; e < h1 * h2 * cn; e += 256)
                         {
-                            const int p = div_small(e, icn), r = e - p * cn;
+                            const int p = div(e, cn, icn), r = e - p * cn;
                             Cx<R>* y = Y + p * m0 * cw + r;
                             map_pencil<R, decltype(H)::value>(W, h0, m0, X + p * h0 * cw + r, cw,
                                                               [&](int j, Cx<R> a) { y[j * cw] = a; });
@@ -213,8 +228,8 @@ __global__ __launch_bounds__(256) void k_transform_cols(int64_t c0, int xsz,
                     {
                         for (int e = tid; e < m0 * h2 * cn; e += 256)
                         {
-                            const int p = div_small(e, icn), r = e - p * cn;
-                            const int i2 = div_small(p, im0), j0 = p - i2 * m0;
+                            const int p = div(e, cn, icn), r = e - p * cn;
+                            const int i2 = div(p, m0, im0), j0 = p - i2 * m0;
                             Cx<R>* x = X + (j0 + m0 * m1 * i2) * cw + r;
                             map_pencil<R, decltype(H)::value>(
                                 W1, h1, m1, Y + (j0 + m0 * h1 * i2) * cw + r, m0 * cw,
@@ -225,24 +240,24 @@ __global__ __launch_bounds__(256) void k_transform_cols(int64_t c0, int xsz,
     const uint32_t mask = cones[cone].mask;
     const int64_t base = cones[cone].fine_base;
     const int l01 = l0 * l1;
-    const float il0 = 1.0f / float(l0), il01 = 1.0f / float(l01), if0 = 1.0f / float(kp.f0);
+    const float il0 = 1.0f / float(l0), il01 = 1.0f / float(l01), if0 = 1.0f / float(f0);
     with_high_order(h2, [&](auto H)
                     {
                         for (int e = tid; e < m0 * m1 * cn; e += 256)
                         {
                             // the pencils of one sub-cone column on consecutive lanes
-                            const int p = div_small(e, icn), r = e - p * cn;
-                            const int s01 = div_small(p, il01), m01 = p - s01 * l01;
-                            const int s1 = div_small(s01, if0), s0 = s01 - s1 * kp.f0;
-                            const int q1 = div_small(m01, il0), q0 = m01 - q1 * l0;
+                            const int p = div(e, cn, icn), r = e - p * cn;
+                            const int s01 = div(p, l01, il01), m01 = p - s01 * l01;
+                            const int s1 = div(s01, f0, if0), s0 = s01 - s1 * f0;
+                            const int q1 = div(m01, l0, il0), q0 = m01 - q1 * l0;
                             const int j01 = s0 * l0 + q0 + m0 * (s1 * l1 + q1);
-                            for (int s2 = 0; s2 < kp.f2; s2++)
+                            for (int s2 = 0; s2 < f2; s2++)
                             {
-                                const int sub = s01 + kp.f0 * kp.f1 * s2;
+                                const int sub = s01 + f0 * f1 * s2;
                                 if (!((mask >> sub) & 1u))
                                     continue;
                                 const int rk = __popc(mask & ((1u << sub) - 1u));
-                                Cx<R>* o = F + ((base + rk) * kp.n_lo + m01) * nc + col0 + r;
+                                Cx<R>* o = F + ((base + rk) * nlo + m01) * nc + col0 + r;
                                 const int os = l01 * nc;
                                 map_pencil<R, decltype(H)::value>(
                                     W2 + s2 * l2 * h2, h2, l2, X + j01 * cw + r, m0 * m1 * cw,
@@ -1058,11 +1073,20 @@ void launch_transform_cols(DevicePlan& D, hipStream_t st, const KParams& kp, int
     const size_t lds = cw * col;
     if (lds > LDS_MAX)
         throw std::runtime_error("interpolation orders too large for the transform kernel's LDS");
-    if (lds > size_t(64) * 1024)
-        HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_transform_cols<R>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    k_transform_cols<R><<<dim3(unsigned((c1 - c0) * nch)), dim3(256), lds, st>>>(
-        c0, xsz, D.cones, V, F, static_cast<const R*>(D.wmat), nc, cw, nch, kp);
+    auto go = [&](auto orders)
+    {
+        using C = decltype(orders);
+        if (lds > size_t(64) * 1024)
+            HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_transform_cols<R, C>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        k_transform_cols<R, C><<<dim3(unsigned((c1 - c0) * nch)), dim3(256), lds, st>>>(
+            c0, xsz, D.cones, V, F, static_cast<const R*>(D.wmat), nc, cw, nch, kp);
+    };
+    // (constants gain nothing in FP64 and at the larger orders, whose chunks are narrower)
+    if constexpr (sizeof(R) == 4)
+        if (order_class(D) == 1 && cw == 8 && nc % 8 == 0)
+            return go(Orders<3, 6, 6, 2, 3, 3, 8>());
+    go(AnyOrders());
 }
 
 // k_far_few_cols for a call of at most FEW_COLUMNS columns, where a cone's coefficients for five

@@ -61,7 +61,7 @@ class _IfgfOperator:
         self._m = None
         self._keep = None
         # mults of device tensors replay the mult's kernels as a HIP graph (one captured graph
-        # for single columns, one for batches of several)
+        # for single columns, one per number of columns for several)
         self.use_graph = False
 
     def __del__(self, _finalizing=sys.is_finalizing):

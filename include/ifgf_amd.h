@@ -56,8 +56,8 @@ extern "C" {
 #define IFGF_DEVICE_POINTERS 1 /* w and out are device pointers; work is enqueued on stream */
 #define IFGF_MULT_GRAPH 2      /* with IFGF_DEVICE_POINTERS: replay the mult's kernels between
                                   the gather and the scatter as a captured HIP graph, one for
-                                  the single-column mult and one for the batched mult of several
-                                  columns (each captured on its first such call and reused;
+                                  the single-column mult and one per number of columns for
+                                  several (each captured on its first such call and reused;
                                   captured again after ifgf_set_launch_shape / ifgf_autotune
                                   change a shape, ifgf_set_dx changes the direction or the batch
                                   buffers change width) */

@@ -582,20 +582,26 @@ void k_far_few_cols(const WorkItem* __restrict__ items, const int32_t* __restric
         qs = -1;
         if (valid && j + grp < jb)
         {
-            FarRec<R> q;
+            auto take = [&](const FarRec<R>& q)
+            {
+                qs = q.slot;
+                q0 = q.x0;
+                q1 = q.x1;
+                q2 = q.x2;
+            };
             if constexpr (PLACE == 0)
             {
                 const int64_t e = int64_t(j + grp) * wi.count;
-                q = rp[e];
+                take(rp[e]);
                 cf = cp[e];
             }
             else
+            {
+                FarRec<R> q;
                 place_pair<R, PLACE == 1>(geo[far_src[j0 + j + grp]], ctab, ang + ang_base, ang_base,
                                           y0, y1, y2, phase, kp, q, cf);
-            qs = q.slot;
-            q0 = q.x0;
-            q1 = q.x1;
-            q2 = q.x2;
+                take(q);
+            }
         }
     };
     fetch(ja);
